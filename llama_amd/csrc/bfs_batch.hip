@@ -574,9 +574,8 @@ __global__ void k_clear_listed(W* p, const uint32_t* lst, uint64_t n) {
 // (streamed, no random reads) and settles the bin's vertices as a pull row
 // would.  Every slot is read and written once per sweep, whatever the rows'
 // state: taken while the rows still open hold a large share of the edges.
-constexpr int kBinBlock = 1024;
 constexpr int kBinUnroll = 8;  // gather: slots per thread in flight
-constexpr int kBinGroup = 8;   // scatter: chunks per wave in flight
+constexpr int kBinGroup = 16;  // scatter: 64-slot pieces per wave in flight
 
 // LDS lane word of the gather (16-bit lanes OR into 32-bit words)
 template <typename W> struct BinAcc { using T = W; };
@@ -615,8 +614,9 @@ __global__ __launch_bounds__(kBinBlock) void k_msb_gather(MsArgs<W> a, const W* 
                                                           const uint32_t* indeg) {
   using A = typename BinAcc<W>::T;
   constexpr uint32_t R = 1u << BB;
-  constexpr uint32_t kPer = R / kBinBlock;
-  static_assert(kPer >= 1 && R % kBinBlock == 0, "bin rows must be a multiple of the block");
+  constexpr uint32_t kPer = R > uint32_t(kBinBlock) ? R / kBinBlock : 1u;
+  static_assert(R <= uint32_t(kBinBlock) || R % kBinBlock == 0,
+                "bin rows must be a multiple of the block, or at most one per thread");
   __shared__ A acc[R];
   const uint64_t b = xcd_block(blockIdx.x, gridDim.x);
   const uint64_t v0 = b << BB;
@@ -670,7 +670,7 @@ template <uint32_t BB, typename W>
 void launch_binned(const PrBins& pb, const W* fr, W* sv, const MsArgs<W>& a,
                    const uint32_t* indeg, hipStream_t s) {
   if constexpr (bins_fit<W>(BB)) {
-    k_msb_scatter<BB, W><<<pb.nbins, kBinBlock, 0, s>>>(fr, a.V, pb.nbins, pb.ct.as<uint2>(),
+      k_msb_scatter<BB, W><<<pb.nbins, kBinBlock, 0, s>>>(fr, a.V, pb.nbins, pb.ct.as<uint2>(),
                                                         pb.sidx.as<uint16_t>(), sv);
     k_msb_gather<BB, W><<<pb.nbins, kBinBlock, 0, s>>>(a, sv, pb.ldst.as<uint16_t>(),
                                                        pb.bstart.as<uint64_t>(), indeg);
@@ -800,8 +800,10 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
   const uint32_t* indeg = nullptr;
   if (bins_opt != 0) {
     const long bb = ctx->options.count("pr_bin_bits") ? ctx->options["pr_bin_bits"] : -1;
-    PrBins* p = ensure_pr_bins(g, level, bb);
-    if (!p && bins_opt == 1) p = ensure_pr_bins(g, level, 12);
+    uint32_t max_bb = kMaxBinBits;  // the largest bins this lane width can gather
+    while (!bins_fit<W>(max_bb)) max_bb--;
+    PrBins* p = ensure_lane_bins(g, level, bb, max_bb);
+    if (!p && bins_opt == 1 && bb == 0) p = ensure_pr_bins(g, level, 12);
     if (p && bins_fit<W>(p->bb)) {
       pb = p;
       indeg = ensure_degrees(g, LL_GPU_DIR_IN, level);
@@ -882,11 +884,9 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
     } else if (binned) {
       if (!sv.p) sv.alloc(std::max<uint64_t>(in.E, 1) * sizeof(W), s);
       TimedLaunch t(ctx, "k_msb_sweep");
-      switch (pb->bb) {
-        case 12: launch_binned<12, W>(*pb, fr.as<W>(), sv.as<W>(), a, indeg, s); break;
-        case 13: launch_binned<13, W>(*pb, fr.as<W>(), sv.as<W>(), a, indeg, s); break;
-        default: launch_binned<14, W>(*pb, fr.as<W>(), sv.as<W>(), a, indeg, s); break;
-      }
+      with_bin_bits(pb->bb, [&](auto k) {
+        launch_binned<k(), W>(*pb, fr.as<W>(), sv.as<W>(), a, indeg, s);
+      });
     } else {
       {
         TimedLaunch t(ctx, "k_ms_pull");

@@ -331,6 +331,7 @@ struct ll_gpu_graph {
   llgpu::PrSegments pr_seg;   // column segments of the in-CSR in slot order
   llgpu::PrHotCold pr_hc;     // hot/cold split of the in-CSR in slot order
   llgpu::PrBins pr_bins;      // binned PageRank layout of the out-CSR
+  llgpu::PrBins lane_bins;    // the same in smaller bins, for lane words pr_bins is too large for
   // weighted in-CSR (rows = heads, sources ascending) + map to out-edge positions
   int w_level = -1;
   llgpu::Csr wcsr;
@@ -409,11 +410,14 @@ void build_pr_hotcold(ll_gpu_graph* g, const Csr& in, const uint32_t* slot_adj, 
 // destinations, and `iters` iterations over it (FP32 ranks in rank_final).
 void build_pr_bins(ll_gpu_graph* g, const Csr& out, uint32_t bb, PrBins& pb);
 // The layout of level `level`'s out-CSR with bins of 2^bin_bits vertices
-// (12..14), built on first use; -1 = automatic (bins of 2^13 while the edges
-// between two such bins number 32 or more on average, else 2^14, while E <
-// 2^32 and the bins of 2^14 number at most 16384; otherwise none); nullptr
-// when there are none (0 or the automatic rule's "none").
+// (12..14), built on first use; -1 = automatic (8..14 by the snapshot's size
+// while E < 2^32 and the bins of 2^14 number at most 16384; otherwise none);
+// nullptr when there are none (0 or the automatic rule's "none").
 PrBins* ensure_pr_bins(ll_gpu_graph* g, int level, long bin_bits);
+// The same for a sweep whose LDS holds bins of at most 2^max_bb vertices: the
+// PageRank layout where it fits, else (automatic bins only) one of its own
+// in bins of 2^max_bb while the chunks stay long enough.
+PrBins* ensure_lane_bins(ll_gpu_graph* g, int level, long bin_bits, uint32_t max_bb);
 void pagerank_bins(ll_gpu_graph* g, const Csr& out, const uint32_t* outdeg, PrBins& pb,
                    int iters, double damping, DevBuf& rank_final, double* last_diff);
 

@@ -315,11 +315,7 @@ void pagerank_device(ll_gpu_graph* g, int level, int iters, double damping, uint
   hipStream_t s = ctx->stream;
   const uint64_t V = g->V;
   // Binned pull over the out-CSR (pr_bins.hip) unless turned off: bins of
-  // 2^pr_bin_bits vertices.  Automatic (-1), while E < 2^32: bins of 2^13
-  // while a chunk (the slots from one bin into another) holds 32 slots on
-  // average, else 2^14 (R-MAT s24: 69 slots per chunk, 1.10 ms per iteration
-  // against 1.49 ms with 2^14; s27: 8.6 slots per chunk, 17.1 ms against
-  // 9.2 ms with 2^14), as long as the bins of 2^14 number at most 16384.
+  // 2^pr_bin_bits vertices, automatic (-1) by the snapshot's size.
   {
     const long bin_bits = ctx->options.count("pr_bin_bits") ? ctx->options["pr_bin_bits"] : -1;
     if (PrBins* pb = ensure_pr_bins(g, level, bin_bits)) {

@@ -43,9 +43,8 @@ namespace llgpu {
 
 namespace {
 
-constexpr int kIterBlock = 1024;
 constexpr int kUnrollA = 8;  // phase A: slots per thread in flight
-constexpr int kGroupC = 8;   // phase C: chunks per wave in flight
+constexpr int kGroupC = 16;  // phase C: 64-slot pieces per wave in flight
 constexpr int kBuildBlock = 512;
 
 // Build items: pieces of one source bin's out-edges, a bin holding more than
@@ -210,14 +209,24 @@ struct PbArgs {
   double base, d, r0;
 };
 
+// x (a contribution: finite, >= 0, below 2) as a multiple of 2^-61, truncated:
+// the mantissa with its leading one at bit 61, shifted down by the exponent.
+// Zero and subnormals shift out (their exponent field is 0: 63 places).
+__device__ __forceinline__ unsigned long long fixed61(float x) {
+  const uint32_t b = __float_as_uint(x);
+  const unsigned long long m = (unsigned long long)((b & 0x7fffffu) | 0x800000u) << 38;
+  return m >> min(127u - (b >> 23), 63u);
+}
+
 // kInit: no accumulation, every rank = r0 (iteration 0's input); kScatter:
 // write the next iteration's binned values; kDiff: add |rank' - rank| of the
 // bin's vertices to *diff.
 template <uint32_t BB, bool kInit, bool kScatter, bool kDiff>
-__global__ __launch_bounds__(kIterBlock) void k_pb_iter(PbArgs a) {
+__global__ __launch_bounds__(kBinBlock) void k_pb_iter(PbArgs a) {
   constexpr uint32_t R = 1u << BB;
-  constexpr uint32_t kPer = R / kIterBlock;
-  static_assert(kPer >= 1 && R % kIterBlock == 0, "bin rows must be a multiple of the block");
+  constexpr uint32_t kPer = R > uint32_t(kBinBlock) ? R / kBinBlock : 1u;
+  static_assert(R <= uint32_t(kBinBlock) || R % kBinBlock == 0,
+                "bin rows must be a multiple of the block, or at most one per thread");
   __shared__ unsigned long long acc[R];
   // neighbouring source bins write neighbouring chunks of every destination
   // bin: keep them on one XCD
@@ -226,38 +235,38 @@ __global__ __launch_bounds__(kIterBlock) void k_pb_iter(PbArgs a) {
   const uint32_t nrows = uint32_t(min(uint64_t(R), a.V - v0));
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (!kInit) {
-    for (uint32_t i = threadIdx.x; i < R; i += kIterBlock) acc[i] = 0;
+    for (uint32_t i = threadIdx.x; i < R; i += kBinBlock) acc[i] = 0;
     __syncthreads();
     const uint64_t k0 = a.bstart[b], k1 = a.bstart[b + 1];
     // kUnrollA slots per thread requested before any is added
-    for (uint64_t k = k0 + threadIdx.x; k < k1; k += kUnrollA * uint64_t(kIterBlock)) {
+    for (uint64_t k = k0 + threadIdx.x; k < k1; k += kUnrollA * uint64_t(kBinBlock)) {
       float x[kUnrollA];
       uint16_t d[kUnrollA];
 #pragma unroll
       for (int u = 0; u < kUnrollA; u++) {
-        const uint64_t q = k + uint64_t(u) * kIterBlock;
+        const uint64_t q = k + uint64_t(u) * kBinBlock;
         x[u] = q < k1 ? a.val_in[q] : 0.f;
         d[u] = q < k1 ? a.ldst[q] : uint16_t(0);
       }
 #pragma unroll
       for (int u = 0; u < kUnrollA; u++)
-        if (k + uint64_t(u) * kIterBlock < k1)
-          atomicAdd(&acc[d[u]], (unsigned long long)(double(x[u]) * 0x1p61));
+        if (k + uint64_t(u) * kBinBlock < k1)
+          atomicAdd(&acc[d[u]], fixed61(x[u]));
     }
     __syncthreads();
   }
   float c[kPer];
-  float dsum = 0.f;
+  double dsum = 0;
 #pragma unroll
   for (uint32_t j = 0; j < kPer; j++) {
-    const uint32_t i = threadIdx.x + j * kIterBlock;
+    const uint32_t i = threadIdx.x + j * kBinBlock;
     c[j] = 0.f;
     if (i < nrows) {
       float r;
       if (kInit) r = float(a.r0);
       else r = float(a.base + a.d * (double(acc[i]) * 0x1p-61));
       a.rank_out[v0 + i] = r;
-      if (kDiff) dsum += fabsf(r - a.rank_in[v0 + i]);
+      if (kDiff) dsum += fabs(double(r) - double(a.rank_in[v0 + i]));
       const uint32_t od = a.outdeg[v0 + i];
       c[j] = od ? r / float(od) : 0.f;
     }
@@ -266,21 +275,22 @@ __global__ __launch_bounds__(kIterBlock) void k_pb_iter(PbArgs a) {
   if (kScatter) {
     if (!kInit) __syncthreads();  // accumulators read by every thread
 #pragma unroll
-    for (uint32_t j = 0; j < kPer; j++) cl[threadIdx.x + j * kIterBlock] = c[j];
+    for (uint32_t j = 0; j < kPer; j++)
+      if (threadIdx.x + j * kBinBlock < R) cl[threadIdx.x + j * kBinBlock] = c[j];
     __syncthreads();
     // chunks (b', b) of every destination bin b'
-    scatter_chunks<kIterBlock, kGroupC>(a.ct + b * a.nb, a.nb, a.sidx, cl, a.val_out);
+    scatter_chunks<kBinBlock, kGroupC>(a.ct + b * a.nb, a.nb, a.sidx, cl, a.val_out);
   }
   if (kDiff) {
     for (int o = 32; o > 0; o >>= 1) dsum += __shfl_down(dsum, o, 64);
     __syncthreads();  // the LDS words below are free again
-    float* red = reinterpret_cast<float*>(acc);
+    double* red = reinterpret_cast<double*>(acc);
     if (lane == 0) red[wave] = dsum;
     __syncthreads();
     if (threadIdx.x == 0) {
-      float t = 0.f;
-      for (int i = 0; i < kIterBlock / 64; i++) t += red[i];
-      atomicAdd(a.diff, double(t));
+      double t = 0;
+      for (int i = 0; i < kBinBlock / 64; i++) t += red[i];
+      unsafeAtomicAdd(a.diff, t);
     }
   }
 }
@@ -288,10 +298,10 @@ __global__ __launch_bounds__(kIterBlock) void k_pb_iter(PbArgs a) {
 template <uint32_t BB>
 void launch_iter(bool init, bool scatter, bool diff, unsigned nb, const PbArgs& a,
                  hipStream_t s) {
-  if (init) k_pb_iter<BB, true, true, false><<<nb, kIterBlock, 0, s>>>(a);
-  else if (scatter) k_pb_iter<BB, false, true, false><<<nb, kIterBlock, 0, s>>>(a);
-  else if (diff) k_pb_iter<BB, false, false, true><<<nb, kIterBlock, 0, s>>>(a);
-  else k_pb_iter<BB, false, false, false><<<nb, kIterBlock, 0, s>>>(a);
+  if (init) k_pb_iter<BB, true, true, false><<<nb, kBinBlock, 0, s>>>(a);
+  else if (scatter) k_pb_iter<BB, false, true, false><<<nb, kBinBlock, 0, s>>>(a);
+  else if (diff) k_pb_iter<BB, false, false, true><<<nb, kBinBlock, 0, s>>>(a);
+  else k_pb_iter<BB, false, false, false><<<nb, kBinBlock, 0, s>>>(a);
 }
 
 __global__ void k_zero_f64(double* p) { *p = 0.0; }
@@ -303,7 +313,7 @@ void build_pr_bins(ll_gpu_graph* g, const Csr& out, uint32_t bb, PrBins& pb) {
   hipStream_t s = ctx->stream;
   const uint64_t V = g->V, E = out.E;
   LLG_CHECK(E < (uint64_t(1) << 32), LL_GPU_ERANGE, "binned PageRank needs E < 2^32");
-  LLG_CHECK(bb >= 12 && bb <= 14, LL_GPU_EINVAL, "bin bits must be 12, 13 or 14");
+  LLG_CHECK(bb >= kMinBinBits && bb <= kMaxBinBits, LL_GPU_EINVAL, "bin bits must be 8..14");
   pb = PrBins();
   const uint32_t nb = uint32_t((V + (uint64_t(1) << bb) - 1) >> bb);
   const uint64_t nc = uint64_t(nb) * nb;
@@ -369,11 +379,9 @@ void build_pr_bins(ll_gpu_graph* g, const Csr& out, uint32_t bb, PrBins& pb) {
     uint32_t* tk = key.as<uint32_t>();
     uint32_t* tv = val.as<uint32_t>();
     uint32_t* tc = th.as<uint32_t>();
-    switch (bb) {
-      case 12: k_pb_keys<12><<<ni, kBuildBlock, lds, s>>>(ofs, adj, di, ni, V, nb, tk, tv, tc); break;
-      case 13: k_pb_keys<13><<<ni, kBuildBlock, lds, s>>>(ofs, adj, di, ni, V, nb, tk, tv, tc); break;
-      default: k_pb_keys<14><<<ni, kBuildBlock, lds, s>>>(ofs, adj, di, ni, V, nb, tk, tv, tc); break;
-    }
+    with_bin_bits(bb, [&](auto k) {
+      k_pb_keys<k()><<<ni, kBuildBlock, lds, s>>>(ofs, adj, di, ni, V, nb, tk, tv, tc);
+    });
     LLG_HIP(hipGetLastError());
     scan_u32_to_u64(th.as<uint32_t>(), X.as<uint64_t>(), nx, s);
     int kbits = 1;
@@ -393,22 +401,62 @@ void build_pr_bins(ll_gpu_graph* g, const Csr& out, uint32_t bb, PrBins& pb) {
   pb.nbins = nb;
 }
 
+namespace {
+
+uint64_t bins_of(uint64_t V, uint32_t bb) { return (V + (uint64_t(1) << bb) - 1) >> bb; }
+
+// Bin bits of the automatic rule; 0 = no bins.  The smallest bins whose chunks
+// hold 40 slots on average, for as many bins as the graph allows to share the
+// work (below that the ends of the chunks cost more than the extra workgroups
+// give); then the next size while chunks hold under 128 slots and 512 bins or
+// more remain.  Microseconds per iteration by bin bits (slots per chunk),
+// single-level R-MAT of 16 edges per vertex unless noted:
+//   10^4 vertices       8 (100) 9.1   9 (400) 11.7   13 (40028) 69
+//   10^5 vertices       8 (10) 20.1   9 (42) 21.0   10 (167) 24.3  13 114
+//   3*10^5 vertices     9 (14) 37.2  10 (56) 32.6   11 (222) 36.0  13 85
+//   2^20 vertices      10 (16) 84.1  11 (64) 65.7   12 (256) 67.1  13 87
+//   2^22 vertices      12 (64) 260   13 (256) 243   14 (1024) 238
+//   2^22, 8 per vertex 12 (32) 153   13 (128) 118   14 (512) 127
+//   2^24 vertices      12 (16) 1250  13 (64) 959    14 (256) 850
+uint32_t auto_bin_bits(uint64_t V, uint64_t E) {
+  if (E >= (uint64_t(1) << 32) || bins_of(V, kMaxBinBits) > 16384) return 0;
+  uint32_t bb = kMinBinBits;
+  auto slots = [&](uint32_t b) { return double(E) / (double(bins_of(V, b)) * bins_of(V, b)); };
+  while (bb < kMaxBinBits && (slots(bb) < 40 || bins_of(V, bb) > 16384)) bb++;
+  while (bb < kMaxBinBits && slots(bb) < 128 && bins_of(V, bb + 1) >= 512) bb++;
+  return bb;
+}
+
+}  // namespace
+
 PrBins* ensure_pr_bins(ll_gpu_graph* g, int level, long bin_bits) {
   const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
   const uint64_t V = g->V;
   if (bin_bits < 0) {
-    // bins of 2^13 while a chunk holds 32 slots on average, else 2^14, while
-    // E < 2^32 and the bins of 2^14 number at most 16384; otherwise none
-    const uint64_t nb13 = (V + (uint64_t(1) << 13) - 1) >> 13;
-    const uint64_t nb14 = (V + (uint64_t(1) << 14) - 1) >> 14;
-    if (out.E >= (uint64_t(1) << 32) || nb14 > 16384) bin_bits = 0;
-    else bin_bits = out.E >= 32 * nb13 * nb13 ? 13 : 14;
+    bin_bits = auto_bin_bits(V, out.E);
+    if (bin_bits == 0) return nullptr;
+  } else {
+    if (bin_bits == 0) return nullptr;
+    LLG_CHECK(bin_bits >= 12 && bin_bits <= 14, LL_GPU_EINVAL, "bin bits must be 0 or 12..14");
   }
-  if (bin_bits == 0) return nullptr;
-  LLG_CHECK(bin_bits >= 12 && bin_bits <= 14, LL_GPU_EINVAL, "bin bits must be 0 or 12..14");
   PrBins& pb = g->pr_bins;
   if (!(pb.valid && pb.level == out.level && pb.bb == uint32_t(bin_bits)))
     build_pr_bins(g, out, uint32_t(bin_bits), pb);
+  return &pb;
+}
+
+PrBins* ensure_lane_bins(ll_gpu_graph* g, int level, long bin_bits, uint32_t max_bb) {
+  PrBins* p = ensure_pr_bins(g, level, bin_bits);
+  if (!p || p->bb <= max_bb) return p;
+  // the PageRank bins are too large for this lane width: a layout of their
+  // own for the sweeps, while its chunks hold 32 slots on average (at 8.6 the
+  // binned sweep loses to the pull)
+  if (bin_bits >= 0) return nullptr;
+  const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
+  const uint64_t nb = bins_of(g->V, max_bb);
+  if (nb > 16384 || out.E < 32 * nb * nb) return nullptr;
+  PrBins& pb = g->lane_bins;
+  if (!(pb.valid && pb.level == out.level && pb.bb == max_bb)) build_pr_bins(g, out, max_bb, pb);
   return &pb;
 }
 
@@ -436,12 +484,7 @@ void pagerank_bins(ll_gpu_graph* g, const Csr& out, const uint32_t* outdeg, PrBi
   a.d = damping;
   a.r0 = 1.0 / double(V);
   auto launch = [&](bool init, bool scatter, bool dflag) {
-    switch (pb.bb) {
-      case 12: launch_iter<12>(init, scatter, dflag, pb.nbins, a, s); break;
-      case 13: launch_iter<13>(init, scatter, dflag, pb.nbins, a, s); break;
-      case 14: launch_iter<14>(init, scatter, dflag, pb.nbins, a, s); break;
-      default: throw Error{LL_GPU_EINVAL, "binned PageRank supports 12, 13 or 14 bin bits"};
-    }
+    with_bin_bits(pb.bb, [&](auto k) { launch_iter<k()>(init, scatter, dflag, pb.nbins, a, s); });
     LLG_HIP(hipGetLastError());
   };
   {

@@ -1,0 +1,58 @@
+"""The binned out-edge layout at every bin size its automatic rule picks: ranks
+are bit-identical to those over explicit bins of 2^12 vertices (row sums are
+integers) and within 1e-6 L1 of the FP64 oracle, and multi-source sweeps over
+it give every lane its single-source levels."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import gpu_case
+from llama_amd.graph import DeviceGraph, HostGraph
+
+pytestmark = pytest.mark.gpu
+
+
+def skewed(V, per, seed):
+    """per * V edges whose heads crowd the low IDs, a hub at V // 2, no self-loops."""
+    rng = np.random.default_rng(seed)
+    n = V * per
+    src = rng.integers(0, V, n)
+    dst = (V * rng.random(n) ** 3).astype(np.int64)
+    dst[: n // 20] = V // 2
+    keep = src != dst
+    g = HostGraph(V)
+    g.add_level(src[keep], dst[keep])
+    return g
+
+
+# vertices, edges per vertex: bins of 2^8 (one, two, fewer than a workgroup's
+# waves, forty), then 2^9, 2^10, 2^11; chunks of a slot to thousands of slots
+@pytest.mark.parametrize("V,per", [(2, 3), (256, 5), (257, 400), (3000, 20), (10007, 16),
+                                   (20011, 8), (140001, 12), (600011, 16)])
+def test_every_bin_size(ctx, V, per):
+    gpu_case(f"bins V={V} per={per}")
+    g = skewed(V, per, V)
+    dg = DeviceGraph(ctx, g)
+    r, diff = dg.pagerank(6)
+    ctx.set_option("pr_bin_bits", 12)
+    try:
+        r12, diff12 = dg.pagerank(6)
+    finally:
+        ctx.set_option("pr_bin_bits", -1)
+    assert np.array_equal(r, r12)
+    # FP64 sums of the same FP32 differences in another order
+    assert abs(diff - diff12) <= 1e-12 * max(abs(diff), 1e-30) + 1e-15
+    if V <= 20011:
+        ref, _ = oracle.OracleGraph.from_host(g).pagerank(6)
+        assert float(np.abs(r - ref).sum() / np.abs(ref).sum()) <= 1e-6
+    roots = np.random.default_rng(V).integers(0, V, 130)
+    ctx.set_option("bfs_batch_bins", 1)
+    try:
+        for lanes in (16, 64, 128):
+            gpu_case(f"bins V={V} lanes={lanes}")
+            lv, reached, _ = dg.bfs_batch(roots, lane_width=lanes)
+            for j in (0, 63, 129):
+                one, n, _ = dg.bfs(int(roots[j]))
+                assert np.array_equal(lv[j], one) and reached[j] == n
+    finally:
+        ctx.set_option("bfs_batch_bins", -1)
