@@ -150,10 +150,7 @@ void drop_snapshots(ll_gpu_graph* g) {
   g->pr_hc = llgpu::PrHotCold();
   g->pr_bins = llgpu::PrBins();
   g->lane_bins = llgpu::PrBins();
-  g->w_level = -1;
-  g->wcsr = Csr();
-  g->wperm.release();
-  g->wrb.clear();
+  for (auto& m : g->wpr) m = llgpu::WprMatrix();
 }
 
 }  // namespace llgpu

@@ -274,6 +274,18 @@ struct PrBins {
   DevBuf ct;      // uint2[nbins * nbins]: [source bin][destination bin] = {first slot, slots}
 };
 
+// One direction of the weighted PageRank sweeps (built by wpr.hip).
+struct WprMatrix {
+  int level = -1;
+  DevBuf slot;      // uint32_t[V]: number of each vertex's row and column (empty: its ID)
+  DevBuf perm;      // uint32_t[E]: entry -> out-edge position (empty: its own)
+  Csr csr;          // not valid: the snapshot's out-CSR
+  DevBuf items;     // sweep items, one wave's work each
+  DevBuf splits;    // rows cut into several pieces
+  uint64_t n = 0, nparts = 0;
+  uint32_t nsplits = 0;
+};
+
 struct DirMirror {
   std::vector<DevBuf> vt;   // per level: the pages the level wrote (all of them for a full push)
   std::vector<std::vector<const VtEntry*>> vt_pages;  // per level: device address of every page
@@ -332,11 +344,7 @@ struct ll_gpu_graph {
   llgpu::PrHotCold pr_hc;     // hot/cold split of the in-CSR in slot order
   llgpu::PrBins pr_bins;      // binned PageRank layout of the out-CSR
   llgpu::PrBins lane_bins;    // the same in smaller bins, for lane words pr_bins is too large for
-  // weighted in-CSR (rows = heads, sources ascending) + map to out-edge positions
-  int w_level = -1;
-  llgpu::Csr wcsr;
-  llgpu::DevBuf wperm;        // uint32_t[E]: weighted in-edge -> out-edge position
-  std::list<llgpu::RowBlocks> wrb;
+  llgpu::WprMatrix wpr[2];    // weighted PageRank: forward, adjoint
 };
 
 namespace llgpu {
@@ -397,6 +405,8 @@ const RowBlocks& ensure_rowblocks(ll_gpu_graph* g, uint32_t dir, int level, uint
 void build_rowblocks(ll_gpu_ctx* ctx, const Csr& c, uint32_t cap, uint32_t piece,
                      RowBlocks& rb);
 void drop_snapshots(ll_gpu_graph* g);
+// inv[v] = position of v by descending `deg` (ties by ID).
+void degree_slots(ll_gpu_ctx* ctx, const uint32_t* deg, uint64_t V, DevBuf& inv);
 // Column segments of `in` (source IDs mapped through `inv` when given) with
 // segments of 2^zb slots (zb raised until at most kMaxSegments segments).
 void build_pr_segments(ll_gpu_graph* g, const Csr& in, const uint32_t* inv, uint32_t zb,

@@ -308,6 +308,31 @@ void launch_pr_pull(uint32_t cap, bool sorted, unsigned nitems, const PrArgs& a,
   else launch_pr_pull_t<kMode, false>(cap, nitems, a, s);
 }
 
+void degree_slots(ll_gpu_ctx* ctx, const uint32_t* deg, uint64_t V, DevBuf& inv) {
+  hipStream_t s = ctx->stream;
+  DevBuf mx, keys, ids, skeys, sids;
+  mx.alloc(4, s);
+  k_fill_u32<<<1, 1, 0, s>>>(mx.as<uint32_t>(), 0u);
+  k_max_u32<<<std::min(grid_for(V, 256), 4u * unsigned(ctx->num_cus)), 256, 0, s>>>(
+      deg, V, mx.as<uint32_t>());
+  LLG_HIP(hipMemcpyAsync(ctx->readback, mx.p, 4, hipMemcpyDeviceToHost, s));
+  LLG_HIP(hipStreamSynchronize(s));
+  const uint32_t maxdeg = *static_cast<const uint32_t*>(ctx->readback);
+  int bits = 1;
+  while (bits < 32 && (maxdeg >> bits) != 0) bits++;
+  keys.alloc(V * 4, s);
+  ids.alloc(V * 4, s);
+  skeys.alloc(V * 4, s);
+  sids.alloc(V * 4, s);
+  k_deg_keys<<<grid_for(V, 256), 256, 0, s>>>(deg, maxdeg, keys.as<uint32_t>(),
+                                              ids.as<uint32_t>(), V);
+  sort_pairs_u32_u32(keys.as<uint32_t>(), skeys.as<uint32_t>(), ids.as<uint32_t>(),
+                     sids.as<uint32_t>(), V, bits, s);
+  inv.alloc(V * 4, s);
+  k_inv_from_sorted<<<grid_for(V, 256), 256, 0, s>>>(sids.as<uint32_t>(), inv.as<uint32_t>(), V);
+  LLG_HIP(hipGetLastError());
+}
+
 // Run `iters` pull iterations; leaves FP32 ranks in rank_final (device).
 void pagerank_device(ll_gpu_graph* g, int level, int iters, double damping, uint32_t cap,
                      DevBuf& rank_final, double* last_diff) {
@@ -341,28 +366,7 @@ void pagerank_device(ll_gpu_graph* g, int level, int iters, double damping, uint
   if (reorder) {
     if (g->pr_level != in.level) {
       TimedLaunch t(ctx, "pr_reorder");
-      DevBuf mx, keys, ids, skeys, sids;
-      mx.alloc(4, s);
-      k_fill_u32<<<1, 1, 0, s>>>(mx.as<uint32_t>(), 0u);
-      k_max_u32<<<std::min(grid_for(V, 256), 4u * unsigned(ctx->num_cus)), 256, 0, s>>>(
-          outdeg, V, mx.as<uint32_t>());
-      LLG_HIP(hipMemcpyAsync(ctx->readback, mx.p, 4, hipMemcpyDeviceToHost, s));
-      LLG_HIP(hipStreamSynchronize(s));
-      const uint32_t maxdeg = *static_cast<const uint32_t*>(ctx->readback);
-      int bits = 1;
-      while (bits < 32 && (maxdeg >> bits) != 0) bits++;
-      keys.alloc(V * 4, s);
-      ids.alloc(V * 4, s);
-      skeys.alloc(V * 4, s);
-      sids.alloc(V * 4, s);
-      k_deg_keys<<<grid_for(V, 256), 256, 0, s>>>(outdeg, maxdeg, keys.as<uint32_t>(),
-                                                  ids.as<uint32_t>(), V);
-      sort_pairs_u32_u32(keys.as<uint32_t>(), skeys.as<uint32_t>(), ids.as<uint32_t>(),
-                         sids.as<uint32_t>(), V, bits, s);
-      g->pr_inv.alloc(V * 4, s);
-      k_inv_from_sorted<<<grid_for(V, 256), 256, 0, s>>>(sids.as<uint32_t>(),
-                                                         g->pr_inv.as<uint32_t>(), V);
-      LLG_HIP(hipGetLastError());
+      degree_slots(ctx, outdeg, V, g->pr_inv);
       g->pr_adj.release();
       g->pr_sadj.release();
       g->pr_sperm.release();

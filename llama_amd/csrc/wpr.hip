@@ -8,12 +8,11 @@
 //   forward:  r0 = p,  r' = (1-d) p + d W^T r            (pull over in-edges)
 //   adjoint:  l0 = g,  l' = g + d W l                     (pull over out-edges)
 //             dL/dw[e=(u,v)] = d r[u] l[v],  dL/dp = (1-d) l
-// The in-edge view carries each edge's out-edge position (radix sort of
-// (head, tail) keys), so the forward gathers w into in-edge order once per
-// call.  Both sweeps use one row-block kernel: a workgroup stages
-// val[e] * x[col[e]] for a run of short rows in LDS with coalesced loads and
-// reduces each row in one thread (FP32 Neumaier); long rows are split into
-// pieces combined in order.  Bytes per sweep: 12 per edge + 16 per vertex.
+// Either direction is one sweep kernel over a CSR whose rows and columns are
+// numbered by descending degree (hot columns then sit in LDS), with a
+// permutation that brings w into entry order once per call; sums are FP64.
+// Bytes per sweep: 8 per edge (column, weight) + 20 per vertex, and a gather
+// of x per edge that misses the LDS table.
 #include "ll_gpu_internal.h"
 #include "rowblocks.h"
 
@@ -22,105 +21,285 @@ namespace llgpu {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr uint32_t kCap = 1024;
+constexpr uint32_t kGradCap = 1024;          // row blocks of the edge gradient
+constexpr int kSpBlock = 1024;
+constexpr uint32_t kCap = 512;               // stream-item capacity of the row blocks
+constexpr uint32_t kEnt = kCap + kCap / 2;   // entries of an item, at most
+constexpr uint32_t kWPiece = kEnt;           // entries of one piece of a long row
+constexpr uint32_t kHot = 24576;             // entries of x kept in LDS
+constexpr uint32_t kThreadRow = 32;          // longest row a single lane sums
+constexpr uint32_t kRowLanes = 8;            // lanes of a longer one
+
+// One item of a sweep: a wave's work.
+struct SpItem {
+  uint32_t row;   // first row; of a split row's piece, its place in `part`
+  uint32_t meta;  // entries | rows << 12 | kind << 24
+  uint64_t e0;    // first entry
+};
+static_assert(sizeof(SpItem) == 16 && kEnt < 4096 && kRowsPerItem < 4096, "SpItem fields");
+constexpr uint32_t kRun = 0, kOneRow = 1, kSplit = 2;
+// A row cut into several pieces.
+struct SpSplit {
+  uint32_t row, part, pieces;
+};
 
 struct SpArgs {
-  const RowItem* items;
-  const uint32_t* slots;
+  const SpItem* items;
+  uint64_t nitems;
+  const SpSplit* splits;
+  uint32_t nsplits;
   const uint64_t* ofs;
   const uint32_t* col;
   const float* val;
   const float* x;
-  const float* base;   // y = base_scale * base[r] + d * S
+  uint64_t nx;
+  const float* base;      // y = base_scale * base + d * (matrix * x)
   float base_scale, d;
   float* y;
-  Neu* part;
+  double* part;           // sums of the pieces of split rows
 };
 
-__device__ inline void sp_finalize(const SpArgs& a, uint32_t r, float S) {
-  a.y[r] = a.base_scale * a.base[r] + a.d * S;
+// Make a wave's LDS writes visible to its other lanes before they read them.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-__global__ __launch_bounds__(kBlock) void k_wspmv(SpArgs a) {
-  __shared__ float vals[kCap + kCap / 2];
-  __shared__ uint64_t rofs[kRowsPerItem + 1];
-  __shared__ Neu red[kBlock / 64];
-  const RowItem it = a.items[blockIdx.x];
-  if (it.npieces == 0) {
-    const uint32_t nrows = it.row_end - it.row_begin;
-    for (uint32_t i = threadIdx.x; i <= nrows; i += kBlock) rofs[i] = a.ofs[it.row_begin + i];
-    __syncthreads();
-    const uint64_t e0 = rofs[0];
-    const uint32_t ne = uint32_t(rofs[nrows] - e0);
-    constexpr uint32_t kPer = (kCap + kCap / 2) / kBlock;
-    uint32_t idx[kPer];
-    float wv[kPer];
+// One sweep: a fixed grid of waves taking items in turn, each wave on its own
+// (no workgroup barrier past the first).
+//
+// Bound by load latency: a CU keeps few enough gathers of x from L2 in flight
+// that they, not the 8 bytes streamed per edge, set the pace.  So rows and
+// columns are numbered by descending degree: the first kHot entries of x,
+// which take most of the gathers of a skewed graph, are copied to LDS once per
+// workgroup, and the others lie close together.  Everything else an item
+// needs (entries, row offsets, base) is loaded while the wave's item before it
+// is summed.
+//
+// A run of short rows: the products are staged in LDS and summed in FP64, rows
+// of up to kThreadRow entries by a lane each, longer ones by kRowLanes lanes
+// each.  A long row is cut into pieces, a wave each; k_wspmv_split adds them
+// in a fixed order, so the result does not depend on the schedule.
+//
+// 2^20 vertices, 16.8 M edges: 69 us a sweep (2.0 TB/s of streamed bytes);
+// 120 us with one workgroup per item and columns by vertex ID, 83 us with the
+// columns but not the rows renumbered (y and base then scattered), 196 us
+// with workgroup-wide items and the same LDS table.  Lanes per row 8 / rows of
+// 32 by a lane: 7.94 ms for 100 sweeps, 16 / 16: 8.22, 8 / 8: 8.14; a table of
+// 8192 entries: 8.87.
+__global__ __launch_bounds__(kSpBlock) void k_wspmv(SpArgs a) {
+  constexpr uint32_t kPer = kEnt / 64;
+  constexpr uint32_t kWaves = kSpBlock / 64;
+  constexpr uint32_t kRowPer = kRowsPerItem / 64;
+  __shared__ float hot[kHot];
+  __shared__ float s_vals[kWaves][kEnt];
+  __shared__ uint16_t s_rofs[kWaves][kRowsPerItem + 1];
+  __shared__ uint16_t s_list[kWaves][kEnt / kThreadRow];  // rows left to lane groups
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  float* vals = s_vals[wave];
+  uint16_t* rofs = s_rofs[wave];
+  uint16_t* list = s_list[wave];
+  const uint64_t stride = uint64_t(gridDim.x) * kWaves;
+  uint64_t i = uint64_t(blockIdx.x) * kWaves + wave;
+  uint32_t idx[kPer], ro[kRowPer];
+  float wv[kPer], rb[kRowPer];
+  auto load = [&](const SpItem& it) {
+    const uint32_t ne = it.meta & 0xfffu, nrows = (it.meta >> 12) & 0xfffu;
 #pragma unroll
     for (uint32_t k = 0; k < kPer; k++) {
-      const uint32_t i = threadIdx.x + k * kBlock;
-      idx[k] = i < ne ? a.col[e0 + i] : 0u;
-      wv[k] = i < ne ? a.val[e0 + i] : 0.f;
+      const uint32_t q = lane + 64 * k;
+      idx[k] = q < ne ? a.col[it.e0 + q] : 0u;
+      wv[k] = q < ne ? a.val[it.e0 + q] : 0.f;
     }
 #pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) {
-      const uint32_t i = threadIdx.x + k * kBlock;
-      if (i < ne) vals[i] = wv[k] * a.x[idx[k]];
+    for (uint32_t k = 0; k < kRowPer; k++) {
+      const uint32_t q = lane + 64 * k;
+      ro[k] = q < nrows ? uint32_t(a.ofs[it.row + q] - it.e0) : 0u;
+      rb[k] = q < nrows ? a.base[it.row + q] : 0.f;
     }
-    __syncthreads();
-    if (threadIdx.x < nrows) {
-      const uint32_t lo = uint32_t(rofs[threadIdx.x] - e0), hi = uint32_t(rofs[threadIdx.x + 1] - e0);
-      Neu s = Neu::zero();
-      for (uint32_t j = lo; j < hi; j++) s.add(vals[j]);
-      sp_finalize(a, it.row_begin + threadIdx.x, s.value());
+  };
+  auto fetch = [&](uint64_t q) { return q < a.nitems ? a.items[q] : SpItem{0u, 0u, 0ull}; };
+  auto uniform = [](SpItem t) {
+    t.row = uint32_t(__builtin_amdgcn_readfirstlane(int(t.row)));
+    t.meta = uint32_t(__builtin_amdgcn_readfirstlane(int(t.meta)));
+    const uint32_t lo = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(t.e0))));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(t.e0 >> 32))));
+    t.e0 = uint64_t(hi) << 32 | lo;
+    return t;
+  };
+  SpItem cur = uniform(fetch(i)), nxt = uniform(fetch(i + stride));
+  load(cur);
+  for (uint32_t q = threadIdx.x; q < kHot; q += kSpBlock) hot[q] = q < a.nx ? a.x[q] : 0.f;
+  __syncthreads();
+  for (; i < a.nitems; i += stride) {
+    const uint32_t ne = cur.meta & 0xfffu, nrows = (cur.meta >> 12) & 0xfffu;
+    const uint32_t kind = cur.meta >> 24;
+    const SpItem after = fetch(i + 2 * stride);
+    float xv[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) xv[k] = idx[k] >= kHot ? a.x[idx[k]] : 0.f;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++)
+      if (idx[k] < kHot) xv[k] = hot[idx[k]];
+    if (kind == kRun) {
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; k++)
+        if (lane + 64 * k < ne) vals[lane + 64 * k] = wv[k] * xv[k];
+      float yb[kRowPer];
+#pragma unroll
+      for (uint32_t k = 0; k < kRowPer; k++) {
+        if (lane + 64 * k < nrows) rofs[lane + 64 * k] = uint16_t(ro[k]);
+        yb[k] = a.base_scale * rb[k];
+      }
+      if (lane == 0) rofs[nrows] = uint16_t(ne);
+      wave_sync();
+      load(nxt);
+      // rows past kThreadRow entries, their sums left at their first product
+      uint32_t lo[kRowPer], n[kRowPer], nl = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kRowPer; k++) {
+        const uint32_t r = lane + 64 * k;
+        lo[k] = n[k] = 0;
+        if (r < nrows) {
+          lo[k] = rofs[r];
+          n[k] = rofs[r + 1] - lo[k];
+        }
+        const uint64_t m = __ballot(n[k] > kThreadRow);
+        if (n[k] > kThreadRow)
+          list[nl + uint32_t(__popcll(m & ((uint64_t(1) << lane) - 1)))] = uint16_t(r);
+        nl += uint32_t(__popcll(m));
+      }
+      wave_sync();
+      for (uint32_t q0 = 0; q0 < nl; q0 += 64 / kRowLanes) {
+        const uint32_t q = q0 + lane / kRowLanes;
+        double S = 0;
+        uint32_t first = 0;
+        if (q < nl) {
+          const uint32_t r = list[q], hi = rofs[r + 1];
+          first = rofs[r];
+#pragma unroll 4
+          for (uint32_t j = first + lane % kRowLanes; j < hi; j += kRowLanes)
+            S += double(vals[j]);
+        }
+        for (int o = kRowLanes / 2; o > 0; o >>= 1) S += __shfl_down(S, o, kRowLanes);
+        if (q < nl && lane % kRowLanes == 0) vals[first] = float(S);
+      }
+      wave_sync();
+#pragma unroll
+      for (uint32_t k = 0; k < kRowPer; k++) {
+        if (64 * k >= nrows) break;
+        double S = 0;
+        const uint32_t hi = lo[k] + (n[k] > kThreadRow ? 1u : n[k]);
+#pragma unroll 4
+        for (uint32_t j = lo[k]; j < hi; j++) S += double(vals[j]);
+        if (lane + 64 * k < nrows) a.y[cur.row + lane + 64 * k] = yb[k] + a.d * float(S);
+      }
+      wave_sync();  // vals, rofs and list are rewritten for the next item
+    } else {
+      double S = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; k++)
+        if (lane + 64 * k < ne) S += double(wv[k] * xv[k]);
+      load(nxt);
+      for (int o = 32; o > 0; o >>= 1) S += __shfl_down(S, o, 64);
+      if (lane == 0) {
+        if (kind == kOneRow) a.y[cur.row] = a.base_scale * a.base[cur.row] + a.d * float(S);
+        else a.part[cur.row] = S;
+      }
     }
-  } else {
-    const uint32_t r = it.row_begin;
-    const uint64_t lo = a.ofs[r] + uint64_t(it.piece) * kPiece;
-    const uint64_t hi = min(a.ofs[r + 1], lo + kPiece);
-    Neu s = Neu::zero();
-    for (uint64_t e = lo + threadIdx.x; e < hi; e += kBlock) s.add(a.val[e] * a.x[a.col[e]]);
-    s = wave_reduce(s);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      Neu t = red[0];
-      for (int i = 1; i < kBlock / 64; i++) t.merge(red[i]);
-      if (it.npieces == 1) sp_finalize(a, r, t.value());
-      else a.part[a.slots[blockIdx.x]] = t;
-    }
+    cur = nxt;
+    nxt = uniform(after);
   }
 }
 
-__global__ void k_wspmv_fixup(SpArgs a, uint64_t nitems) {
+// Split rows: kSplitLanes lanes add a row's pieces, always in the same order.
+constexpr uint32_t kSplitLanes = 16;
+__global__ void k_wspmv_split(SpArgs a) {
+  const uint32_t q = (blockIdx.x * blockDim.x + threadIdx.x) / kSplitLanes;
+  const uint32_t lane = threadIdx.x % kSplitLanes;
+  if (q >= a.nsplits) return;  // whole lane groups
+  const SpSplit t = a.splits[q];
+  double S = 0;
+#pragma unroll 4
+  for (uint32_t p = lane; p < t.pieces; p += kSplitLanes) S += a.part[t.part + p];
+  for (int o = kSplitLanes / 2; o > 0; o >>= 1) S += __shfl_down(S, o, kSplitLanes);
+  if (lane == 0) a.y[t.row] = a.base_scale * a.base[t.row] + a.d * float(S);
+}
+
+// Sweep items and split rows (counted in *cnt) of row blocks.
+__global__ void k_sweep_items(const RowItem* items, const uint32_t* pslot, uint64_t n,
+                              const uint64_t* ofs, SpItem* out, SpSplit* splits, uint32_t* cnt) {
   const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= nitems) return;
-  const RowItem it = a.items[i];
-  if (it.npieces > 1 && it.piece == 0) {
-    Neu t = a.part[a.slots[i]];
-    for (uint32_t p = 1; p < it.npieces; p++) t.merge(a.part[a.slots[i + p]]);
-    sp_finalize(a, it.row_begin, t.value());
+  if (i >= n) return;
+  const RowItem it = items[i];
+  uint64_t e0 = ofs[it.row_begin], e1 = ofs[it.row_end];
+  SpItem t;
+  t.row = it.row_begin;
+  uint32_t kind = kRun, nrows = it.row_end - it.row_begin;
+  if (it.npieces) {
+    e0 += uint64_t(it.piece) * kWPiece;
+    e1 = min(e1, e0 + kWPiece);
+    kind = kOneRow;
+    nrows = 0;
+    if (it.npieces > 1) {
+      kind = kSplit;
+      t.row = pslot[i];
+      if (it.piece == 0) splits[atomicAdd(cnt, 1u)] = SpSplit{it.row_begin, t.row, it.npieces};
+    }
   }
+  t.meta = uint32_t(e1 - e0) | nrows << 12 | kind << 24;
+  t.e0 = e0;
+  out[i] = t;
 }
 
-__global__ void k_wkeys(const uint64_t* ofs, const uint32_t* adj, uint64_t V, uint64_t* keys,
-                        uint32_t* pos) {
-  const uint64_t u = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (u >= V) return;
-  for (uint64_t e = ofs[u], end = ofs[u + 1]; e < end; e++) {
-    keys[e] = (uint64_t(adj[e]) << 32) | u;
-    pos[e] = uint32_t(e);
-  }
+__global__ void k_zero_u32(uint32_t* p) { *p = 0; }
+
+// Tail of every out-edge, a wave per row.
+__global__ void k_edge_tails(const uint64_t* ofs, uint64_t V, uint32_t* tail) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t nw = uint64_t(gridDim.x) * (blockDim.x / 64);
+  for (uint64_t u = uint64_t(blockIdx.x) * (blockDim.x / 64) + (threadIdx.x >> 6); u < V; u += nw)
+    for (uint64_t e = ofs[u] + lane, end = ofs[u + 1]; e < end; e += 64) tail[e] = uint32_t(u);
 }
 
-// CSR rows from sorted (head << 32 | tail) keys.
-__global__ void k_key_rows(const uint64_t* keys, uint64_t m, uint64_t V, uint64_t* ofs,
-                           uint32_t* col) {
+// Edge e's row (its number in `slot` when given) as the sort key, e as the value.
+__global__ void k_row_keys(const uint32_t* row, const uint32_t* slot, uint32_t* key,
+                           uint32_t* pos, uint64_t n) {
+  const uint64_t e = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  key[e] = slot ? slot[row[e]] : row[e];
+  pos[e] = uint32_t(e);
+}
+
+// Row offsets of the sorted rows.
+__global__ void k_row_offsets(const uint32_t* rows, uint64_t m, uint64_t V, uint64_t* ofs) {
   const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i > m) return;
-  const uint64_t a = i < m ? keys[i] >> 32 : V;
-  const uint64_t p = i == 0 ? 0 : (keys[i - 1] >> 32) + 1;
+  const uint64_t a = i < m ? rows[i] : V;
+  const uint64_t p = i == 0 ? 0 : uint64_t(rows[i - 1]) + 1;
   for (uint64_t x = p; x <= a && x <= V; x++) ofs[x] = i;
-  if (i < m) col[i] = uint32_t(keys[i]);
+}
+
+// col[i] = column of edge perm[i] (its number in `slot` when given).
+__global__ void k_columns(const uint32_t* perm, const uint32_t* column, const uint32_t* slot,
+                          uint32_t* col, uint64_t n) {
+  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t c = column[perm[i]];
+  col[i] = slot ? slot[c] : c;
+}
+
+// xs[slot[v]] = x[v].
+__global__ void k_to_slots(const float* x, const uint32_t* slot, float* xs, uint64_t n) {
+  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) xs[slot[i]] = x[i];
+}
+
+// x[v] = xs[slot[v]].
+__global__ void k_from_slots(const float* xs, const uint32_t* slot, float* x, uint64_t n) {
+  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) x[i] = xs[slot[i]];
 }
 
 __global__ void k_gather_w(const float* w, const uint32_t* perm, float* out, uint64_t n) {
@@ -161,87 +340,154 @@ __global__ __launch_bounds__(kBlock) void k_edge_grad(const RowItem* items, cons
   }
 }
 
-void sweep(ll_gpu_ctx* ctx, const RowBlocks& rb, const Csr& c, const float* val, const float* x,
-           const float* base, float base_scale, float d, float* y, DevBuf& part, const char* name) {
+// The sweep items of matrix `c`.
+void build_sweep_items(ll_gpu_ctx* ctx, const Csr& c, WprMatrix& m) {
   hipStream_t s = ctx->stream;
-  SpArgs a;
-  a.items = rb.items.as<RowItem>();
-  a.slots = rb.slots.as<uint32_t>();
+  RowBlocks rb;
+  build_rowblocks(ctx, c, kCap, kWPiece, rb);
+  DevBuf cnt;
+  cnt.alloc(4, s);
+  m.items.alloc(std::max<uint64_t>(rb.n, 1) * sizeof(SpItem), s);
+  m.splits.alloc(std::max<uint64_t>(rb.nsplit, 1) * sizeof(SpSplit), s);
+  k_zero_u32<<<1, 1, 0, s>>>(cnt.as<uint32_t>());
+  k_sweep_items<<<grid_for(rb.n, 256), 256, 0, s>>>(
+      rb.items.as<RowItem>(), rb.slots.as<uint32_t>(), rb.n, c.ofs.as<uint64_t>(),
+      m.items.as<SpItem>(), m.splits.as<SpSplit>(), cnt.as<uint32_t>());
+  LLG_HIP(hipGetLastError());
+  LLG_HIP(hipMemcpyAsync(ctx->readback, cnt.p, 4, hipMemcpyDeviceToHost, s));
+  LLG_HIP(hipStreamSynchronize(s));
+  m.nsplits = *static_cast<const uint32_t*>(ctx->readback);
+  m.n = rb.n;
+  m.nparts = rb.nsplit;
+}
+
+// The matrix of one direction of the sweeps.  forward: rows = heads, columns =
+// tails; adjoint: rows = tails, columns = heads.  Entries of a row in out-edge
+// order.  Rows and columns are numbered by descending degree on the column
+// side, unless all of x fits the LDS table anyway.  The adjoint's rows are the
+// out-CSR's own when they keep their numbers (also past 2^32 edges, where no
+// u32 permutation exists).
+const WprMatrix& ensure_wpr_matrix(ll_gpu_graph* g, int level, bool forward) {
+  level = resolve_level(g, level);
+  WprMatrix& m = g->wpr[forward ? 0 : 1];
+  if (m.level == level) return m;
+  ll_gpu_ctx* ctx = g->ctx;
+  hipStream_t s = ctx->stream;
+  const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
+  const uint64_t V = g->V, E = out.E;
+  const bool fits = E < (uint64_t(1) << 32);
+  LLG_CHECK(fits || !forward, LL_GPU_ERANGE, "weighted PageRank needs E < 2^32");
+  m = WprMatrix();
+  const bool renumber = V > kHot && fits;
+  if (!forward && !renumber) {
+    build_sweep_items(ctx, out, m);
+    m.level = level;
+    return m;
+  }
+  if (renumber)
+    degree_slots(ctx, ensure_degrees(g, forward ? LL_GPU_DIR_OUT : LL_GPU_DIR_IN, level), V, m.slot);
+  const uint32_t* slot = m.slot.as<uint32_t>();
+  const uint64_t n = std::max<uint64_t>(E, 1);
+  DevBuf tail, key, pos, rows;
+  tail.alloc(n * 4, s);
+  key.alloc(n * 4, s);
+  pos.alloc(n * 4, s);
+  rows.alloc(n * 4, s);
+  m.perm.alloc(n * 4, s);
+  k_edge_tails<<<unsigned(std::min<uint64_t>((V + 3) / 4, uint64_t(ctx->num_cus) * 32)), 256, 0,
+                 s>>>(out.ofs.as<uint64_t>(), V, tail.as<uint32_t>());
+  const uint32_t* heads = out.adj.as<uint32_t>();
+  k_row_keys<<<grid_for(E, 256), 256, 0, s>>>(forward ? heads : tail.as<uint32_t>(), slot,
+                                              key.as<uint32_t>(), pos.as<uint32_t>(), E);
+  LLG_HIP(hipGetLastError());
+  int bits = 1;
+  while (bits < 32 && ((V - 1) >> bits) != 0) bits++;
+  sort_pairs_u32_u32(key.as<uint32_t>(), rows.as<uint32_t>(), pos.as<uint32_t>(),
+                     m.perm.as<uint32_t>(), E, bits, s);
+  m.csr.ofs.alloc((V + 1) * 8, s);
+  m.csr.adj.alloc(n * 4, s);
+  k_row_offsets<<<grid_for(E + 1, 256), 256, 0, s>>>(rows.as<uint32_t>(), E, V,
+                                                     m.csr.ofs.as<uint64_t>());
+  k_columns<<<grid_for(E, 256), 256, 0, s>>>(m.perm.as<uint32_t>(),
+                                             forward ? tail.as<uint32_t>() : heads, slot,
+                                             m.csr.adj.as<uint32_t>(), E);
+  LLG_HIP(hipGetLastError());
+  m.csr.valid = true;
+  m.csr.level = level;
+  m.csr.V = V;
+  m.csr.E = E;
+  build_sweep_items(ctx, m.csr, m);
+  m.level = level;
+  return m;
+}
+
+// iters >= 1 sweeps y = base_scale * base + d * (matrix * y) from y = base;
+// the last y, by vertex, in `out`.
+void wpr_sweeps(ll_gpu_graph* g, int level, bool forward, const float* w, const float* base,
+                float base_scale, float d, int iters, float* out, const char* name) {
+  ll_gpu_ctx* ctx = g->ctx;
+  hipStream_t s = ctx->stream;
+  const WprMatrix& m = ensure_wpr_matrix(g, level, forward);
+  const Csr& c = m.csr.valid ? m.csr : ensure_csr(g, LL_GPU_DIR_OUT, level);
+  const uint64_t V = g->V;
+  const uint32_t* slot = m.slot.as<uint32_t>();
+  DevBuf w_in, base_in, buf[2], part;
+  if (m.perm.p) {
+    w_in.alloc(std::max<uint64_t>(c.E, 1) * 4, s);
+    k_gather_w<<<grid_for(c.E, 256), 256, 0, s>>>(w, m.perm.as<uint32_t>(), w_in.as<float>(), c.E);
+    w = w_in.as<float>();
+  }
+  if (slot) {
+    base_in.alloc(V * 4, s);
+    k_to_slots<<<grid_for(V, 256), 256, 0, s>>>(base, slot, base_in.as<float>(), V);
+    base = base_in.as<float>();
+  }
+  LLG_HIP(hipGetLastError());
+  buf[0].alloc(V * 4, s);
+  buf[1].alloc(V * 4, s);
+  part.alloc(m.nparts * 8, s);
+  SpArgs a{};
+  a.items = m.items.as<SpItem>();
+  a.nitems = m.n;
+  a.splits = m.splits.as<SpSplit>();
+  a.nsplits = m.nsplits;
   a.ofs = c.ofs.as<uint64_t>();
   a.col = c.adj.as<uint32_t>();
-  a.val = val;
-  a.x = x;
+  a.val = w;
+  a.x = base;
+  a.nx = V;
   a.base = base;
   a.base_scale = base_scale;
   a.d = d;
-  a.y = y;
-  a.part = part.as<Neu>();
-  {
-    TimedLaunch t(ctx, name);
-    k_wspmv<<<unsigned(rb.n), kBlock, 0, s>>>(a);
+  a.part = part.as<double>();
+  constexpr uint64_t kWaves = kSpBlock / 64;
+  const unsigned grid =
+      unsigned(std::min<uint64_t>((m.n + kWaves - 1) / kWaves, uint64_t(ctx->num_cus)));
+  for (int it = 0; it < iters; it++) {
+    a.y = it == iters - 1 && !slot ? out : buf[it & 1].as<float>();
+    {
+      TimedLaunch t(ctx, name);
+      k_wspmv<<<grid, kSpBlock, 0, s>>>(a);
+    }
+    if (a.nsplits) k_wspmv_split<<<grid_for(uint64_t(a.nsplits) * kSplitLanes, 64), 64, 0, s>>>(a);
+    LLG_HIP(hipGetLastError());
+    a.x = a.y;
   }
-  if (rb.nsplit) k_wspmv_fixup<<<grid_for(rb.n, 256), 256, 0, s>>>(a, rb.n);
+  if (slot) k_from_slots<<<grid_for(V, 256), 256, 0, s>>>(a.x, slot, out, V);
   LLG_HIP(hipGetLastError());
 }
 
 }  // namespace
 
-void ensure_wcsr(ll_gpu_graph* g, int level) {
-  level = resolve_level(g, level);
-  if (g->w_level == level) return;
-  hipStream_t s = g->ctx->stream;
-  const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
-  const uint64_t V = g->V, E = out.E;
-  LLG_CHECK(E < (uint64_t(1) << 32), LL_GPU_ERANGE, "weighted PageRank needs E < 2^32");
-  DevBuf keys, pos, skeys;
-  keys.alloc(std::max<uint64_t>(E, 1) * 8, s);
-  pos.alloc(std::max<uint64_t>(E, 1) * 4, s);
-  skeys.alloc(std::max<uint64_t>(E, 1) * 8, s);
-  g->wperm.alloc(std::max<uint64_t>(E, 1) * 4, s);
-  k_wkeys<<<grid_for(V, 256), 256, 0, s>>>(out.ofs.as<uint64_t>(), out.adj.as<uint32_t>(), V,
-                                            keys.as<uint64_t>(), pos.as<uint32_t>());
-  LLG_HIP(hipGetLastError());
-  sort_pairs_u64_u32(keys.as<uint64_t>(), skeys.as<uint64_t>(), pos.as<uint32_t>(),
-                     g->wperm.as<uint32_t>(), E, 64, s);
-  g->wcsr = Csr();
-  g->wcsr.ofs.alloc((V + 1) * 8, s);
-  g->wcsr.adj.alloc(std::max<uint64_t>(E, 1) * 4, s);
-  k_key_rows<<<grid_for(E + 1, 256), 256, 0, s>>>(skeys.as<uint64_t>(), E, V,
-                                                  g->wcsr.ofs.as<uint64_t>(),
-                                                  g->wcsr.adj.as<uint32_t>());
-  LLG_HIP(hipGetLastError());
-  g->wcsr.valid = true;
-  g->wcsr.level = level;
-  g->wcsr.V = V;
-  g->wcsr.E = E;
-  g->wrb.clear();
-  g->wrb.emplace_back();
-  build_rowblocks(g->ctx, g->wcsr, kCap, kPiece, g->wrb.back());
-  g->w_level = level;
-}
-
 // Forward: iters sweeps from r0 = p; result in r_out (device).
 void wpr_forward_device(ll_gpu_graph* g, int level, const float* w, const float* p, int iters,
                         double d, float* r_out) {
-  ll_gpu_ctx* ctx = g->ctx;
-  hipStream_t s = ctx->stream;
-  ensure_wcsr(g, level);
-  const uint64_t V = g->V, E = g->wcsr.E;
-  const RowBlocks& rb = g->wrb.back();
-  DevBuf w_in, buf[2], part;
-  w_in.alloc(std::max<uint64_t>(E, 1) * 4, s);
-  k_gather_w<<<grid_for(E, 256), 256, 0, s>>>(w, g->wperm.as<uint32_t>(), w_in.as<float>(), E);
-  buf[0].alloc(V * 4, s);
-  buf[1].alloc(V * 4, s);
-  part.alloc(std::max<uint64_t>(rb.nsplit, 1) * sizeof(Neu), s);
-  const float* x = p;
-  for (int it = 0; it < iters; it++) {
-    float* y = it == iters - 1 ? r_out : buf[it & 1].as<float>();
-    sweep(ctx, rb, g->wcsr, w_in.as<float>(), x, p, float(1.0 - d), float(d), y, part,
-          "k_wspmv_fwd");
-    x = y;
+  if (iters > 0) {
+    wpr_sweeps(g, level, true, w, p, float(1.0 - d), float(d), iters, r_out, "k_wspmv_fwd");
+  } else {
+    ensure_wpr_matrix(g, level, true);
+    LLG_HIP(hipMemcpyAsync(r_out, p, g->V * 4, hipMemcpyDeviceToDevice, g->ctx->stream));
   }
-  if (iters == 0) LLG_HIP(hipMemcpyAsync(r_out, p, V * 4, hipMemcpyDeviceToDevice, s));
 }
 
 void wpr_adjoint_device(ll_gpu_graph* g, int level, const float* w, const float* r,
@@ -249,17 +495,14 @@ void wpr_adjoint_device(ll_gpu_graph* g, int level, const float* w, const float*
   ll_gpu_ctx* ctx = g->ctx;
   hipStream_t s = ctx->stream;
   const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
-  const RowBlocks& rb = ensure_rowblocks(g, LL_GPU_DIR_OUT, level, kCap, kPiece);
+  const RowBlocks& rb = ensure_rowblocks(g, LL_GPU_DIR_OUT, level, kGradCap, kPiece);
   const uint64_t V = g->V;
-  DevBuf buf[2], part;
-  buf[0].alloc(V * 4, s);
-  buf[1].alloc(V * 4, s);
-  part.alloc(std::max<uint64_t>(rb.nsplit, 1) * sizeof(Neu), s);
+  DevBuf lam_v;
   const float* lam = gr;
-  for (int it = 0; it < iters; it++) {
-    float* y = buf[it & 1].as<float>();
-    sweep(ctx, rb, out, w, lam, gr, 1.0f, float(d), y, part, "k_wspmv_adj");
-    lam = y;
+  if (iters > 0) {
+    lam_v.alloc(V * 4, s);
+    wpr_sweeps(g, level, false, w, gr, 1.0f, float(d), iters, lam_v.as<float>(), "k_wspmv_adj");
+    lam = lam_v.as<float>();
   }
   if (dw) {
     TimedLaunch t(ctx, "k_edge_grad");

@@ -1,0 +1,58 @@
+"""Weighted PageRank sweeps at the edges of the sweep items: rows of 0, 1, 8,
+32, 33, 255..257, 511..513, 767..769 and thousands of entries, graphs whose x
+fits the LDS table and one that does not, against FP64."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import gpu_case
+from llama_amd.autograd import weighted_pagerank
+from llama_amd.graph import SlcsrGraph, csr_of
+
+pytestmark = pytest.mark.gpu
+
+DEGS = [0, 1, 7, 8, 9, 31, 32, 33, 64, 255, 256, 257, 511, 512, 513, 767, 768, 769, 1535, 1537, 9000]
+D, K = 0.85, 12
+# each sweep rounds the products, the sum and the result to FP32 (3 * 2^-24
+# relative, every term positive), and the errors of earlier sweeps are damped
+# by D per sweep: 3 * 2^-24 / (1 - D) = 1.2e-6; twice that allowed
+TOL = 2.4e-6
+
+
+@pytest.mark.parametrize("V", [1, 70, 4001, 24576, 24577, 90001])
+def test_rows_of_every_length(ctx, V):
+    gpu_case(f"wpr rows V={V}")
+    rng = np.random.default_rng(V)
+    src, dst = [], []
+    for i, d in enumerate(DEGS * 3):
+        if V < 2 or d >= 4 * V:
+            continue
+        v = int(rng.integers(0, V))
+        other = rng.integers(0, V, d)
+        (src if i % 2 else dst).append(np.full(d, v))
+        (dst if i % 2 else src).append(other)
+    src.append(rng.integers(0, V, 3 * V))
+    dst.append(rng.integers(0, V, 3 * V))
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    ofs, adj = csr_of(V, src, dst)
+    tail = np.repeat(np.arange(V), np.diff(ofs))
+    E = adj.size
+    dg = SlcsrGraph(ctx, V, (ofs, adj), csr_of(V, dst, src))
+    outdeg = np.maximum(np.diff(ofs), 1)
+    w = (rng.random(E) / outdeg[tail]).astype(np.float32)
+    p = (rng.random(V) / V).astype(np.float32)
+    grad = rng.random(V).astype(np.float32)
+    wt = torch.tensor(w, device="cuda", requires_grad=True)
+    pt = torch.tensor(p, device="cuda", requires_grad=True)
+    r = weighted_pagerank(wt, pt, dg, K, D)
+    r.backward(torch.tensor(grad, device="cuda"))
+    w64, x, lam = w.astype(np.float64), p.astype(np.float64), grad.astype(np.float64)
+    for _ in range(K):
+        x = (1 - D) * p + D * np.bincount(adj, w64 * x[tail], V)
+        lam = grad + D * np.bincount(tail, w64 * lam[adj], V)
+    assert np.all(np.abs(r.detach().cpu().numpy() - x) <= TOL * x)
+    assert np.all(np.abs(pt.grad.cpu().numpy() - (1 - D) * lam) <= TOL * lam)
+    ref = D * x[tail] * lam[adj]
+    assert np.all(np.abs(wt.grad.cpu().numpy() - ref) <= 2 * TOL * ref + 1e-30)
+    again = weighted_pagerank(wt, pt, dg, K, D)
+    assert torch.equal(again, r)  # the sums do not depend on the schedule
