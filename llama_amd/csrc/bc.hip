@@ -485,7 +485,7 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
       }
       LLG_HIP(hipGetLastError());
     }
-    if (bc_out) LLG_HIP(hipMemcpyAsync(bc_out, bc.p, V * 4, hipMemcpyDeviceToHost, s));
+    if (bc_out) copy_to_host(ctx, bc_out, bc.p, V * 4);
     LLG_HIP(hipStreamSynchronize(s));
     return LL_GPU_OK;
   } catch (const Error& e) {

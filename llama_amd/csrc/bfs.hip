@@ -1015,10 +1015,7 @@ int ll_gpu_bfs_ex(ll_gpu_graph* g, int level, int64_t root, int32_t* levels_out,
     LLG_CHECK(root >= 0 && uint64_t(root) < g->V, LL_GPU_EINVAL, "root outside [0, max_nodes)");
     llgpu::DevBuf lv;
     llgpu::BfsResult r = llgpu::bfs_device(g, level, uint32_t(root), lv);
-    if (levels_out) {
-      LLG_HIP(hipMemcpyAsync(levels_out, lv.p, g->V * 4, hipMemcpyDeviceToHost, g->ctx->stream));
-      LLG_HIP(hipStreamSynchronize(g->ctx->stream));
-    }
+    if (levels_out) llgpu::copy_to_host(g->ctx, levels_out, lv.p, g->V * 4);
     if (reached) *reached = r.reached;
     if (edges_examined) *edges_examined = r.examined;
     if (edges_traversed) *edges_traversed = r.traversed;

@@ -1004,10 +1004,8 @@ int ll_gpu_bfs_batch_ex(ll_gpu_graph* g, int level, const int64_t* roots, int n,
         default: msbfs_batch<W128>(g, level, d_roots.as<int64_t>(), m, b, lvp, rp, sweeps); break;
       }
     }
-    if (levels_out)
-      LLG_HIP(hipMemcpyAsync(levels_out, d_lv.p, size_t(n) * V * 4, hipMemcpyDeviceToHost, s));
-    if (reached_out)
-      LLG_HIP(hipMemcpyAsync(reached_out, d_reached.p, size_t(n) * 8, hipMemcpyDeviceToHost, s));
+    if (levels_out) copy_to_host(g->ctx, levels_out, d_lv.p, size_t(n) * V * 4);
+    if (reached_out) copy_to_host(g->ctx, reached_out, d_reached.p, size_t(n) * 8);
     LLG_HIP(hipStreamSynchronize(s));
     return LL_GPU_OK;
   } catch (const Error& e) {

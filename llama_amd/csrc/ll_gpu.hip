@@ -66,6 +66,23 @@ __global__ void k_apply_patches(const uint64_t* const* et_table, const uint64_t*
     et[idx] = (w & llgpu::kIndexMask) | (uint64_t(ml) << llgpu::kBitsIndex);
 }
 
+// Bytes a thread of the copy pool moves at a time.
+constexpr size_t kCopySlice = size_t(256) << 10;
+
+// memcpy on the copy pool.
+void pool_memcpy(ll_gpu_ctx* c, char* dst, const char* src, size_t n) {
+  if (n <= 2 * kCopySlice) {
+    std::memcpy(dst, src, n);
+    return;
+  }
+  c->copies.run((n + kCopySlice - 1) / kCopySlice,
+                [&](size_t i) {
+                  const size_t o = i * kCopySlice;
+                  std::memcpy(dst + o, src + o, std::min(kCopySlice, n - o));
+                },
+                [] {});
+}
+
 // Copy host bytes to device through the double-buffered pinned staging area.
 void upload(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
   const char* s = static_cast<const char*>(src);
@@ -76,8 +93,13 @@ void upload(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
     size_t m = std::min(half, bytes - off);
     LLG_HIP(hipEventSynchronize(c->pinned_ev[slot]));
     char* stage = static_cast<char*>(c->pinned) + slot * half;
-    std::memcpy(stage, s + off, m);
-    LLG_HIP(hipMemcpyAsync(d + off, stage, m, hipMemcpyHostToDevice, c->stream));
+    // a slice at a time, so the device copies the first while the next are staged
+    constexpr size_t kStep = 16 * kCopySlice;
+    for (size_t o = 0; o < m; o += kStep) {
+      const size_t k = std::min(kStep, m - o);
+      pool_memcpy(c, stage + o, s + off + o, k);
+      LLG_HIP(hipMemcpyAsync(d + off + o, stage + o, k, hipMemcpyHostToDevice, c->stream));
+    }
     LLG_HIP(hipEventRecord(c->pinned_ev[slot], c->stream));
   }
 }
@@ -107,6 +129,61 @@ TimedLaunch::~TimedLaunch() {
   if (!a) return;
   if (hipEventRecord(b, ctx->stream) == hipSuccess)
     ctx->timer.pending.push_back({name, a, b});
+}
+
+void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
+  char* d = static_cast<char*>(dst);
+  const char* p = static_cast<const char*>(src);
+  if (bytes == 0) {
+    LLG_HIP(hipStreamSynchronize(c->stream));
+    return;
+  }
+  if (bytes <= kReadbackBytes) {
+    LLG_HIP(hipMemcpyAsync(c->readback, p, bytes, hipMemcpyDeviceToHost, c->stream));
+    LLG_HIP(hipStreamSynchronize(c->stream));
+    std::memcpy(d, c->readback, bytes);
+    return;
+  }
+  // the staging is refilled from its start for every c->pinned_bytes of result
+  for (size_t off = 0; off < bytes; off += c->pinned_bytes) {
+    const size_t m = std::min(c->pinned_bytes, bytes - off);
+    // one chunk under 1 MiB (waking the pool costs as much as the copy), else
+    // chunks of 512 KiB to 2 MiB (each costs the device about 8 us besides its
+    // 40 us per 2 MiB), which the pool moves on in slices
+    const bool whole = m < (size_t(1) << 20);
+    const size_t chunk = whole ? m : m < (size_t(8) << 20) ? size_t(512) << 10 : size_t(2) << 20;
+    const size_t slice = whole ? m : kCopySlice;
+    const size_t n = (m + chunk - 1) / chunk;
+    while (c->chunk_ev.size() < n) {
+      hipEvent_t e;
+      LLG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      c->chunk_ev.push_back(e);
+    }
+    char* stage = static_cast<char*>(c->pinned);
+    for (size_t i = 0; i < n; i++) {
+      const size_t o = i * chunk;
+      LLG_HIP(hipMemcpyAsync(stage + o, p + off + o, std::min(chunk, m - o),
+                             hipMemcpyDeviceToHost, c->stream));
+      LLG_HIP(hipEventRecord(c->chunk_ev[i], c->stream));
+    }
+    std::atomic<size_t> ready{0};  // chunks in the staging; n + 1 = given up
+    hipError_t err = hipSuccess;
+    c->copies.run((m + slice - 1) / slice,
+                  [&](size_t i) {
+                    const size_t o = i * slice;
+                    size_t r;
+                    while ((r = ready.load(std::memory_order_acquire)) <= o / chunk)
+                      std::this_thread::yield();
+                    if (r <= n) std::memcpy(d + off + o, stage + o, std::min(slice, m - o));
+                  },
+                  [&] {
+                    for (size_t i = 0; i < n && err == hipSuccess; i++) {
+                      err = hipEventSynchronize(c->chunk_ev[i]);
+                      ready.store(err == hipSuccess ? i + 1 : n + 1, std::memory_order_release);
+                    }
+                  });
+    LLG_HIP(err);
+  }
 }
 
 int resolve_level(const ll_gpu_graph* g, int level) {
@@ -210,6 +287,7 @@ void ll_gpu_destroy(ll_gpu_ctx* c) {
   for (auto e : c->timer.pool) (void)hipEventDestroy(e);
   for (auto& ev : c->pinned_ev)
     if (ev) (void)hipEventDestroy(ev);
+  for (auto& ev : c->chunk_ev) (void)hipEventDestroy(ev);
   if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->readback) (void)hipHostFree(c->readback);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -323,8 +401,14 @@ void upload_pages(ll_gpu_ctx* c, llgpu::VtEntry* dst, const std::vector<const vo
     const size_t n = std::min(per_half, src.size() - i0);
     LLG_HIP(hipEventSynchronize(c->pinned_ev[slot]));
     char* stage = static_cast<char*>(c->pinned) + slot * (c->pinned_bytes / 2);
-    for (size_t i = 0; i < n; i++)
-      std::memcpy(stage + i * page_bytes, src[i0 + i], entries[i0 + i] * sizeof(llgpu::VtEntry));
+    constexpr size_t kPages = 64;  // a pool thread moves this many pages at a time
+    auto move = [&](size_t b) {
+      for (size_t i = b * kPages; i < std::min(n, (b + 1) * kPages); i++)
+        std::memcpy(stage + i * page_bytes, src[i0 + i], entries[i0 + i] * sizeof(llgpu::VtEntry));
+    };
+    const size_t nb = (n + kPages - 1) / kPages;
+    if (nb > 1) c->copies.run(nb, move, [] {});
+    else move(0);
     LLG_HIP(hipMemcpyAsync(dst + i0 * kVtPageEntries, stage, n * page_bytes,
                            hipMemcpyHostToDevice, c->stream));
     LLG_HIP(hipEventRecord(c->pinned_ev[slot], c->stream));

@@ -12,6 +12,7 @@
 #include <string>
 #include <vector>
 
+#include "host_copy.h"
 #include "ll_gpu.h"
 
 namespace llgpu {
@@ -177,6 +178,8 @@ struct ll_gpu_ctx {
   void* pinned = nullptr;      // staging for uploads
   size_t pinned_bytes = 0;
   hipEvent_t pinned_ev[2] = {nullptr, nullptr};
+  std::vector<hipEvent_t> chunk_ev;  // results: one per staging chunk
+  llgpu::CopyPool copies;      // threads between the staging and the caller's arrays
   void* readback = nullptr;    // small pinned buffer for per-level counter reads
   std::map<std::string, int> tuned;    // autotuner decisions
   std::map<std::string, long> options; // ll_gpu_set_option knobs
@@ -405,6 +408,9 @@ const RowBlocks& ensure_rowblocks(ll_gpu_graph* g, uint32_t dir, int level, uint
 void build_rowblocks(ll_gpu_ctx* ctx, const Csr& c, uint32_t cap, uint32_t piece,
                      RowBlocks& rb);
 void drop_snapshots(ll_gpu_graph* g);
+// Copies `bytes` device bytes to the caller's array, ordered after the work on
+// the context's stream; returns when they are there.
+void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes);
 // inv[v] = position of v by descending `deg` (ties by ID).
 void degree_slots(ll_gpu_ctx* ctx, const uint32_t* deg, uint64_t V, DevBuf& inv);
 // Column segments of `in` (source IDs mapped through `inv` when given) with

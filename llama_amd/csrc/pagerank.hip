@@ -527,8 +527,7 @@ void widen_to_host(ll_gpu_graph* g, const float* dev, double* host, uint64_t n) 
   w.alloc(n * 8, s);
   k_widen<<<grid_for(n, 256), 256, 0, s>>>(dev, w.as<double>(), n);
   LLG_HIP(hipGetLastError());
-  LLG_HIP(hipMemcpyAsync(host, w.p, n * 8, hipMemcpyDeviceToHost, s));
-  LLG_HIP(hipStreamSynchronize(s));
+  copy_to_host(g->ctx, host, w.p, n * 8);
 }
 
 }  // namespace llgpu

@@ -128,8 +128,8 @@ int ll_gpu_pagerank_push(ll_gpu_graph* g, int level, int iters, double damping,
                                               last ? diff.as<double>() : nullptr);
       LLG_HIP(hipGetLastError());
     }
-    if (ranks_out) LLG_HIP(hipMemcpyAsync(ranks_out, rank.p, V * 8, hipMemcpyDeviceToHost, s));
-    if (last_diff) LLG_HIP(hipMemcpyAsync(last_diff, diff.p, 8, hipMemcpyDeviceToHost, s));
+    if (ranks_out) copy_to_host(ctx, ranks_out, rank.p, V * 8);
+    if (last_diff) copy_to_host(ctx, last_diff, diff.p, 8);
     LLG_HIP(hipStreamSynchronize(s));
     return LL_GPU_OK;
   } catch (const Error& e) {

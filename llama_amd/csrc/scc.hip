@@ -358,10 +358,7 @@ int ll_gpu_scc_ex(ll_gpu_graph* g, int level, int64_t* labels_out, uint64_t* num
     LLG_HIP(hipSetDevice(g->ctx->device));
     llgpu::DevBuf lab;
     llgpu::SccResult r = llgpu::scc_device(g, level, lab);
-    if (labels_out) {
-      LLG_HIP(hipMemcpyAsync(labels_out, lab.p, g->V * 8, hipMemcpyDeviceToHost, g->ctx->stream));
-      LLG_HIP(hipStreamSynchronize(g->ctx->stream));
-    }
+    if (labels_out) llgpu::copy_to_host(g->ctx, labels_out, lab.p, g->V * 8);
     if (num_scc) *num_scc = r.num_scc;
     if (sweeps) *sweeps = r.sweeps;
     return LL_GPU_OK;

@@ -501,6 +501,34 @@ const Csr& ensure_csr(ll_gpu_graph* g, uint32_t dir, int level) {
   return c;
 }
 
+namespace {
+
+__global__ void k_zero_count(unsigned long long* p) { *p = 0; }
+
+__global__ __launch_bounds__(256) void k_count_nonzero(const uint32_t* x, uint64_t n,
+                                                       unsigned long long* out) {
+  unsigned long long c = 0;
+  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += uint64_t(gridDim.x) * blockDim.x)
+    c += x[i] > 0 ? 1ull : 0ull;
+  block_atomic_add(out, c);
+}
+
+uint64_t count_nonzero(ll_gpu_ctx* ctx, const uint32_t* x, uint64_t n) {
+  hipStream_t s = ctx->stream;
+  DevBuf cnt;
+  cnt.alloc(8, s);
+  k_zero_count<<<1, 1, 0, s>>>(cnt.as<unsigned long long>());
+  k_count_nonzero<<<std::min(grid_for(n, 256), 4u * unsigned(ctx->num_cus)), 256, 0, s>>>(
+      x, n, cnt.as<unsigned long long>());
+  LLG_HIP(hipGetLastError());
+  uint64_t h = 0;
+  copy_to_host(ctx, &h, cnt.p, 8);
+  return h;
+}
+
+}  // namespace
+
 }  // namespace llgpu
 
 extern "C" {
@@ -518,10 +546,7 @@ int ll_gpu_snapshot_stats(ll_gpu_graph* g, int level, ll_gpu_snapshot_info* info
     uint64_t with_edges = 0;
     {
       const uint32_t* deg = llgpu::ensure_degrees(g, LL_GPU_DIR_OUT, level);
-      std::vector<uint32_t> h(g->V);
-      LLG_HIP(hipMemcpyAsync(h.data(), deg, g->V * 4, hipMemcpyDeviceToHost, g->ctx->stream));
-      LLG_HIP(hipStreamSynchronize(g->ctx->stream));
-      for (uint32_t d : h) with_edges += d > 0;
+      with_edges = llgpu::count_nonzero(g->ctx, deg, g->V);
     }
     info->continuations = c.segments >= with_edges ? c.segments - with_edges : 0;
     info->materialize_ms = c.ms;
@@ -541,10 +566,8 @@ int ll_gpu_snapshot_adjacency(ll_gpu_graph* g, int level, uint32_t dir, uint64_t
     LLG_HIP(hipSetDevice(g->ctx->device));
     const llgpu::Csr& c = llgpu::ensure_csr(g, dir, level);
     hipStream_t s = g->ctx->stream;
-    if (offsets)
-      LLG_HIP(hipMemcpyAsync(offsets, c.ofs.p, (c.V + 1) * 8, hipMemcpyDeviceToHost, s));
-    if (neighbours && c.E)
-      LLG_HIP(hipMemcpyAsync(neighbours, c.adj.p, c.E * 4, hipMemcpyDeviceToHost, s));
+    if (offsets) llgpu::copy_to_host(g->ctx, offsets, c.ofs.p, (c.V + 1) * 8);
+    if (neighbours && c.E) llgpu::copy_to_host(g->ctx, neighbours, c.adj.p, c.E * 4);
     LLG_HIP(hipStreamSynchronize(s));
     return LL_GPU_OK;
   } catch (const llgpu::Error& e) {
@@ -560,8 +583,7 @@ int ll_gpu_snapshot_degrees(ll_gpu_graph* g, int level, uint32_t dir, uint32_t* 
   try {
     LLG_HIP(hipSetDevice(g->ctx->device));
     const uint32_t* d = llgpu::ensure_degrees(g, dir, level);
-    LLG_HIP(hipMemcpyAsync(degrees, d, g->V * 4, hipMemcpyDeviceToHost, g->ctx->stream));
-    LLG_HIP(hipStreamSynchronize(g->ctx->stream));
+    llgpu::copy_to_host(g->ctx, degrees, d, g->V * 4);
     return LL_GPU_OK;
   } catch (const llgpu::Error& e) {
     g->ctx->err = e.msg;

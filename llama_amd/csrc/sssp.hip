@@ -525,7 +525,7 @@ int ll_gpu_sssp(ll_gpu_graph* g, int level, int64_t root, float* dist_out, uint6
         dist.as<uint32_t>(), V, cnt.as<unsigned long long>(),
         reinterpret_cast<uint32_t*>(cnt.as<unsigned long long>() + 1));
     LLG_HIP(hipGetLastError());
-    if (dist_out) LLG_HIP(hipMemcpyAsync(dist_out, dist.p, V * 4, hipMemcpyDeviceToHost, s));
+    if (dist_out) copy_to_host(ctx, dist_out, dist.p, V * 4);
     LLG_HIP(hipMemcpyAsync(ctx->readback, cnt.p, 16, hipMemcpyDeviceToHost, s));
     LLG_HIP(hipStreamSynchronize(s));
     if (reached) *reached = rb[0];

@@ -412,16 +412,16 @@ class DeviceGraph:
 
     def adjacency(self, direction: int, level: int = -1) -> tuple[np.ndarray, np.ndarray]:
         info = self.snapshot_info(level)
-        ofs = np.zeros(self.V + 1, np.uint64)
+        ofs = np.empty(self.V + 1, np.uint64)
         # in- and out-directions hold the same number of live edges
-        adj = np.zeros(max(int(info.live_edges), 1), np.uint32)
+        adj = np.empty(max(int(info.live_edges), 1), np.uint32)
         self.ctx.check(self.lib.ll_gpu_snapshot_adjacency(
             self._h, level, direction, ofs.ctypes.data_as(C.POINTER(C.c_uint64)),
             adj.ctypes.data_as(C.POINTER(C.c_uint32))))
         return ofs, adj[: int(ofs[-1])]
 
     def degrees(self, direction: int, level: int = -1) -> np.ndarray:
-        d = np.zeros(self.V, np.uint32)
+        d = np.empty(self.V, np.uint32)
         self.ctx.check(self.lib.ll_gpu_snapshot_degrees(self._h, level, direction,
                                                         d.ctypes.data_as(C.POINTER(C.c_uint32))))
         return d
@@ -429,7 +429,7 @@ class DeviceGraph:
     # ---- algorithms --------------------------------------------------------------
     def pagerank(self, iters: int = 10, damping: float = 0.85, level: int = -1,
                  cap: int = 0, want_ranks: bool = True) -> tuple[np.ndarray | None, float]:
-        out = np.zeros(self.V, np.float64) if want_ranks else None
+        out = np.empty(self.V, np.float64) if want_ranks else None
         diff = C.c_double()
         self.ctx.check(self.lib.ll_gpu_pagerank_ex(
             self._h, level, iters, damping, cap,
@@ -440,7 +440,7 @@ class DeviceGraph:
     def pagerank_push(self, iters: int = 10, damping: float = 0.85,
                       level: int = -1) -> tuple[np.ndarray, float]:
         """Push PageRank (FP64 atomics over out-edges): (ranks, last L1 change)."""
-        out = np.zeros(self.V, np.float64)
+        out = np.empty(self.V, np.float64)
         diff = C.c_double()
         self.ctx.check(self.lib.ll_gpu_pagerank_push(
             self._h, level, iters, damping, out.ctypes.data_as(C.POINTER(C.c_double)),
@@ -449,7 +449,7 @@ class DeviceGraph:
 
     def sssp(self, root: int, level: int = -1, want_dist: bool = True):
         """Weighted SSSP: (dist float32[V] or None, reached, max distance, rounds)."""
-        dist = np.zeros(self.V, np.float32) if want_dist else None
+        dist = np.empty(self.V, np.float32) if want_dist else None
         reached, mx, rounds = C.c_uint64(), C.c_double(), C.c_uint64()
         self.ctx.check(self.lib.ll_gpu_sssp(
             self._h, level, root,
@@ -460,14 +460,14 @@ class DeviceGraph:
     def bc(self, sources=None, level: int = -1) -> np.ndarray:
         """Betweenness centrality, FP32[V]: every vertex a source (bc_adj) when
         sources is None, else the given sources in order (bc_random)."""
-        out = np.zeros(self.V, np.float32)
         if sources is None:
             src, n = None, 0
         else:
             src = np.ascontiguousarray(sources, dtype=np.int64)
             n = src.size
             if n == 0:
-                return out
+                return np.zeros(self.V, np.float32)
+        out = np.empty(self.V, np.float32)
         self.ctx.check(self.lib.ll_gpu_bc(
             self._h, level, src.ctypes.data_as(C.POINTER(C.c_int64)) if src is not None else None,
             n, out.ctypes.data_as(C.POINTER(C.c_float))))
@@ -475,7 +475,7 @@ class DeviceGraph:
 
     def bfs(self, root: int, level: int = -1, want_levels: bool = True):
         """Direction-optimising BFS: (levels or None, reached, edges examined)."""
-        lv = np.zeros(self.V, np.int32) if want_levels else None
+        lv = np.empty(self.V, np.int32) if want_levels else None
         reached, exam, trav = C.c_uint64(), C.c_uint64(), C.c_uint64()
         self.ctx.check(self.lib.ll_gpu_bfs_ex(
             self._h, level, root, lv.ctypes.data_as(C.POINTER(C.c_int32)) if lv is not None
@@ -487,7 +487,7 @@ class DeviceGraph:
         """Multi-source BFS: (levels [n x V] or None, reached [n], pull sweeps)."""
         r = np.ascontiguousarray(roots, dtype=np.int64)
         n = r.size
-        lv = np.zeros((n, self.V), np.int32) if want_levels else None
+        lv = np.empty((n, self.V), np.int32) if want_levels else None
         reached = np.zeros(n, np.uint64)
         sweeps = C.c_uint64()
         self.ctx.check(self.lib.ll_gpu_bfs_batch_ex(
@@ -512,7 +512,7 @@ class DeviceGraph:
 
     def scc(self, level: int = -1, want_labels: bool = True):
         """Canonical SCC labels (min vertex ID per component) and the count."""
-        lab = np.zeros(self.V, np.int64) if want_labels else None
+        lab = np.empty(self.V, np.int64) if want_labels else None
         n, sweeps = C.c_uint64(), C.c_uint64()
         self.ctx.check(self.lib.ll_gpu_scc_ex(
             self._h, level, lab.ctypes.data_as(C.POINTER(C.c_int64)) if lab is not None else None,
@@ -524,7 +524,7 @@ class DeviceGraph:
                   batch_width: int = 0, level: int = -1, want_ranks: bool = True):
         """Batched personalized PageRank: (ranks [V x n] FP32 or None, iterations run)."""
         sd = np.ascontiguousarray(seeds, dtype=np.int64)
-        out = np.zeros((self.V, sd.size), np.float32) if want_ranks else None
+        out = np.empty((self.V, sd.size), np.float32) if want_ranks else None
         done = C.c_int()
         self.ctx.check(self.lib.ll_gpu_ppr_batch(
             self._h, level, sd.ctypes.data_as(C.POINTER(C.c_int64)), sd.size, iters, damping,

@@ -1,0 +1,59 @@
+"""Results and uploads through the staging buffer, at the sizes where the path
+changes: the read-back buffer (64 KiB), one chunk (1 MiB), chunks of 512 KiB
+and 2 MiB (8 MiB), and more than the staging holds (64 MiB)."""
+import threading
+
+import numpy as np
+import pytest
+
+from conftest import gpu_case
+from llama_amd.graph import DIR_IN, DIR_OUT, GpuContext, SlcsrGraph
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+def graph(ctx, V, E, seed):
+    rng = np.random.default_rng(seed)
+    begin = np.zeros(V + 1, np.int64)
+    begin[1:-1] = np.sort(rng.integers(0, E + 1, V - 1))
+    begin[-1] = E
+    vals = rng.integers(0, V, E)
+    return SlcsrGraph(ctx, V, (begin, vals), (begin, vals[::-1].copy())), begin, vals
+
+
+# bytes of the neighbour array
+@pytest.mark.parametrize("nbytes", [4, 65532, 65536, 65540, MB - 4, MB, MB + 4, 8 * MB - 4,
+                                    8 * MB + 4, 64 * MB, 64 * MB + 4, 133 * MB])
+def test_round_trip(ctx, nbytes):
+    gpu_case(f"host copy {nbytes} bytes")
+    V, E = 1000, nbytes // 4
+    dg, begin, vals = graph(ctx, V, E, nbytes)
+    for d, ref in ((DIR_OUT, vals), (DIR_IN, vals[::-1])):
+        ofs, adj = dg.adjacency(d)
+        assert np.array_equal(ofs, begin.astype(np.uint64))
+        assert np.array_equal(adj, ref.astype(np.uint32))
+    assert np.array_equal(dg.degrees(DIR_OUT), np.diff(begin).astype(np.uint32))
+
+
+def test_contexts_on_threads():
+    """Two contexts, a host thread each, copy at the same time."""
+    bad = []
+
+    def work(seed):
+        c = GpuContext(0)
+        dg, _, vals = graph(c, 50_000, 3_000_000, seed)
+        for _ in range(4):
+            if not np.array_equal(dg.adjacency(DIR_OUT)[1], vals.astype(np.uint32)):
+                bad.append(seed)
+        dg.close()
+        c.close()
+
+    gpu_case("host copy, two contexts")
+    ts = [threading.Thread(target=work, args=(s,)) for s in (1, 2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
