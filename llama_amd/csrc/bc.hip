@@ -393,14 +393,15 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
     for (int64_t i = 0; sources && i < n; i++)
       LLG_CHECK(sources[i] >= 0 && uint64_t(sources[i]) < V, LL_GPU_EINVAL,
                 "source outside [0, max_nodes)");
-    const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
-    const Csr& in = ensure_csr(g, LL_GPU_DIR_IN, level);
+    const BfsPrepared bfs = bfs_prepare(g, level);
+    const Csr& out = *bfs.out;
+    const Csr& in = *bfs.in;
     const RowBlocks& in_rb = ensure_rowblocks(g, LL_GPU_DIR_IN, level, kCap, kPiece);
     const RowBlocks& out_rb = ensure_rowblocks(g, LL_GPU_DIR_OUT, level, kCap, kPiece);
-    const uint32_t* outdeg = ensure_degrees(g, LL_GPU_DIR_OUT, level);
     const uint64_t nin = std::max<uint64_t>(in_rb.n, 1), nout = std::max<uint64_t>(out_rb.n, 1);
-    DevBuf lv, visited, st, bc, part, in_mask, out_mask, in_list, out_list, cnt, hub;
+    DevBuf lv, bfs_ws, st, bc, part, in_mask, out_mask, in_list, out_list, cnt, hub;
     lv.alloc(V * 4, s);
+    bfs_ws.alloc(bfs_work_bytes(V), s);
     st.alloc(V * sizeof(VState), s);
     bc.alloc(V * 4, s);
     part.alloc(std::max(nin, nout) * 4, s);
@@ -414,13 +415,11 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
     uint32_t* c_in = cnt.as<uint32_t>();
     uint32_t* c_out = c_in + 32;
     uint32_t* c_long = c_in + 64;
-    const uint64_t* dead = ensure_dead_rows(g, in);
     for (int64_t i = 0; i < ns; i++) {
       const uint32_t src = uint32_t(sources ? sources[i] : i);
       // the search's step count bounds the deepest level (a last step may
       // find nothing): a level without rows has an empty list
-      const int32_t D =
-          bfs_core(g, out, in, outdeg, src, dead, visited, lv.as<int32_t>()).levels;
+      const int32_t D = bfs_single_ws(g, bfs, src, bfs_ws.p, lv.as<int32_t>(), true).levels;
       k_bc_source_init<<<grid_for(V, 256), 256, 0, s>>>(lv.as<int32_t>(), st.as<VState>(), V,
                                                         src);
       k_fill_u64<<<1, 64, 0, s>>>(reinterpret_cast<unsigned long long*>(c_in), 48);

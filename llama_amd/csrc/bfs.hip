@@ -74,30 +74,28 @@ __device__ inline Counters* stripe(Counters* c) { return c + (blockIdx.x & (kStr
 
 // `excluded` (may be null) marks rows no search from this root enters; when
 // `alt` is given and the root's check set use_alt (Counters::aux of stripe
-// 0), `alt` is used instead.
+// 0), `alt` is used instead.  The root is the first frontier: level 0,
+// visited, queue[0]; its out-edges go to stripe 0.
 __global__ void k_bfs_init(int32_t* lv, uint64_t* visited, const uint64_t* excluded,
-                           const uint64_t* alt, const Counters* c, uint64_t V, uint64_t words) {
+                           const uint64_t* alt, Counters* c, uint64_t V, uint64_t words,
+                           uint32_t root, const uint32_t* outdeg, uint32_t* queue) {
   uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (alt && c->aux) excluded = alt;
-  if (lv && i < V) lv[i] = kUnreached;
+  if (lv && i < V) lv[i] = i == root ? 0 : kUnreached;
   if (i < words) {
     // bits beyond V (and excluded vertices) count as visited, so no step claims them
     uint64_t lo = i * 64;
     uint64_t w = 0;
     if (lo + 64 > V) w = V > lo ? ~((uint64_t(1) << (V - lo)) - 1) : ~uint64_t(0);
     if (excluded) w |= excluded[i];
+    if (i == (root >> 6)) w |= uint64_t(1) << (root & 63);
     visited[i] = w;
   }
-}
-
-__global__ void k_bfs_root(int32_t* lv, uint64_t* visited, uint32_t* queue, uint32_t root,
-                           const uint32_t* outdeg, Counters* c) {
-  if (lv) lv[root] = 0;
-  visited[root >> 6] |= uint64_t(1) << (root & 63);
-  queue[0] = root;
-  c->n_next = outdeg[root] > 0 ? 1 : 0;
-  c->m_next = outdeg[root];
-  c->examined = 0;
+  if (i == 0) {
+    queue[0] = root;
+    c->n_next = outdeg[root] > 0 ? 1 : 0;
+    c->m_next = outdeg[root];
+  }
 }
 
 __global__ void k_fill_u64(uint64_t* p, uint64_t n, uint64_t v) {
@@ -118,23 +116,33 @@ __global__ void k_zero_counters(Counters* c) {  // <<<sets, kStripes>>>
   zero_stripe(c + uint64_t(blockIdx.x) * kStripes + threadIdx.x);
 }
 
-// Counters::aux of stripe 0 = 1 when every vertex the search from `root` can
-// reach lies in the reach set R (the complement bitmap `notr` clear): the
-// root is in R, or all its out-neighbours are (R is closed under successors).
-// One workgroup.
-__global__ void k_reach_check(uint32_t root, const uint64_t* notr, const uint64_t* ofs,
-                              const uint32_t* adj, Counters* c) {
-  __shared__ int bad;
-  if (threadIdx.x == 0) bad = 0;
+// Whether every vertex the search from `root` can reach lies in the reach set
+// R (the complement bitmap `notr` clear): the root is in R, or all its
+// out-neighbours are (R is closed under successors).  Every thread of the
+// workgroup calls it; *bad is a word of LDS.
+__device__ inline bool stays_in_reach(uint32_t root, const uint64_t* notr, const uint64_t* ofs,
+                                      const uint32_t* adj, int* bad) {
+  if (threadIdx.x == 0) *bad = 0;
   __syncthreads();
   const bool in_r = !((notr[root >> 6] >> (root & 63)) & 1);
   if (!in_r)
     for (uint64_t e = ofs[root] + threadIdx.x; e < ofs[root + 1]; e += blockDim.x) {
       const uint32_t w = adj[e];
-      if ((notr[w >> 6] >> (w & 63)) & 1) bad = 1;
+      if ((notr[w >> 6] >> (w & 63)) & 1) *bad = 1;
     }
   __syncthreads();
-  if (threadIdx.x == 0) c->aux = (in_r || !bad) ? 1ull : 0ull;
+  return in_r || !*bad;
+}
+
+// Start of a search: `sets` counter sets to zero, and Counters::aux of stripe
+// 0 = 1 when the search may exclude the complement of R (notr null: 0).  One
+// workgroup.
+__global__ void k_search_start(uint32_t root, const uint64_t* notr, const uint64_t* ofs,
+                               const uint32_t* adj, Counters* c, int sets) {
+  __shared__ int bad;
+  for (int i = threadIdx.x; i < sets * kStripes; i += blockDim.x) zero_stripe(c + i);
+  const bool in = notr && stays_in_reach(root, notr, ofs, adj, &bad);
+  if (threadIdx.x == 0) c->aux = in ? 1ull : 0ull;
 }
 
 // Stage the calling lane's vertex (when it has out-edges) in the workgroup's
@@ -160,6 +168,75 @@ __device__ inline void wave_stage(bool take, uint32_t v, uint32_t outdeg, uint32
   if (take && outdeg > 0) lq[qbase + uint32_t(__popcll(mq & ((uint64_t(1) << lane) - 1)))] = v;
 }
 
+// The workgroup's staged vertices (lq, *lqn of them) to the next queue, one
+// reservation per workgroup.  Every thread calls it; *base is a word of LDS.
+__device__ inline void flush_stage(const uint32_t* lq, const uint32_t* lqn,
+                                   unsigned long long* base, uint32_t* q_next, Counters* c) {
+  __syncthreads();
+  if (threadIdx.x == 0 && *lqn) *base = atomicAdd(&c->n_next, (unsigned long long)*lqn);
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < *lqn; k += kBlock) q_next[*base + k] = lq[k];
+}
+
+// Claims v for the next level; true for the one claim that finds it unvisited.
+__device__ inline bool claim(uint32_t v, uint64_t* visited, int32_t* lv, int32_t next_lv) {
+  const uint64_t bit = uint64_t(1) << (v & 63);
+  if (visited[v >> 6] & bit) return false;
+  if (atomicOr((unsigned long long*)&visited[v >> 6], (unsigned long long)bit) & bit) return false;
+  if (lv) lv[v] = next_lv;
+  return true;
+}
+
+// Level 1, before the host has seen the root's degree: the root's out-edges
+// in blocks of kEdgesPerBlock over a fixed grid.
+__global__ __launch_bounds__(kBlock) void k_root_expand(uint32_t root, const uint64_t* ofs,
+                                                        const uint32_t* adj,
+                                                        const uint32_t* outdeg,
+                                                        uint64_t* visited, int32_t* lv,
+                                                        uint32_t* q_next, Counters* c) {
+  __shared__ uint32_t l_q[kEdgesPerBlock];
+  __shared__ uint32_t l_qn;
+  __shared__ unsigned long long l_qbase;
+  const uint64_t e0 = ofs[root], e1 = ofs[root + 1];
+  for (uint64_t x0 = e0 + uint64_t(blockIdx.x) * kEdgesPerBlock; x0 < e1;
+       x0 += uint64_t(gridDim.x) * kEdgesPerBlock) {
+    const uint64_t x1 = min(e1, x0 + kEdgesPerBlock);
+    if (threadIdx.x == 0) {
+      l_qn = 0;
+      atomicAdd(&stripe(c)->examined, (unsigned long long)(x1 - x0));
+    }
+    __syncthreads();
+    for (uint64_t base = x0; base < x1; base += kBlock) {
+      const uint64_t x = base + threadIdx.x;
+      bool take = false;
+      uint32_t v = 0, od = 0;
+      if (x < x1) {
+        v = adj[x];
+        take = claim(v, visited, lv, 1);
+        if (take) od = outdeg[v];
+      }
+      wave_stage(take, v, od, l_q, &l_qn, c);
+    }
+    flush_stage(l_q, &l_qn, &l_qbase, q_next, c);
+    __syncthreads();  // l_q and l_qn are reused
+  }
+}
+
+// Largest i in [0, n) with ofs[i] <= x (ofs ascending, ofs[0] <= x): a wave
+// probes 64 positions at a time.
+__device__ inline uint64_t wave_search(const uint64_t* ofs, uint64_t n, uint64_t x) {
+  const uint32_t lane = threadIdx.x & 63;
+  uint64_t lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const uint64_t step = (hi - lo + 63) / 64;
+    const uint64_t i = lo + lane * step;
+    const uint64_t m = __ballot(i < hi && ofs[i] <= x);
+    lo += (uint64_t(__popcll(m)) - 1) * step;
+    hi = min(hi, lo + step);
+  }
+  return lo;
+}
+
 __global__ __launch_bounds__(kBlock) void k_td_expand(
     const uint32_t* q, const uint64_t* qofs, uint64_t nq, uint64_t m_f, const uint64_t* ofs,
     const uint32_t* adj, const uint32_t* outdeg, uint64_t* visited, int32_t* lv, int32_t next_lv,
@@ -175,15 +252,13 @@ __global__ __launch_bounds__(kBlock) void k_td_expand(
   // the counter set of the next top-down level (read by the host before this
   // launch) starts at zero
   if (blockIdx.x == 0 && threadIdx.x < kStripes) zero_stripe(zero_next + threadIdx.x);
-  if (threadIdx.x == 0) {
-    uint64_t lo = 0, hi = nq;
-    while (hi - lo > 1) { uint64_t mid = (lo + hi) / 2; if (qofs[mid] <= x0) lo = mid; else hi = mid; }
-    sh_lo = lo;
-    uint64_t lo2 = lo, hi2 = nq;
-    while (hi2 - lo2 > 1) { uint64_t mid = (lo2 + hi2) / 2; if (qofs[mid] <= x1 - 1) lo2 = mid; else hi2 = mid; }
-    sh_hi = lo2;
-    l_qn = 0;
+  // first and last queue entry of the block, a wave each
+  if (threadIdx.x < 128) {
+    const bool second = threadIdx.x >= 64;
+    const uint64_t i = wave_search(qofs, nq, second ? x1 - 1 : x0);
+    if ((threadIdx.x & 63) == 0) *(second ? &sh_hi : &sh_lo) = i;
   }
+  if (threadIdx.x == 0) l_qn = 0;
   __syncthreads();
   const uint64_t lo = sh_lo;
   const uint32_t n = uint32_t(sh_hi - lo + 1);
@@ -200,25 +275,13 @@ __global__ __launch_bounds__(kBlock) void k_td_expand(
       uint32_t a = 0, b = n;
       while (b - a > 1) { uint32_t mid = (a + b) >> 1; if (l_qofs[mid] <= x) a = mid; else b = mid; }
       v = adj[l_base[a] + (x - l_qofs[a])];
-      const uint64_t bit = uint64_t(1) << (v & 63);
-      if (!(visited[v >> 6] & bit)) {
-        const uint64_t old = atomicOr((unsigned long long*)&visited[v >> 6], (unsigned long long)bit);
-        if (!(old & bit)) {
-          take = true;
-          if (lv) lv[v] = next_lv;
-          od = outdeg[v];
-        }
-      }
+      take = claim(v, visited, lv, next_lv);
+      if (take) od = outdeg[v];
     }
     wave_stage(take, v, od, l_q, &l_qn, c);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    atomicAdd(&stripe(c)->examined, (unsigned long long)(x1 - x0));
-    if (l_qn) l_qbase = atomicAdd(&c->n_next, (unsigned long long)l_qn);
-  }
-  __syncthreads();
-  for (uint32_t k = threadIdx.x; k < l_qn; k += kBlock) q_next[l_qbase + k] = l_q[k];
+  if (threadIdx.x == 0) atomicAdd(&stripe(c)->examined, (unsigned long long)(x1 - x0));
+  flush_stage(l_q, &l_qn, &l_qbase, q_next, c);
 }
 
 __global__ void k_queue_to_bitmap(const uint32_t* q, uint64_t n, uint64_t* bm) {
@@ -241,57 +304,70 @@ __global__ void k_queue_to_bitmap(const uint32_t* q, uint64_t n, uint64_t* bm) {
 // fixed grid over them.
 constexpr uint32_t kLongRow = 32;
 
-// Lists of the open rows, short and long, from the visited bitmap: a thread
-// per kOpenWords bitmap words, one list reservation (atomic) per workgroup and
-// list, rows in ascending order.  `merge` (may be null): a bitmap of rows
-// found by the level before, OR-ed into visited first (and written back);
-// `clear` (may be null): a bitmap zeroed over the same words (the level's
-// next frontier).  A row is long by the snapshot's long-row bitmap when one
-// is given, else by its offsets.
-constexpr int kOpenWords = 4;
+// Lists of the open rows, short and long, from the visited bitmap: a wave
+// takes `per` words (at most 64, a lane each), then writes the rows of one
+// word after another, a lane per row, so the stores are coalesced; one list
+// reservation (atomic) per workgroup and list, rows in ascending order within
+// it.  `merge` (may be null): a bitmap of rows found by the level before,
+// OR-ed into visited first (and written back); `clear` (may be null): a bitmap
+// zeroed over the same words (the level's next frontier).  A row is long by
+// the snapshot's long-row bitmap when one is given, else by its offsets.
+// With a thread per four words (its 256 rows one after another) a listing of
+// 131101 vertices took 23 to 92 us; now 3 to 5 us.
+constexpr int kOpenBlock = 1024;
+constexpr int kOpenWaves = kOpenBlock / 64;
 
-__global__ __launch_bounds__(kBlock) void k_open_rows(uint64_t* visited, const uint64_t* merge,
-                                                      uint64_t* clear, uint64_t words,
-                                                      const uint64_t* ofs,
-                                                      const uint64_t* longrows,
-                                                      uint32_t* rows_short, uint32_t* rows_long,
-                                                      Counters* c) {
-  __shared__ uint32_t wsum[2][kBlock / 64];
+// Words per wave: enough workgroups to spread a small bitmap, few enough that
+// the reservations of a large one do not queue on the two counters.
+inline uint32_t open_words_per_wave(uint64_t words) {
+  return uint32_t(std::min<uint64_t>(64, std::max<uint64_t>(4, words / 8192)));
+}
+
+__device__ inline uint64_t lane_u64(uint64_t x, uint32_t lane) {
+  const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(x)), int(lane)));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(x >> 32)), int(lane)));
+  return uint64_t(hi) << 32 | lo;
+}
+
+__global__ __launch_bounds__(kOpenBlock) void k_open_rows(uint64_t* visited,
+                                                          const uint64_t* merge, uint64_t* clear,
+                                                          uint64_t words, uint32_t per,
+                                                          const uint64_t* ofs,
+                                                          const uint64_t* longrows,
+                                                          uint32_t* rows_short,
+                                                          uint32_t* rows_long, Counters* c) {
+  __shared__ uint32_t wsum[2][kOpenWaves];
   __shared__ unsigned long long base[2];
-  const uint64_t w0 = (uint64_t(blockIdx.x) * kBlock + threadIdx.x) * kOpenWords;
-  uint64_t open[kOpenWords], longm[kOpenWords];
-  uint32_t nl = 0, ns = 0;
-#pragma unroll
-  for (int k = 0; k < kOpenWords; k++) {
-    const uint64_t w = w0 + uint64_t(k);
-    open[k] = 0;
-    longm[k] = 0;
-    if (w < words) {
-      uint64_t v = visited[w];
-      if (merge) {
-        v |= merge[w];
-        visited[w] = v;
-      }
-      if (clear) clear[w] = 0;
-      open[k] = ~v;  // padding bits are set in visited
-      if (longrows) {
-        longm[k] = open[k] & longrows[w];
-      } else {
-        for (uint64_t b = open[k]; b; b &= b - 1) {
-          const int i = __ffsll((long long)b) - 1;
-          const uint64_t r = w * 64 + uint64_t(i);
-          if (ofs[r + 1] - ofs[r] > kLongRow) longm[k] |= uint64_t(1) << i;
-        }
-      }
-      nl += uint32_t(__popcll(longm[k]));
-      ns += uint32_t(__popcll(open[k] & ~longm[k]));
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const uint64_t w0 = (uint64_t(blockIdx.x) * kOpenWaves + wave) * per;
+  const uint32_t n = w0 < words ? uint32_t(min(uint64_t(per), words - w0)) : 0u;
+  uint64_t open = 0, longm = 0;
+  if (lane < n) {
+    const uint64_t w = w0 + lane;
+    uint64_t v = visited[w];
+    if (merge) {
+      v |= merge[w];
+      visited[w] = v;
     }
+    if (clear) clear[w] = 0;
+    open = ~v;  // padding bits are set in visited
+    if (longrows) longm = open & longrows[w];
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (!longrows)
+    for (uint32_t k = 0; k < n; k++) {
+      const uint64_t o = lane_u64(open, k);
+      if (!o) continue;
+      const uint64_t r = (w0 + k) * 64 + lane;
+      const bool isl = ((o >> lane) & 1) && ofs[r + 1] - ofs[r] > kLongRow;
+      const uint64_t m = __ballot(isl);
+      if (lane == k) longm = m;
+    }
+  const uint32_t nl = uint32_t(__popcll(longm)), ns = uint32_t(__popcll(open & ~longm));
   uint32_t xs = ns, xl = nl;
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t ys = __shfl_up(xs, o, 64), yl = __shfl_up(xl, o, 64);
-    if (lane >= o) {
+    if (lane >= uint32_t(o)) {
       xs += ys;
       xl += yl;
     }
@@ -303,24 +379,29 @@ __global__ __launch_bounds__(kBlock) void k_open_rows(uint64_t* visited, const u
   __syncthreads();
   if (threadIdx.x < 2) {
     uint32_t t = 0;
-    for (int k = 0; k < kBlock / 64; k++) t += wsum[threadIdx.x][k];
+    for (int k = 0; k < kOpenWaves; k++) t += wsum[threadIdx.x][k];
     unsigned long long* dst = threadIdx.x == 0 ? &c->n_short : &c->n_long;
     base[threadIdx.x] = t ? atomicAdd(dst, (unsigned long long)t) : 0ull;
   }
   __syncthreads();
-  unsigned long long os = base[0] + xs - ns, ol = base[1] + xl - nl;
-  for (int k = 0; k < wave; k++) {
+  unsigned long long os = base[0], ol = base[1];
+  for (uint32_t k = 0; k < wave; k++) {
     os += wsum[0][k];
     ol += wsum[1][k];
   }
-#pragma unroll
-  for (int k = 0; k < kOpenWords; k++)
-    for (uint64_t b = open[k]; b; b &= b - 1) {
-      const int i = __ffsll((long long)b) - 1;
-      const uint32_t r = uint32_t((w0 + uint64_t(k)) * 64 + uint64_t(i));
-      if ((longm[k] >> i) & 1) rows_long[ol++] = r;
-      else rows_short[os++] = r;
+  const uint64_t below = (uint64_t(1) << lane) - 1;
+  for (uint32_t k = 0; k < n; k++) {
+    const uint64_t o = lane_u64(open, k);
+    if (!o) continue;
+    const uint64_t lm = lane_u64(longm, k);
+    const uint32_t r = uint32_t((w0 + k) * 64 + lane);
+    if ((o >> lane) & 1) {
+      if ((lm >> lane) & 1) rows_long[ol + uint32_t(__popcll(lm & below))] = r;
+      else rows_short[os + uint32_t(__popcll(o & ~lm & below))] = r;
     }
+    os += uint32_t(__popcll(o & ~lm));
+    ol += uint32_t(__popcll(lm));
+  }
 }
 
 __device__ inline void found_row(uint32_t r, int32_t* lv, int32_t next_lv, uint64_t* nbm) {
@@ -600,8 +681,150 @@ __global__ void k_dead_rows(const uint64_t* ofs, uint64_t V, uint64_t words, uin
   }
 }
 
-// Summed stripes (aux from stripe 0); with `extra`, one more device word is
-// read back in the same round trip into *extra_out.
+// A whole search by one workgroup, for graphs whose search costs less than the
+// launches and host round trips of the level-by-level form: visited, frontier
+// and next-frontier bitmaps and the frontier queues in LDS.  A level goes
+// top-down from the queue (the workgroup over one vertex's edges while the
+// queue is short, else a wave per vertex) until the frontier's out-edges
+// exceed the unexplored edges / alpha or a level finds more than kTinyQueue
+// vertices, bottom-up then (a thread per open row).  The counts go straight
+// to the host's read-back buffer.  Bound by the latency of one CU's loads, so
+// it stops where the whole chip catches up; us per search, counts only, this
+// form / level by level: 5000 vertices, 80000 edges 70 / 147; 20000, 320000
+// 119 / 215; 32000, 512000 137 / 153; 65000, 520000 262 / 180; 65000, 1.04 M
+// 263 / 156.
+constexpr uint64_t kTinyV = 32768;
+constexpr uint64_t kTinyE = 600000;
+constexpr uint32_t kTinyQueue = 4096;
+constexpr int kTinyBlock = 1024;
+struct TinyResult {
+  unsigned long long reached, examined, traversed, levels;
+};
+
+__global__ __launch_bounds__(kTinyBlock) void k_bfs_tiny(
+    uint32_t root, const uint64_t* fofs, const uint32_t* fadj, const uint32_t* fdeg,
+    const uint64_t* rofs, const uint32_t* radj, const uint64_t* excluded, const uint64_t* notr,
+    uint64_t E, uint64_t e_reach, uint32_t V, uint64_t alpha, int32_t* lv, uint64_t* visited,
+    TinyResult* out) {
+  constexpr uint32_t kWords = uint32_t(kTinyV / 64);
+  __shared__ unsigned long long vis[kWords], fr[kWords], nx[kWords];
+  __shared__ uint32_t q[2][kTinyQueue];
+  __shared__ uint32_t qn, found;
+  __shared__ unsigned long long m_next, exam;
+  __shared__ int bad;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t words = (V + 63) / 64;
+  if (notr && stays_in_reach(root, notr, fofs, fadj, &bad)) {
+    excluded = notr;
+    E = e_reach;
+  }
+  for (uint32_t i = tid; i < words; i += kTinyBlock) {
+    unsigned long long w = excluded ? excluded[i] : 0ull, f = 0;
+    if (i * 64 + 64 > V) w |= ~((1ull << (V - i * 64)) - 1);
+    if (i == (root >> 6)) {
+      f = 1ull << (root & 63);
+      w |= f;
+    }
+    vis[i] = w;
+    fr[i] = f;
+  }
+  if (lv)
+    for (uint32_t v = tid; v < V; v += kTinyBlock) lv[v] = v == root ? 0 : kUnreached;
+  if (tid == 0) {
+    q[0][0] = root;
+    exam = 0;
+  }
+  uint32_t nq = 1, n_f = 1;
+  uint64_t m_f = fdeg[root], m_vis = m_f, reached = 1;
+  int32_t lvl = 0;
+  int cur = 0;
+  while (n_f > 0 && m_f > 0) {
+    const uint64_t m_u = E > m_vis ? E - m_vis : 0;
+    const bool bottom_up = nq > kTinyQueue || m_f > m_u / alpha;
+    __syncthreads();  // the level before is read
+    for (uint32_t i = tid; i < words; i += kTinyBlock) nx[i] = 0;
+    if (tid == 0) {
+      qn = 0;
+      found = 0;
+      m_next = 0;
+    }
+    __syncthreads();
+    uint32_t my_found = 0;
+    unsigned long long my_m = 0, my_exam = 0;
+    auto take = [&](uint32_t v) {
+      if (lv) lv[v] = lvl + 1;
+      atomicOr(&nx[v >> 6], 1ull << (v & 63));
+      const uint32_t od = fdeg[v];
+      my_found++;
+      my_m += od;
+      if (od) {
+        const uint32_t p = atomicAdd(&qn, 1u);
+        if (p < kTinyQueue) q[cur ^ 1][p] = v;
+      }
+    };
+    if (!bottom_up) {
+      const bool all = nq < kTinyBlock / 64;  // the workgroup takes one vertex at a time
+      const uint32_t step = all ? kTinyBlock : 64, at = all ? tid : lane;
+      for (uint32_t k = all ? 0 : wave; k < nq; k += all ? 1 : kTinyBlock / 64) {
+        const uint32_t u = q[cur][k];
+        const uint64_t e1 = fofs[u + 1];
+        for (uint64_t e = fofs[u] + at; e < e1; e += step) {
+          const uint32_t v = fadj[e];
+          const unsigned long long bit = 1ull << (v & 63);
+          my_exam++;
+          if (!(vis[v >> 6] & bit) && !(atomicOr(&vis[v >> 6], bit) & bit)) take(v);
+        }
+      }
+    } else {
+      for (uint32_t r = tid; r < V; r += kTinyBlock) {
+        if ((vis[r >> 6] >> (r & 63)) & 1) continue;
+        const uint64_t hi = rofs[r + 1];
+        bool hit = false;
+        for (uint64_t e = rofs[r]; e < hi && !hit; e += 4) {
+          const uint32_t m = uint32_t(min(uint64_t(4), hi - e));
+          uint32_t u[4];
+#pragma unroll
+          for (uint32_t k = 0; k < 4; k++) u[k] = radj[e + (k < m ? k : 0)];
+#pragma unroll
+          for (uint32_t k = 0; k < 4; k++) {
+            if (k < m && !hit) {
+              my_exam++;
+              hit = (fr[u[k] >> 6] >> (u[k] & 63)) & 1;
+            }
+          }
+        }
+        if (hit) take(r);
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      my_found += __shfl_down(my_found, o, 64);
+      my_m += __shfl_down(my_m, o, 64);
+      my_exam += __shfl_down(my_exam, o, 64);
+    }
+    if (lane == 0) {
+      if (my_found) {
+        atomicAdd(&found, my_found);
+        atomicAdd(&m_next, my_m);
+      }
+      atomicAdd(&exam, my_exam);
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < words; i += kTinyBlock) {
+      fr[i] = nx[i];
+      vis[i] |= nx[i];
+    }
+    nq = qn;
+    n_f = found;
+    m_f = m_next;
+    m_vis += m_f;
+    reached += n_f;
+    cur ^= 1;
+    lvl++;
+  }
+  for (uint32_t i = tid; i < words; i += kTinyBlock) visited[i] = vis[i];  // own words
+  if (tid == 0) *out = TinyResult{reached, exam, m_vis, (unsigned long long)lvl};
+}
+
 // The summed stripes of n consecutive counter sets, one read-back.
 void read_counter_sets(ll_gpu_ctx* ctx, const Counters* c, int n, Counters* out) {
   static_assert(kBuBatch * kStripes * sizeof(Counters) <= kReadbackBytes,
@@ -623,25 +846,9 @@ void read_counter_sets(ll_gpu_ctx* ctx, const Counters* c, int n, Counters* out)
   }
 }
 
-Counters read_counters(ll_gpu_ctx* ctx, const Counters* c, const uint64_t* extra = nullptr,
-                       uint64_t* extra_out = nullptr) {
-  static_assert(kStripes * sizeof(Counters) + 8 <= kReadbackBytes,
-                "stripes fit the read-back buffer");
-  const Counters* st = static_cast<const Counters*>(ctx->readback);
-  uint64_t* ex = reinterpret_cast<uint64_t*>(static_cast<char*>(ctx->readback) +
-                                             kStripes * sizeof(Counters));
-  LLG_HIP(hipMemcpyAsync(ctx->readback, c, kStripes * sizeof(Counters), hipMemcpyDeviceToHost,
-                         ctx->stream));
-  if (extra) LLG_HIP(hipMemcpyAsync(ex, extra, 8, hipMemcpyDeviceToHost, ctx->stream));
-  LLG_HIP(hipStreamSynchronize(ctx->stream));
-  if (extra) *extra_out = *ex;
-  Counters h = st[0];
-  for (int i = 1; i < kStripes; i++) {
-    h.n_next += st[i].n_next;
-    h.m_next += st[i].m_next;
-    h.examined += st[i].examined;
-    h.found += st[i].found;
-  }
+Counters read_counters(ll_gpu_ctx* ctx, const Counters* c) {
+  Counters h;
+  read_counter_sets(ctx, c, 1, &h);
   return h;
 }
 
@@ -701,38 +908,55 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
   const uint64_t words = (V + 63) / 64;
   uint64_t* fbm = w.fbm;  // frontier / next-frontier bitmaps, swapped per bottom-up level
   uint64_t* nbm = w.nbm;
-  // set 0: the root and bottom-up levels; top-down levels alternate sets 1
-  // and 0, each expansion zeroing the other
-  k_zero_counters<<<2, kStripes, 0, s>>>(w.cnt);
-  if (notr)
-    k_reach_check<<<1, 256, 0, s>>>(root, notr, fwd.ofs.as<uint64_t>(), fwd.adj.as<uint32_t>(),
-                                    w.cnt);
-  else
-    k_fill_u64<<<1, 1, 0, s>>>(reinterpret_cast<uint64_t*>(&w.cnt->aux), 1, 0);
-  k_bfs_init<<<grid_for(std::max(V, words), 256), 256, 0, s>>>(lv, w.visited, excluded, notr,
-                                                              w.cnt, V, words);
-  k_bfs_root<<<1, 1, 0, s>>>(lv, w.visited, w.q[0], root, fdeg,
-                             w.cnt);
-  LLG_HIP(hipGetLastError());
-  Counters h = read_counters(ctx, w.cnt);
-  BfsResult r;
-  const unsigned bu_grid = 8u * unsigned(ctx->num_cus);
-  uint64_t nq = h.n_next;       // queue entries (vertices with out-edges)
-  uint64_t n_f = 1;             // frontier vertices
-  uint64_t m_f = h.m_next;      // frontier out-edges
-  uint64_t m_visited = h.m_next;
-  r.reached = 1;
-  bool bottom_up = false;
-  int td = 1;  // counter set of the next top-down level (zeroed)
-  int cur = 0;
-  int32_t lvl = 0;
-  // out-edges a search can still reach: those inside R when R excludes the rest
-  const uint64_t E = h.aux ? e_reach : fwd.E;
   const long a_opt = ctx->options.count("bfs_alpha") ? ctx->options["bfs_alpha"] : -1;
   const long b_opt = ctx->options.count("bfs_beta") ? ctx->options["bfs_beta"] : -1;
   const uint64_t alpha = a_opt > 0 ? uint64_t(a_opt) : 10;
+  BfsResult r;
+  if (V <= kTinyV && fwd.E <= kTinyE) {
+    MaybeTimed t(ctx, "k_bfs_tiny", w.timed);
+    auto* res = static_cast<TinyResult*>(ctx->readback);
+    k_bfs_tiny<<<1, kTinyBlock, 0, s>>>(root, fwd.ofs.as<uint64_t>(), fwd.adj.as<uint32_t>(),
+                                        fdeg, rev.ofs.as<uint64_t>(), rev.adj.as<uint32_t>(),
+                                        excluded, notr, fwd.E, e_reach, uint32_t(V), alpha, lv,
+                                        w.visited, res);
+    LLG_HIP(hipGetLastError());
+    LLG_HIP(hipStreamSynchronize(s));
+    r.reached = res->reached;
+    r.examined = res->examined;
+    r.traversed = res->traversed;
+    r.levels = int(res->levels);
+    return r;
+  }
+  // set 0: the root and bottom-up levels; top-down levels alternate sets 1
+  // and 2, each expansion zeroing the other.  Level 1 is expanded before the
+  // host has seen the root's degree (one round trip for both).
+  k_search_start<<<1, 256, 0, s>>>(root, notr, fwd.ofs.as<uint64_t>(), fwd.adj.as<uint32_t>(),
+                                   w.cnt, 3);
+  k_bfs_init<<<grid_for(std::max(V, words), 256), 256, 0, s>>>(
+      lv, w.visited, excluded, notr, w.cnt, V, words, root, fdeg, w.q[0]);
+  k_root_expand<<<64, kBlock, 0, s>>>(root, fwd.ofs.as<uint64_t>(), fwd.adj.as<uint32_t>(), fdeg,
+                                      w.visited, lv, w.q[1], w.cnt + kStripes);
+  LLG_HIP(hipGetLastError());
+  Counters h0[2];
+  read_counter_sets(ctx, w.cnt, 2, h0);
+  Counters h = h0[1];
+  const unsigned bu_grid = std::min(grid_for(V, kBlock), 8u * unsigned(ctx->num_cus));
+  const uint32_t open_per = open_words_per_wave(words);
+  const unsigned open_grid = grid_for(words, uint32_t(kOpenWaves) * open_per);
+  uint64_t nq = h.n_next;       // queue entries (vertices with out-edges)
+  uint64_t n_f = h.found;       // frontier vertices
+  uint64_t m_f = h.m_next;      // frontier out-edges
+  uint64_t m_visited = h0[0].m_next + h.m_next;
+  r.reached = 1 + h.found;
+  r.examined = h.examined;
+  bool bottom_up = false;
+  int td = 2;   // counter set of the next top-down level (zeroed)
+  int cur = 1;
+  int32_t lvl = h0[0].m_next > 0 ? 1 : 0;
+  // out-edges a search can still reach: those inside R when R excludes the rest
+  const uint64_t E = h0[0].aux ? e_reach : fwd.E;
   // beta 0: no return to top-down
-  const uint64_t beta = b_opt > 0 ? uint64_t(b_opt) : (h.aux ? 0 : 24);
+  const uint64_t beta = b_opt > 0 ? uint64_t(b_opt) : (h0[0].aux ? 0 : 24);
   while (n_f > 0 && m_f > 0) {
     const uint64_t m_u = E > m_visited ? E - m_visited : 0;
     if (!bottom_up && m_f > m_u / alpha) {
@@ -753,8 +977,8 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
           // bitmap); the last level's are never merged: no later step reads
           // visited in a search that stays bottom-up.  The next frontier's
           // bitmap is cleared in the same pass.
-          k_open_rows<<<grid_for(words, kBlock * kOpenWords), kBlock, 0, s>>>(
-              w.visited, fbm, nbm, words, rev.ofs.as<uint64_t>(), w.longrows, w.rows_short,
+          k_open_rows<<<open_grid, kOpenBlock, 0, s>>>(
+              w.visited, fbm, nbm, words, open_per, rev.ofs.as<uint64_t>(), w.longrows, w.rows_short,
               w.rows_long, ck);
           k_bu_short<<<bu_grid, kBlock, 0, s>>>(w.rows_short, rev.ofs.as<uint64_t>(),
                                                 rev.adj.as<uint32_t>(), fdeg, fbm, nbm, lv,
@@ -786,8 +1010,8 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
       k_zero_counters<<<1, kStripes, 0, s>>>(w.cnt);
       {
         MaybeTimed t(ctx, "k_bu_step", w.timed);
-        k_open_rows<<<grid_for(words, kBlock * kOpenWords), kBlock, 0, s>>>(
-            w.visited, nullptr, nbm, words, rev.ofs.as<uint64_t>(), w.longrows, w.rows_short,
+        k_open_rows<<<open_grid, kOpenBlock, 0, s>>>(
+            w.visited, nullptr, nbm, words, open_per, rev.ofs.as<uint64_t>(), w.longrows, w.rows_short,
             w.rows_long, w.cnt);
         k_bu_short<<<bu_grid, kBlock, 0, s>>>(w.rows_short, rev.ofs.as<uint64_t>(),
                                               rev.adj.as<uint32_t>(), fdeg, fbm, nbm, lv,
@@ -804,7 +1028,7 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
       k_td_expand<<<grid_for(m_f, kEdgesPerBlock), kBlock, 0, s>>>(
           w.q[cur], w.qofs, nq, m_f, fwd.ofs.as<uint64_t>(),
           fwd.adj.as<uint32_t>(), fdeg, w.visited, lv, lvl + 1,
-          w.q[cur ^ 1], cl, w.cnt + (1 - td) * kStripes);
+          w.q[cur ^ 1], cl, w.cnt + (3 - td) * kStripes);
     }
     LLG_HIP(hipGetLastError());
     h = read_counters(ctx, cl);
@@ -822,7 +1046,7 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
       if (beta > 0 && shrinking && n_f < V / beta) {
         bottom_up = false;
         // set 0 counts the queue; set 1 serves the next top-down level
-        k_zero_counters<<<2, kStripes, 0, s>>>(w.cnt);
+        k_zero_counters<<<3, kStripes, 0, s>>>(w.cnt);
         k_bitmap_to_queue<<<grid_for(words, kBlock), kBlock, 0, s>>>(
             fbm, V, fdeg, w.q[cur], w.cnt);
         LLG_HIP(hipGetLastError());
@@ -837,7 +1061,7 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
       n_f = n_next;
       m_f = h.m_next;
       cur ^= 1;
-      td ^= 1;
+      td = 3 - td;
     }
   }
   r.levels = lvl;
