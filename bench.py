@@ -326,6 +326,7 @@ def bench_tc(dg, E: int, V: int, args) -> dict:
     _, ms_w = ctx.kernel_time("k_tc_wave")
     _, ms_b = ctx.kernel_time("k_tc_block")
     _, ms_g = ctx.kernel_time("k_tc_global")
+    _, ms_c = ctx.kernel_time("k_tc_core")
     ctx.profile(False)
     t0 = time.perf_counter()
     tci = dg.tc_i()
@@ -335,11 +336,12 @@ def bench_tc(dg, E: int, V: int, args) -> dict:
     t_tci = time.perf_counter() - t0
     # B_TC: every intersection element read once (4 B) and one offset pair per vertex
     alg = 4 * work + 8 * V
-    k_ms = (ms_w + ms_b + ms_g) / args.tc_reps
+    k_ms = (ms_c + ms_w + ms_b + ms_g) / args.tc_reps
     out = {"triangles": tri, "repeat_equal": tri2 == tri, "dag_arcs": arcs, "work": work,
            "first_call_s": round(t_first, 4), "count_s": round(t, 4),
            "kernel_ms": round(k_ms, 3),
-           "kernel_ms_by_row_class": {"wave": round(ms_w / args.tc_reps, 3),
+           "kernel_ms_by_row_class": {"core": round(ms_c / args.tc_reps, 3),
+                                      "wave": round(ms_w / args.tc_reps, 3),
                                       "workgroup": round(ms_b / args.tc_reps, 3),
                                       "global": round(ms_g / args.tc_reps, 3)},
            "alg_bytes": alg,

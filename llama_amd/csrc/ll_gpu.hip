@@ -214,6 +214,7 @@ void drop_snapshots(ll_gpu_graph* g) {
   g->sym_adj.release();
   g->sym_mult.release();
   g->sym_rows.release();
+  g->tc_core = llgpu::TcCore();
   g->dead_level = -1;
   g->dead_in.release();
   g->reach_level = -1;

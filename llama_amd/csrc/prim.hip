@@ -436,8 +436,8 @@ void sort_pairs_u64_u32(const uint64_t* keys_in, uint64_t* keys_out, const uint3
 }
 
 void sort_pairs_u32_u32(const uint32_t* keys_in, uint32_t* keys_out, const uint32_t* vals_in,
-                        uint32_t* vals_out, uint64_t n, int end_bit, hipStream_t s) {
-  radix_sort<uint32_t, true>(keys_in, keys_out, vals_in, vals_out, n, end_bit, s);
+                        uint32_t* vals_out, uint64_t n, int end_bit, hipStream_t s, bool probe) {
+  radix_sort<uint32_t, true>(keys_in, keys_out, vals_in, vals_out, n, end_bit, s, probe);
 }
 
 void sort_pairs_u32_u32_split(const uint32_t* keys_in, uint32_t* keys_work,
@@ -448,8 +448,8 @@ void sort_pairs_u32_u32_split(const uint32_t* keys_in, uint32_t* keys_work,
 }
 
 void sort_keys_u64(const uint64_t* keys_in, uint64_t* keys_out, uint64_t n, int end_bit,
-                   hipStream_t s) {
-  radix_sort<uint64_t, false>(keys_in, keys_out, nullptr, nullptr, n, end_bit, s);
+                   hipStream_t s, bool probe) {
+  radix_sort<uint64_t, false>(keys_in, keys_out, nullptr, nullptr, n, end_bit, s, probe);
 }
 
 uint64_t unique_u64(const uint64_t* in, uint64_t* out, uint64_t n, hipStream_t s) {

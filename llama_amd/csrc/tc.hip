@@ -654,6 +654,16 @@ TcResult tc_device(ll_gpu_graph* g, int level, bool weighted) {
   ll_gpu_ctx* ctx = g->ctx;
   hipStream_t s = ctx->stream;
   const uint64_t V = g->V;
+  if (!weighted && ensure_tc_core(g, level)) {
+    TcResult r;
+    uint64_t maxrow = 0;
+    tc_core_count(g, &r.triangles, &r.work, &maxrow);
+    r.arcs = g->tc_core.arcs;
+    LLG_CHECK(r.arcs <= kOfsMask, LL_GPU_ERANGE, "oriented arcs beyond 2^48");
+    LLG_CHECK(maxrow < (1ull << 31), LL_GPU_ERANGE,
+              "a DAG row's neighbour lists hold 2^31 or more entries in total");
+    return r;
+  }
   ensure_dag(g, level);
   const uint64_t* ofs = g->sym_ofs.as<uint64_t>();
   const uint32_t* nbr = g->sym_adj.as<uint32_t>();

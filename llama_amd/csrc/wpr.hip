@@ -403,7 +403,7 @@ const WprMatrix& ensure_wpr_matrix(ll_gpu_graph* g, int level, bool forward) {
   int bits = 1;
   while (bits < 32 && ((V - 1) >> bits) != 0) bits++;
   sort_pairs_u32_u32(key.as<uint32_t>(), rows.as<uint32_t>(), pos.as<uint32_t>(),
-                     m.perm.as<uint32_t>(), E, bits, s);
+                     m.perm.as<uint32_t>(), E, bits, s, false);
   m.csr.ofs.alloc((V + 1) * 8, s);
   m.csr.adj.alloc(n * 4, s);
   k_row_offsets<<<grid_for(E + 1, 256), 256, 0, s>>>(rows.as<uint32_t>(), E, V,

@@ -1,0 +1,53 @@
+"""Triangle counts over the degree-numbered DAG: graphs within the core (32768
+vertices), past it with hubs (most lists in the core), past it with even
+degrees (many entries outside: the filter and its confirmation), and too even
+for it (the form by vertex ID), against the CPU count; W and the arcs equal
+the definition."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import gpu_case
+from llama_amd.graph import DeviceGraph, HostGraph
+
+pytestmark = pytest.mark.gpu
+
+
+def dag_stats(V, src, dst):
+    """Arcs and W = sum over arcs of d+(a) + d+(b), by the definition."""
+    deg = np.bincount(src, minlength=V) + np.bincount(dst, minlength=V)
+    k = src != dst
+    s, d = src[k], dst[k]
+    up = (deg[s] < deg[d]) | ((deg[s] == deg[d]) & (s < d))
+    a, b = np.where(up, s, d), np.where(up, d, s)
+    arcs = np.unique(a.astype(np.int64) * V + b)
+    a, b = arcs // V, arcs % V
+    dp = np.bincount(a, minlength=V)
+    return arcs.size, int((dp[a] + dp[b]).sum())
+
+
+def clustered(V, per, seed, skew):
+    """Edges with closed wedges: random pairs, then ends of two-edge paths."""
+    rng = np.random.default_rng(seed)
+    n = V * per // 2
+    s = (V * rng.random(n) ** skew).astype(np.int64)
+    d = (V * rng.random(n) ** skew).astype(np.int64)
+    near = (s + rng.integers(1, 40, n)) % V
+    return np.concatenate([s, s]), np.concatenate([d, near])
+
+
+@pytest.mark.parametrize("V,per,skew", [(3, 4, 1), (65, 30, 1), (2049, 40, 3), (32768, 10, 2),
+                                        (32769, 12, 2), (70001, 16, 4), (100003, 12, 1),
+                                        (220001, 8, 1), (250007, 10, 5)])
+def test_counts(ctx, V, per, skew):
+    gpu_case(f"tc core V={V} per={per} skew={skew}")
+    src, dst = clustered(V, per, V, skew)
+    g = HostGraph(V)
+    g.add_level(src, dst)  # duplicates, both directions and self-loops included
+    dg = DeviceGraph(ctx, g)
+    n, arcs, work = dg.triangles(stats=True)
+    assert n == oracle.OracleGraph.from_host(g).triangles()
+    assert (arcs, work) == dag_stats(V, src, dst)
+    assert dg.triangles() == n  # again, over the DAG already built
+    assert dg.tc_i() >= n
+    assert dg.triangles() == n
