@@ -307,10 +307,11 @@ int ll_gpu_tuned(ll_gpu_ctx* ctx, const char* prefix, int* value);
  * "pr_hot_bits" (hot/cold split of the pull at slot 2^N; 0 = off, -1 =
  * automatic = off), "sssp_delta_milli" (weighted SSSP near/far threshold
  * step in thousandths of the mean edge weight; 0 = no far pile, plain
- * Bellman-Ford rounds; -1 = automatic = 5), "sssp_min_queue" (once edges worth
+ * Bellman-Ford rounds; -1 = automatic = 5 from 2^24 vertices up, growing with
+ * the root of 2^24 / max_nodes below, to 160), "sssp_min_queue" (once edges worth
  * half the snapshot have been relaxed, the smallest queue a near/far phase
  * starts with when the far pile holds that many -- smaller queues rejoin the
- * pile; 0 = off, -1 = automatic = max_nodes / 32), "bfs_alpha" / "bfs_beta"
+ * pile; 0 = off, -1 = automatic = max_nodes / 8), "bfs_alpha" / "bfs_beta"
  * (direction-optimising BFS switches to bottom-up when the frontier's
  * out-edges exceed the unexplored edges / alpha, back to top-down when a
  * shrinking frontier holds under max_nodes / beta vertices; <= 0 = defaults:

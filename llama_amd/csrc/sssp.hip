@@ -6,12 +6,13 @@
 // The reference runs synchronous Bellman-Ford rounds over the vertices
 // updated in the previous round.  Here the rounds follow the near/far
 // schedule (Davidson, Baxter, Garland, Owens, IPDPS 2014): a round relaxes
-// the out-edges of a queue of vertices edge-parallel (LDS binary search over
-// the queue's degree prefix, as the top-down BFS does) with atomicMin on the
-// distances' bit patterns -- non-negative FP32 values order like their
+// the out-edges of a queue of vertices edge-parallel, in one launch, with
+// atomicMin on the distances' bit patterns -- non-negative FP32 values order like their
 // unsigned bit patterns.  A vertex whose distance dropped below the threshold
 // T is queued for the next round once (round stamp); one whose new distance is
-// >= T is flagged far.  When the queue runs dry, T grows by delta and the far
+// >= T is flagged far.  Rounds are launched several at a time: their queue
+// lengths and the decision whether a round runs stay on the device, and the
+// host reads them back per batch.  When the queue runs dry, T grows by delta and the far
 // vertices now below T whose distance changed since their edges were last
 // relaxed form the next queue.  Every order of relaxations ends at the same
 // fixed point, dist[v] = min over paths of the FP32 sums dist[u] + w taken in
@@ -21,6 +22,7 @@
 // reference stores them.
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstring>
 
 #include "ll_gpu_internal.h"
@@ -30,141 +32,298 @@ namespace llgpu {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr uint32_t kEdgesPerBlock = 2048;
+constexpr int kWaves = kBlock / 64;
 constexpr float kUnreachedDist = float(INT_MAX - 1);
-constexpr double kAutoDeltaMilli = 5;      // threshold step: 0.5% of the mean edge weight
-constexpr uint64_t kAutoMinQueueDiv = 32;  // smallest tail phase queue: V / 32 vertices
+constexpr uint64_t kAutoMinQueueDiv = 8;  // smallest tail phase queue: V / 8 vertices
+constexpr uint32_t kBigRow = 256;         // out-edges past which a queued vertex is shared by the grid
+constexpr uint32_t kChunk = 1024;         // edges of such a vertex one workgroup takes
+constexpr uint32_t kStage = 2048;         // appends a workgroup stages
+constexpr uint32_t kNotRelaxed = ~0u;     // a NaN pattern: equal to no distance; -1 as an int
+
+// A round's queue: n vertices of up to kBigRow out-edges, n_big chunks of
+// vertices with more; the edges relaxed by the round itself and by all rounds before it.  Rounds use
+// a ring of slots: round r reads slot r, fills slot r + 1 and zeroes slot r + 2.
+struct alignas(64) Slot {
+  unsigned long long n, n_big, edges, before;
+};
+constexpr int kSlots = 8;
+// rounds launched per host read-back; those past the end of a phase find an
+// empty queue
+constexpr int kBatch = 3;
+static_assert(kBatch + 3 <= kSlots, "the slots of a batch and its neighbours are distinct");
+
+struct Queues {
+  uint32_t* q[2];  // by round parity
+  uint2* big[2];   // {vertex, chunk}
+};
+
+struct RelaxArgs {
+  Queues qs;
+  Slot* slots;
+  const uint64_t* ofs;
+  const uint32_t* adj;
+  const float* w;
+  const uint32_t* outdeg;
+  uint32_t* dist;
+  int32_t* stamp;
+  uint8_t* far;
+  uint32_t* relaxed;
+  uint64_t E, min_queue;
+  uint32_t t_bits;
+  bool near_far;
+};
+
+// A vertex of more than kBigRow out-edges (d) joins its round's list, chunk by
+// chunk.  Several waves read its distance, which may drop meanwhile, so
+// `relaxed` keeps the largest one any of them used since the vertex last left
+// the far pile (as ints; the scatter resets it to -1, below every distance).
+// It is not reset when a round lists the vertex: chunks of it may still be
+// waiting in that same round, and a later small value would hide that the
+// earlier ones used a larger distance.
+__device__ inline void list_chunks(uint2* big, uint64_t at, uint32_t v, uint32_t d) {
+  for (uint32_t c = 0; c < (d + kChunk - 1) / kChunk; c++) big[at + c] = make_uint2(v, c);
+}
 
 __global__ void k_sssp_init(uint32_t* dist, int32_t* stamp, uint8_t* far, uint32_t* relaxed,
-                            uint64_t V, uint32_t root, uint32_t* queue) {
+                            uint64_t V, uint32_t root, const uint32_t* outdeg, Queues qs,
+                            Slot* slots, uint32_t* hist, uint32_t nhist) {
   const uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (v < V) {
     dist[v] = v == root ? __float_as_uint(0.0f) : __float_as_uint(kUnreachedDist);
-    stamp[v] = v == root ? 0 : -1;
-    far[v] = 0;
-    relaxed[v] = ~0u;  // a NaN pattern: equal to no distance
+    stamp[v] = -1;
+    relaxed[v] = kNotRelaxed;
   }
-  if (v == 0) queue[0] = root;  // a root without out-edges gives an empty first round
-}
-
-// Queue entry i: out-degree, and the distance its edges are relaxed with
-// (recorded in relaxed[v]; a later drop queues v again).
-__global__ void k_queue_prep(const uint32_t* q, uint64_t n, const uint64_t* ofs,
-                             const uint32_t* dist, uint32_t* d, uint32_t* qd,
-                             uint32_t* relaxed, unsigned long long* n_next) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i == 0) *n_next = 0;
-  if (i < n) {
-    const uint32_t v = q[i];
-    d[i] = uint32_t(ofs[v + 1] - ofs[v]);
-    const uint32_t x = dist[v];
-    qd[i] = x;
-    relaxed[v] = x;
-  }
-}
-
-// First and last queue entry of each relaxation block of kEdgesPerBlock
-// edges; the edge total m = qofs[nq] is read on the device (fixed grid).
-__global__ void k_relax_blocks(const uint64_t* qofs, uint64_t nq, uint64_t* blk) {
-  const uint64_t m = qofs[nq];
-  const uint64_t nblk = (m + kEdgesPerBlock - 1) / kEdgesPerBlock;
-  for (uint64_t b = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; b < nblk;
-       b += uint64_t(gridDim.x) * blockDim.x) {
-  const uint64_t x0 = b * kEdgesPerBlock, x1 = min(m, x0 + kEdgesPerBlock);
-  auto search = [&](uint64_t lo, uint64_t x) {  // largest i with qofs[i] <= x
-    uint64_t hi = nq;
-    while (hi - lo > 1) {
-      const uint64_t mid = (lo + hi) / 2;
-      if (qofs[mid] <= x) lo = mid;
-      else hi = mid;
+  if (v < (V + 3) / 4 * 4) far[v] = 0;
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < kSlots) {
+      Slot t{0, 0, 0, 0};
+      if (threadIdx.x == 0) {  // a root without out-edges gives an empty first round
+        const uint32_t d = outdeg[root];
+        t.n = d > 0 && d <= kBigRow ? 1 : 0;
+        t.n_big = d > kBigRow ? (d + kChunk - 1) / kChunk : 0;
+      }
+      slots[threadIdx.x] = t;
     }
-    return lo;
-  };
-  const uint64_t lo = search(0, x0);
-  blk[2 * b] = lo;
-  blk[2 * b + 1] = search(lo, x1 - 1);
+    for (uint32_t i = threadIdx.x; i < nhist; i += blockDim.x) hist[i] = i + 1 < nhist ? 0u : ~0u;
+  }
+  if (v == root) {
+    qs.q[0][0] = root;
+    if (outdeg[root] > kBigRow) list_chunks(qs.big[0], 0, root, outdeg[root]);
   }
 }
 
-// Relax the queue's out-edges.  An improved vertex with out-edges is
-// appended to the next queue once per round (stamp) when its distance is
-// below the threshold (bits t_bits), else flagged far.  An edge block's
-// appends are staged in LDS and reserved in the next queue with one atomic,
-// not one per wave: the queue counter is a single address every workgroup
-// adds to.
-__global__ __launch_bounds__(kBlock) void k_relax(const uint32_t* q, const uint32_t* qd,
-                                                  const uint64_t* qofs, uint64_t nq,
-                                                  const uint64_t* blk, const uint64_t* ofs,
-                                                  const uint32_t* adj, const float* w,
-                                                  uint32_t* dist, int32_t* stamp, uint8_t* far,
-                                                  uint32_t t_bits, int32_t round,
-                                                  uint32_t* q_next, unsigned long long* n_next) {
-  __shared__ uint64_t l_qofs[kEdgesPerBlock + 1];
-  __shared__ uint64_t l_base[kEdgesPerBlock];
-  __shared__ float l_dist[kEdgesPerBlock];
-  __shared__ uint32_t l_q[kEdgesPerBlock];  // at most one append per edge
-  __shared__ uint32_t l_qn;
-  __shared__ unsigned long long l_qbase;
-  const uint64_t m = qofs[nq];
-  const uint64_t nblk = (m + kEdgesPerBlock - 1) / kEdgesPerBlock;
+// Whether a round of n queued vertices runs: small queues rejoin the far pile
+// in the tail, once edges worth half the snapshot have been relaxed (early
+// phases keep the step).
+__host__ __device__ inline bool round_runs(uint64_t n, uint64_t done, uint64_t E,
+                                           uint64_t min_queue, bool near_far, bool force) {
+  return n > 0 && (!near_far || force || done * 2 < E || n >= min_queue);
+}
+
+// One edge: lowers the distance of its head; a head with out-edges whose
+// distance dropped below the threshold is queued for the next round once
+// (stamp), else flagged far.  Returns 1 (queue), 2 (queue, big row) or 0.
+__device__ inline int relax_edge(const RelaxArgs& a, uint32_t v, float cand, int32_t next) {
+  const uint32_t cb = __float_as_uint(cand);
+  if (cb >= a.dist[v] || cb >= atomicMin(&a.dist[v], cb)) return 0;
+  const uint32_t od = a.outdeg[v];
+  if (od == 0) return 0;
+  if (cb >= a.t_bits) {
+    a.far[v] = 1;
+    return 0;
+  }
+  if (atomicExch(&a.stamp[v], next) == next) return 0;
+  return od > kBigRow ? 2 : 1;
+}
+
+// Big vertices of a workgroup, staged in LDS so that their chunks take one
+// reservation on the list's counter (one each: 1.1 ms for the 30000 of a
+// split at 2^24 vertices).
+struct BigStage {
+  static constexpr uint32_t kRoom = 512;
+  uint32_t v[kRoom], at[kRoom];
+  uint32_t n, chunks;
+  unsigned long long base;
+
+  __device__ void clear() {  // one thread
+    n = 0;
+    chunks = 0;
+  }
+  __device__ void add(uint32_t x, uint32_t d, uint2* big, unsigned long long* n_big) {
+    const uint32_t k = (d + kChunk - 1) / kChunk;
+    const uint32_t i = atomicAdd(&n, 1u);
+    if (i < kRoom) {
+      v[i] = x;
+      at[i] = atomicAdd(&chunks, k);
+    } else {
+      list_chunks(big, atomicAdd(n_big, (unsigned long long)k), x, d);
+    }
+  }
+  // every thread of the workgroup, the stage complete; clears it
+  __device__ void flush(const uint32_t* outdeg, uint2* big, unsigned long long* n_big) {
+    __syncthreads();
+    const uint32_t m = min(n, kRoom);
+    if (m) {  // uniform
+      if (threadIdx.x == 0) base = atomicAdd(n_big, (unsigned long long)chunks);
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < m; i += kBlock) list_chunks(big, base + at[i], v[i], outdeg[v[i]]);
+      __syncthreads();
+      if (threadIdx.x == 0) clear();
+    }
+  }
+};
+
+// The calling wave's appends (take) to the workgroup's stage, or straight to
+// the queue once the stage is full: *l_end is the first position that did not
+// fit (every later one does not either), so the stage holds the positions
+// below min(*l_n, *l_end).
+__device__ inline void wave_append(bool take, uint32_t v, uint32_t* l_q, uint32_t* l_n,
+                                   uint32_t* l_end, uint32_t* q, unsigned long long* n) {
+  const uint64_t m = __ballot(take);
+  if (!m) return;
   const int lane = threadIdx.x & 63;
-  if (blockIdx.x == 0 && threadIdx.x == 0) n_next[1] = m;  // the round's edges, read back with n_next[0]
-  // equal-sized edge blocks: a fixed grid takes them in turn
-  for (uint64_t bi = blockIdx.x; bi < nblk; bi += gridDim.x) {
-    const uint64_t x0 = bi * kEdgesPerBlock;
-    const uint64_t x1 = min(m, x0 + kEdgesPerBlock);
-    const uint64_t lo = blk[2 * bi];
-    const uint32_t n = uint32_t(blk[2 * bi + 1] - lo + 1);
-    for (uint32_t i = threadIdx.x; i <= n; i += kBlock) {
-      l_qofs[i] = qofs[lo + i];
-      if (i < n) {
-        l_dist[i] = __uint_as_float(qd[lo + i]);
-        l_base[i] = ofs[q[lo + i]];
-      }
+  const int leader = __ffsll((long long)m) - 1;
+  const uint32_t k = uint32_t(__popcll(m));
+  const uint32_t rank = uint32_t(__popcll(m & ((uint64_t(1) << lane) - 1)));
+  uint32_t at = 0;
+  if (lane == leader) at = atomicAdd(l_n, k);
+  at = uint32_t(__shfl(int(at), leader, 64));
+  if (at + k <= kStage) {
+    if (take) l_q[at + rank] = v;
+  } else {
+    unsigned long long g = 0;
+    if (lane == leader) {
+      atomicMin(l_end, at);
+      g = atomicAdd(n, (unsigned long long)k);
     }
-    if (threadIdx.x == 0) l_qn = 0;
-    __syncthreads();
-    for (uint64_t base = x0; base < x1; base += kBlock) {
-      const uint64_t x = base + threadIdx.x;
-      bool take = false;
-      uint32_t v = 0;
-      if (x < x1) {
-        uint32_t a = 0, b = n;
-        while (b - a > 1) {
-          const uint32_t mid = (a + b) >> 1;
-          if (l_qofs[mid] <= x) a = mid;
-          else b = mid;
-        }
-        const uint64_t e = l_base[a] + (x - l_qofs[a]);
-        v = adj[e];
-        const float cand = l_dist[a] + w[e];
-        const uint32_t cb = __float_as_uint(cand);
-        if (cb < dist[v]) {
-          const uint32_t old = atomicMin(&dist[v], cb);
-          // only vertices with out-edges are queued: every queue entry then
-          // owns at least one edge, so an edge block spans at most
-          // kEdgesPerBlock entries (the LDS arrays above)
-          if (cb < old && ofs[v + 1] > ofs[v]) {
-            if (cb < t_bits) take = atomicExch(&stamp[v], round + 1) != round + 1;
-            else far[v] = 1;
-          }
-        }
-      }
-      const uint64_t mk = __ballot(take);
-      if (mk) {
-        const int leader = __ffsll((long long)mk) - 1;
-        uint32_t qb = 0;
-        if (lane == leader) qb = atomicAdd(&l_qn, uint32_t(__popcll(mk)));
-        qb = uint32_t(__shfl(int(qb), leader, 64));
-        if (take) l_q[qb + uint32_t(__popcll(mk & ((uint64_t(1) << lane) - 1)))] = v;
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && l_qn) l_qbase = atomicAdd(n_next, (unsigned long long)l_qn);
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < l_qn; k += kBlock) q_next[l_qbase + k] = l_q[k];
-    __syncthreads();  // the LDS slice and queue are reloaded for the next block
+    g = __shfl(g, leader, 64);
+    if (take) q[g + rank] = v;
   }
+}
+
+// One round in one launch over a fixed grid: no prefix sum of the queue's
+// degrees is needed.  A wave takes 64 queued vertices, scans their degrees in
+// registers and relaxes their edges flattened over its lanes; the workgroups
+// share the edges of the big ones.  Appends are staged in LDS and reserved
+// with one atomic per workgroup (the queue counter is a single address).
+// Bound by the gathers of the heads' distances and, in most rounds, by the
+// launch and the latency of the wave's dependent loads.  2^20 vertices, 16.8 M
+// edges: 4.19 -> 1.86 ms a search against one launch each for the queue's
+// degrees, their prefix sum, the blocks' bounds and the relaxation with a
+// round trip per round (2.34 with the same steps); 2^24 vertices 9.6 -> 8.3.
+// kBigRow 512: 2.01, 1024: 2.08; 64 queued vertices a wave whatever their
+// number: 6.6.
+__global__ __launch_bounds__(kBlock) void k_relax(RelaxArgs a, uint32_t round, bool force) {
+  __shared__ uint32_t l_pre[kWaves][64];
+  __shared__ uint64_t l_base[kWaves][64];
+  __shared__ float l_dist[kWaves][64];
+  __shared__ uint32_t l_q[kStage];
+  __shared__ uint32_t l_n, l_end;
+  __shared__ BigStage l_big;
+  __shared__ unsigned long long l_at;
+  Slot& cur = a.slots[round % kSlots];
+  Slot& nxt = a.slots[(round + 1) % kSlots];
+  const Slot& prev = a.slots[(round + kSlots - 1) % kSlots];
+  const unsigned long long done = prev.before + prev.edges;
+  const uint64_t n = cur.n, n_big = cur.n_big;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    cur.before = done;
+    a.slots[(round + 2) % kSlots] = Slot{0, 0, 0, 0};
+  }
+  if (!round_runs(n + n_big, done, a.E, a.min_queue, a.near_far, force)) return;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t* q = a.qs.q[round & 1];
+  uint32_t* q_next = a.qs.q[(round + 1) & 1];
+  uint2* big_next = a.qs.big[(round + 1) & 1];
+  const int32_t next = int32_t(round + 1);
+  if (threadIdx.x == 0) {
+    l_n = 0;
+    l_end = kStage;
+    l_big.clear();
+  }
+  __syncthreads();
+  unsigned long long edges = 0;
+  // entries a wave takes at a time: as few as spread the queue over the grid
+  const uint64_t waves = uint64_t(gridDim.x) * kWaves;
+  const uint32_t per = uint32_t(min(uint64_t(64), (n + waves - 1) / waves));
+  for (uint64_t i0 = (uint64_t(blockIdx.x) * kWaves + wave) * per; i0 < n; i0 += waves * per) {
+    uint32_t d = 0;
+    if (lane < per && i0 + lane < n) {
+      const uint32_t v = q[i0 + lane];
+      d = a.outdeg[v];
+      const uint32_t x = a.dist[v];
+      a.relaxed[v] = x;
+      l_dist[wave][lane] = __uint_as_float(x);
+      l_base[wave][lane] = a.ofs[v];
+    }
+    uint32_t inc = d;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(inc, o, 64);
+      if (lane >= uint32_t(o)) inc += y;
+    }
+    const uint32_t total = __shfl(inc, 63, 64);
+    l_pre[wave][lane] = inc;  // edges of the entries up to this one
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (lane == 0) edges += total;
+    for (uint32_t x0 = 0; x0 < total; x0 += 64 * 4) {
+      uint32_t head[4];
+      float cand[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const uint32_t x = x0 + 64u * uint32_t(k) + lane;
+        uint32_t lo = 0;  // the first entry with l_pre > x
+#pragma unroll
+        for (uint32_t h = 32; h > 0; h >>= 1)
+          if (l_pre[wave][lo + h - 1] <= x) lo += h;
+        lo = min(lo, 63u);
+        const uint64_t e = l_base[wave][lo] + (x - (lo ? l_pre[wave][lo - 1] : 0u));
+        const bool in = x < total;
+        head[k] = in ? a.adj[e] : 0u;
+        cand[k] = in ? l_dist[wave][lo] + a.w[e] : kUnreachedDist;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int r = x0 + 64u * uint32_t(k) + lane < total ? relax_edge(a, head[k], cand[k], next) : 0;
+        if (r == 2) l_big.add(head[k], a.outdeg[head[k]], big_next, &nxt.n_big);
+        wave_append(r == 1, head[k], l_q, &l_n, &l_end, q_next, &nxt.n);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();  // the wave's LDS is rewritten
+  }
+  // big vertices: a workgroup per chunk
+  const uint2* big = a.qs.big[round & 1];
+  for (uint64_t k = blockIdx.x; k < n_big; k += gridDim.x) {
+    const uint2 t = big[k];
+    const uint32_t v = t.x;
+    const uint64_t e0 = a.ofs[v];
+    const uint64_t lo = e0 + uint64_t(t.y) * kChunk, hi = min(e0 + a.outdeg[v], lo + kChunk);
+    // one read for the wave
+    const uint32_t xb = uint32_t(__shfl(int(lane == 0 ? a.dist[v] : 0u), 0, 64));
+    if (lane == 0) atomicMax(reinterpret_cast<int*>(&a.relaxed[v]), int(xb));
+    const float xd = __uint_as_float(xb);
+    if (threadIdx.x == 0) edges += hi - lo;
+    uint32_t head[kChunk / kBlock];
+    float cand[kChunk / kBlock];
+#pragma unroll
+    for (uint32_t u = 0; u < kChunk / kBlock; u++) {
+      const uint64_t e = lo + u * kBlock + threadIdx.x;
+      head[u] = e < hi ? a.adj[e] : 0u;
+      cand[u] = e < hi ? xd + a.w[e] : kUnreachedDist;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kChunk / kBlock; u++) {
+      const int r = lo + u * kBlock + threadIdx.x < hi ? relax_edge(a, head[u], cand[u], next) : 0;
+      if (r == 2) l_big.add(head[u], a.outdeg[head[u]], big_next, &nxt.n_big);
+      wave_append(r == 1, head[u], l_q, &l_n, &l_end, q_next, &nxt.n);
+    }
+  }
+  l_big.flush(a.outdeg, big_next, &nxt.n_big);
+  const uint32_t staged = min(l_n, l_end);
+  if (threadIdx.x == 0 && staged) l_at = atomicAdd(&nxt.n, (unsigned long long)staged);
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < staged; k += kBlock) q_next[l_at + k] = l_q[k];
+  block_atomic_add(&cur.edges, edges);
 }
 
 // The far pile.  far[v] = 1 marks a far vertex; a split bins every far
@@ -172,144 +331,118 @@ __global__ __launch_bounds__(kBlock) void k_relax(const uint32_t* q, const uint3
 // (bin 0 also holds anything below base + delta, the last bin everything past
 // the others) and stores the bin in far[v] as 2 + bin, so the scatter takes
 // exactly the vertices the histogram counted.  Far vertices whose edges were
-// relaxed with their current distance are dropped.  The kernels run over
-// fixed vertex ranges, one per workgroup, without shared counters.
-constexpr unsigned kSplitBlocks = 2048;
+// relaxed with their current distance are dropped.  hist[kBins] = the smallest
+// far distance's bits.
 constexpr unsigned kBins = 128;
-
-__device__ inline uint32_t split_range(uint64_t V) {
-  return uint32_t(((V + kSplitBlocks - 1) / kSplitBlocks + kBlock - 1) / kBlock * kBlock);
-}
 
 __global__ __launch_bounds__(kBlock) void k_far_hist(uint8_t* far, const uint32_t* dist,
                                                      const uint32_t* relaxed, uint64_t V,
-                                                     float base, float delta, uint32_t* hist,
-                                                     uint32_t* mins) {
+                                                     float base, float delta, uint32_t* hist) {
   __shared__ uint32_t h[kBins];
-  __shared__ uint32_t rm[kBlock / 64];
+  __shared__ uint32_t rm[kWaves];
   for (uint32_t i = threadIdx.x; i < kBins; i += kBlock) h[i] = 0;
   __syncthreads();
-  const uint32_t chunk = split_range(V);
-  const uint64_t v0 = uint64_t(blockIdx.x) * chunk, v1 = min(V, v0 + chunk);
   uint32_t mn = ~0u;
-  for (uint64_t v = v0 + threadIdx.x; v < v1; v += kBlock) {
-    if (!far[v]) continue;
-    const uint32_t d = dist[v];
-    if (d == relaxed[v]) {
-      far[v] = 0;
-      continue;
+  // four flags at a time (the array is padded to a multiple of four)
+  const uint64_t words = (V + 3) / 4;
+  for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < words;
+       i += uint64_t(gridDim.x) * kBlock) {
+    uint32_t f = reinterpret_cast<const uint32_t*>(far)[i];
+    if (!f) continue;
+    for (uint32_t k = 0; k < 4; k++) {
+      if (!((f >> (8 * k)) & 0xffu)) continue;
+      const uint64_t v = i * 4 + k;
+      const uint32_t d = dist[v];
+      uint32_t mark = 0;
+      if (d != relaxed[v]) {
+        const float x = (__uint_as_float(d) - base) / delta;
+        const uint32_t bin = x >= 1.0f ? uint32_t(min(x, float(kBins - 1))) : 0u;
+        mark = 2 + bin;
+        atomicAdd(&h[bin], 1u);
+        mn = min(mn, d);
+      }
+      f = (f & ~(0xffu << (8 * k))) | mark << (8 * k);
     }
-    const float x = (__uint_as_float(d) - base) / delta;
-    const uint32_t bin = x >= 1.0f ? uint32_t(min(x, float(kBins - 1))) : 0u;
-    far[v] = uint8_t(2 + bin);
-    atomicAdd(&h[bin], 1u);
-    mn = min(mn, d);
+    reinterpret_cast<uint32_t*>(far)[i] = f;
   }
   for (int o = 32; o > 0; o >>= 1) mn = min(mn, uint32_t(__shfl_xor(int(mn), o, 64)));
   if ((threadIdx.x & 63) == 0) rm[threadIdx.x >> 6] = mn;
   __syncthreads();
-  // stored as inclusive prefix counts: hist[range][b] = far vertices in bins <= b
+  for (uint32_t i = threadIdx.x; i < kBins; i += kBlock)
+    if (h[i]) atomicAdd(&hist[i], h[i]);
   if (threadIdx.x == 0) {
-    uint32_t run = 0;
-    for (uint32_t i = 0; i < kBins; i++) {
-      run += h[i];
-      h[i] = run;
-    }
-    for (int i = 1; i < kBlock / 64; i++) mn = min(mn, rm[i]);
-    mins[blockIdx.x] = mn;
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < kBins; i += kBlock) hist[uint64_t(blockIdx.x) * kBins + i] = h[i];
-}
-
-// Column sums of the per-range prefix counts, one workgroup per bin, and the
-// smallest far distance (workgroup kBins): tot[b] = far vertices in bins <= b,
-// tot[kBins] = the smallest distance's bits.
-__global__ __launch_bounds__(kBlock) void k_hist_total(const uint32_t* hist, const uint32_t* mins,
-                                                       unsigned long long* tot) {
-  __shared__ unsigned long long rs[kBlock / 64];
-  __shared__ uint32_t rm[kBlock / 64];
-  const uint32_t bin = blockIdx.x;
-  unsigned long long t = 0;
-  uint32_t mn = ~0u;
-  for (uint32_t r = threadIdx.x; r < kSplitBlocks; r += kBlock) {
-    if (bin < kBins) t += hist[uint64_t(r) * kBins + bin];
-    else mn = min(mn, mins[r]);
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    t += __shfl_xor(t, o, 64);
-    mn = min(mn, uint32_t(__shfl_xor(int(mn), o, 64)));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    rs[threadIdx.x >> 6] = t;
-    rm[threadIdx.x >> 6] = mn;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < kBlock / 64; i++) {
-      t += rs[i];
-      mn = min(mn, rm[i]);
-    }
-    tot[bin] = bin < kBins ? t : (unsigned long long)mn;
+    for (int i = 1; i < kWaves; i++) mn = min(mn, rm[i]);
+    if (mn != ~0u) atomicMin(&hist[kBins], mn);
   }
 }
 
-// Offsets of each range's taken vertices (bins 0..k), exclusive scan over the
-// ranges in one workgroup, kBlock ranges at a time.
-__global__ __launch_bounds__(kBlock) void k_far_offsets(const uint32_t* hist, uint32_t k,
-                                                        uint32_t* offs) {
-  __shared__ uint32_t part[kBlock];
-  __shared__ uint32_t carry;
-  if (threadIdx.x == 0) carry = 0;
-  for (uint32_t c0 = 0; c0 < kSplitBlocks; c0 += kBlock) {
-    const uint32_t i = c0 + threadIdx.x;
-    const uint32_t t = hist[uint64_t(i) * kBins + k];
-    part[threadIdx.x] = t;
-    __syncthreads();
-    for (uint32_t o = 1; o < kBlock; o <<= 1) {  // inclusive Hillis-Steele scan
-      const uint32_t x = threadIdx.x >= o ? part[threadIdx.x - o] : 0u;
-      __syncthreads();
-      part[threadIdx.x] += x;
-      __syncthreads();
-    }
-    offs[i] = carry + part[threadIdx.x] - t;
-    __syncthreads();
-    if (threadIdx.x == kBlock - 1) carry += part[kBlock - 1];
-    __syncthreads();
-  }
+__global__ void k_hist_zero(uint32_t* hist) {  // <<<1, kBins + 1>>>
+  hist[threadIdx.x] = threadIdx.x < kBins ? 0u : ~0u;
 }
 
-// Take the far vertices of bins 0..k into the queue, in vertex order.
+// Take the far vertices of bins 0..k into the queue of `slot`.  A workgroup
+// walks a contiguous range, stages what it takes and reserves queue entries
+// when the stage may overflow and at its end.  Workgroup 0 also clears the
+// histogram (read by the host) for the next split.
 __global__ __launch_bounds__(kBlock) void k_far_scatter(uint8_t* far, uint64_t V, uint32_t k,
-                                                        const uint32_t* offs, uint32_t* q) {
-  const uint32_t chunk = split_range(V);
-  const uint64_t v0 = uint64_t(blockIdx.x) * chunk, v1 = min(V, v0 + chunk);
-  __shared__ uint32_t wcnt[kBlock / 64];
-  uint32_t pos = offs[blockIdx.x];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (uint64_t b = v0; b < v1; b += kBlock) {
-    const uint64_t v = b + threadIdx.x;
-    const uint32_t f = v < v1 ? far[v] : 0u;
-    const bool take = f >= 2 && f - 2 <= k;
-    if (take) far[v] = 0;
-    const uint64_t mk = __ballot(take);
-    if (lane == 0) wcnt[wave] = uint32_t(__popcll(mk));
-    __syncthreads();
-    uint32_t before = 0, total = 0;
-    for (int i = 0; i < kBlock / 64; i++) {
-      before += i < wave ? wcnt[i] : 0u;
-      total += wcnt[i];
+                                                        const uint32_t* outdeg, uint32_t* relaxed,
+                                                        uint32_t* q, uint2* big, Slot* slot,
+                                                        uint32_t* hist) {
+  __shared__ uint32_t l_q[kStage];
+  __shared__ uint32_t l_n;
+  __shared__ BigStage l_big;
+  __shared__ unsigned long long l_at;
+  if (blockIdx.x == 0)
+    for (uint32_t i = threadIdx.x; i <= kBins; i += kBlock) hist[i] = i < kBins ? 0u : ~0u;
+  const uint64_t words = (V + 3) / 4;
+  const uint64_t per = (words + gridDim.x - 1) / gridDim.x;
+  const uint64_t w0 = uint64_t(blockIdx.x) * per, w1 = min(words, w0 + per);
+  if (threadIdx.x == 0) {
+    l_n = 0;
+    l_big.clear();
+  }
+  __syncthreads();
+  for (uint64_t b = w0; b < w1; b += kBlock) {
+    const uint64_t i = b + threadIdx.x;
+    uint32_t f = i < w1 ? reinterpret_cast<const uint32_t*>(far)[i] : 0u;
+    if (f) {
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t m = (f >> (8 * j)) & 0xffu;
+        if (m < 2 || m - 2 > k) continue;
+        f &= ~(0xffu << (8 * j));
+        const uint32_t v = uint32_t(i * 4 + j);
+        const uint32_t d = outdeg[v];
+        if (d > kBigRow) {
+          relaxed[v] = kNotRelaxed;
+          l_big.add(v, d, big, &slot->n_big);
+        } else {
+          l_q[atomicAdd(&l_n, 1u)] = v;  // at most 4 * kBlock per round
+        }
+      }
+      reinterpret_cast<uint32_t*>(far)[i] = f;
     }
-    if (take) q[pos + before + __popcll(mk & ((uint64_t(1) << lane) - 1))] = uint32_t(v);
-    pos += total;
+    __syncthreads();
+    const uint32_t n = l_n;
+    if (n > kStage - 4 * kBlock || b + kBlock >= w1) {  // uniform
+      if (threadIdx.x == 0 && n) l_at = atomicAdd(&slot->n, (unsigned long long)n);
+      __syncthreads();
+      for (uint32_t t = threadIdx.x; t < n; t += kBlock) q[l_at + t] = l_q[t];
+      __syncthreads();
+      if (threadIdx.x == 0) l_n = 0;
+    }
     __syncthreads();
   }
+  l_big.flush(outdeg, big, &slot->n_big);
 }
+static_assert(kStage >= 8 * kBlock, "a round of the scatter fits beside what is staged");
 
 // A queue too small for a round of its own rejoins the far pile.
-__global__ void k_queue_to_far(const uint32_t* q, uint64_t n, uint8_t* far) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) far[q[i]] = 1;
+__global__ void k_queue_to_far(const uint32_t* q, const uint2* big, const Slot* slot,
+                               uint8_t* far) {
+  const uint64_t n = slot->n, n_big = slot->n_big;
+  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n + n_big;
+       i += uint64_t(gridDim.x) * blockDim.x)
+    far[i < n ? q[i] : big[i - n].x] = 1;
 }
 
 // Sum of the edge weights (for the threshold step), FP64, fixed grid.
@@ -359,6 +492,19 @@ __global__ void k_sssp_summary(const uint32_t* dist, uint64_t V, unsigned long l
   }
 }
 
+// Threshold step in thousandths of the mean edge weight: 5 from 2^24 vertices
+// up, growing with the root of 2^24 / V below (to 160), since a phase of a
+// small graph costs its launches and the round trip more than repeated
+// relaxations.  ms by step (16 edges per vertex unless noted), the smallest
+// tail queue V / 8: 2000 vertices, 8 edges 10: 1.51, 20: 1.06, 160: 0.57;
+// 20000 10: 1.49, 20: 1.07, 145 (the rule) 0.73; 150000, 12 edges 10: 1.56,
+// 20: 1.28, 53 (rule) 1.02; 2^20 5: 2.4, 20 (rule) 1.86, 40: 2.1; 2^24 2:
+// 10.3, 5 (rule) 9.8, 10: 10.4 (before the staged big vertices).  V / 32 as
+// the smallest tail queue: 0.71, 0.87, 1.25, 2.43 at those sizes.
+double auto_delta_milli(uint64_t V) {
+  return std::min(160.0, std::max(5.0, 5.0 * std::sqrt(double(1 << 24) / double(V))));
+}
+
 __global__ void k_sssp_summary_init(unsigned long long* reached, uint32_t* max_bits) {
   *reached = 0;
   *max_bits = 0;
@@ -386,7 +532,7 @@ int ll_gpu_sssp(ll_gpu_graph* g, int level, int64_t root, float* dist_out, uint6
     // near/far threshold step in thousandths of the mean edge weight (0 = no
     // far pile: every improved vertex is queued)
     const long dm = ctx->options.count("sssp_delta_milli") ? ctx->options["sssp_delta_milli"] : -1;
-    const double delta_milli = dm < 0 ? kAutoDeltaMilli : double(dm);
+    const double delta_milli = dm < 0 ? auto_delta_milli(V) : double(dm);
     const auto* rb = static_cast<const unsigned long long*>(ctx->readback);
     if (delta_milli > 0 && out.w_mean < 0) {
       DevBuf sum;
@@ -413,89 +559,90 @@ int ll_gpu_sssp(ll_gpu_graph* g, int level, int64_t root, float* dist_out, uint6
     const long mq_opt = ctx->options.count("sssp_min_queue") ? ctx->options["sssp_min_queue"] : -1;
     const uint64_t min_queue = mq_opt < 0 ? std::max<uint64_t>(V / kAutoMinQueueDiv, 1)
                                           : uint64_t(mq_opt);
-    DevBuf dist, stamp, far, relaxed, q[2], qdeg, qd, qofs, cnt, blk, hist, tot;
+    const uint32_t* outdeg = ensure_degrees(g, LL_GPU_DIR_OUT, level);
+    DevBuf dist, stamp, far, relaxed, q[2], big[2], cnt, slots, hist;
     dist.alloc(V * 4, s);
     stamp.alloc(V * 4, s);
-    far.alloc(V, s);
+    far.alloc((V + 3) / 4 * 4, s);
     relaxed.alloc(V * 4, s);
-    q[0].alloc(V * 4, s);
-    q[1].alloc(V * 4, s);
-    qdeg.alloc(V * 4, s);
-    qd.alloc(V * 4, s);
-    qofs.alloc((V + 1) * 8, s);
+    // chunks of the vertices past kBigRow: at most their edges / kChunk, one more each
+    const uint64_t max_big = out.E / kChunk + out.E / kBigRow + 2;
+    for (int i = 0; i < 2; i++) {
+      q[i].alloc(V * 4, s);
+      big[i].alloc(max_big * sizeof(uint2), s);
+    }
     cnt.alloc(16, s);
-    hist.alloc((uint64_t(kSplitBlocks) * kBins + 2 * kSplitBlocks) * 4, s);
-    tot.alloc((kBins + 1) * 8, s);
-    uint32_t* h_bins = hist.as<uint32_t>();
-    uint32_t* h_mins = h_bins + uint64_t(kSplitBlocks) * kBins;
-    uint32_t* h_offs = h_mins + kSplitBlocks;
-    // a round queues each vertex once, so its edges are at most E
-    blk.alloc((out.E / kEdgesPerBlock + 1) * 16, s);
-    k_sssp_init<<<grid_for(V, 256), 256, 0, s>>>(dist.as<uint32_t>(), stamp.as<int32_t>(),
-                                                 far.as<uint8_t>(), relaxed.as<uint32_t>(), V,
-                                                 uint32_t(root), q[0].as<uint32_t>());
+    slots.alloc(kSlots * sizeof(Slot), s);
+    hist.alloc((kBins + 1) * 4, s);
+    RelaxArgs a{};
+    a.qs = Queues{{q[0].as<uint32_t>(), q[1].as<uint32_t>()},
+                  {big[0].as<uint2>(), big[1].as<uint2>()}};
+    a.slots = slots.as<Slot>();
+    a.ofs = out.ofs.as<uint64_t>();
+    a.adj = out.adj.as<uint32_t>();
+    a.w = out.w.as<float>();
+    a.outdeg = outdeg;
+    a.dist = dist.as<uint32_t>();
+    a.stamp = stamp.as<int32_t>();
+    a.far = far.as<uint8_t>();
+    a.relaxed = relaxed.as<uint32_t>();
+    a.E = out.E;
+    a.min_queue = min_queue;
+    a.near_far = near_far;
+    k_sssp_init<<<grid_for((V + 3) / 4 * 4, 256), 256, 0, s>>>(
+        a.dist, a.stamp, a.far, a.relaxed, V, uint32_t(root), outdeg, a.qs, a.slots,
+        hist.as<uint32_t>(), kBins + 1);
     LLG_HIP(hipGetLastError());
-    const unsigned relax_grid = 3u * unsigned(ctx->num_cus);  // 48 KB LDS per workgroup
-    uint64_t nq = 1, nrounds = 0;
-    int cur = 0;
+    const unsigned relax_grid = std::min(grid_for(V, 64), 4u * unsigned(ctx->num_cus));
+    const unsigned far_grid = std::min(grid_for((V + 3) / 4, kBlock), 4u * unsigned(ctx->num_cus));
+    uint64_t nrounds = 0;
+    uint32_t r = 0;      // slot number of the next round
     double T = near_far ? delta : double(kUnreachedDist);
-    uint32_t t_bits = near_far ? bits_of(T) : ~0u;
-    bool force = true;  // the root's queue, and a queue just taken from the far pile
+    a.t_bits = near_far ? bits_of(T) : ~0u;
+    bool force = true;   // the root's queue, and a queue just taken from the far pile
     uint64_t work_done = 0;  // edges relaxed so far
     for (;;) {
-      // small queues rejoin the far pile only in the tail, once edges worth
-      // half the snapshot have been relaxed: early phases keep the step delta
-      const bool tail = work_done * 2 >= out.E;
-      if (nq > 0 && (!near_far || force || !tail || nq >= min_queue)) {
-        // one round; one host round trip: the edge total stays on the device
-        k_queue_prep<<<grid_for(nq, 256), 256, 0, s>>>(
-            q[cur].as<uint32_t>(), nq, out.ofs.as<uint64_t>(), dist.as<uint32_t>(),
-            qdeg.as<uint32_t>(), qd.as<uint32_t>(), relaxed.as<uint32_t>(),
-            cnt.as<unsigned long long>());
-        scan_u32_to_u64(qdeg.as<uint32_t>(), qofs.as<uint64_t>(), nq, s);
-        k_relax_blocks<<<256, 256, 0, s>>>(qofs.as<uint64_t>(), nq, blk.as<uint64_t>());
-        {
-          TimedLaunch t(ctx, "k_relax");
-          k_relax<<<relax_grid, kBlock, 0, s>>>(
-              q[cur].as<uint32_t>(), qd.as<uint32_t>(), qofs.as<uint64_t>(), nq,
-              blk.as<uint64_t>(), out.ofs.as<uint64_t>(), out.adj.as<uint32_t>(),
-              out.w.as<float>(), dist.as<uint32_t>(), stamp.as<int32_t>(), far.as<uint8_t>(),
-              t_bits, int32_t(nrounds), q[cur ^ 1].as<uint32_t>(), cnt.as<unsigned long long>());
-        }
-        LLG_HIP(hipGetLastError());
-        LLG_HIP(hipMemcpyAsync(ctx->readback, cnt.p, 16, hipMemcpyDeviceToHost, s));
-        LLG_HIP(hipStreamSynchronize(s));
-        nq = rb[0];
-        work_done += rb[1];
-        nrounds++;
-        cur ^= 1;
-        force = false;
-        continue;
+      for (int k = 0; k < kBatch; k++) {
+        TimedLaunch t(ctx, "k_relax");
+        k_relax<<<relax_grid, kBlock, 0, s>>>(a, r + uint32_t(k), force && k == 0);
       }
+      LLG_HIP(hipGetLastError());
+      Slot h[kSlots];
+      LLG_HIP(hipMemcpyAsync(ctx->readback, slots.p, sizeof(h), hipMemcpyDeviceToHost, s));
+      LLG_HIP(hipStreamSynchronize(s));
+      std::memcpy(h, ctx->readback, sizeof(h));
+      int k = 0;
+      for (; k < kBatch; k++) {
+        const Slot& c = h[r % kSlots];
+        if (!round_runs(c.n + c.n_big, c.before, out.E, min_queue, near_far, force)) break;
+        work_done = c.before + c.edges;
+        force = false;
+        nrounds++;
+        r++;
+      }
+      if (k == kBatch) continue;
+      // the queue of slot r is empty, or too small for the tail
       if (!near_far) break;
-      if (nq > 0)
-        k_queue_to_far<<<grid_for(nq, 256), 256, 0, s>>>(q[cur].as<uint32_t>(), nq,
-                                                         far.as<uint8_t>());
+      if (h[r % kSlots].n + h[r % kSlots].n_big > 0)
+        k_queue_to_far<<<far_grid, kBlock, 0, s>>>(a.qs.q[r & 1], a.qs.big[r & 1],
+                                                   a.slots + r % kSlots, a.far);
       // split: histogram of the far pile in steps of delta above T
-      uint64_t c[kBins + 1];
+      uint32_t c[kBins + 1];
       for (;;) {
-        k_far_hist<<<kSplitBlocks, kBlock, 0, s>>>(far.as<uint8_t>(), dist.as<uint32_t>(),
-                                                   relaxed.as<uint32_t>(), V, float(T),
-                                                   float(delta), h_bins, h_mins);
-        k_hist_total<<<kBins + 1, kBlock, 0, s>>>(h_bins, h_mins, tot.as<unsigned long long>());
+        k_far_hist<<<far_grid, kBlock, 0, s>>>(a.far, a.dist, a.relaxed, V, float(T),
+                                               float(delta), hist.as<uint32_t>());
         LLG_HIP(hipGetLastError());
-        LLG_HIP(hipMemcpyAsync(ctx->readback, tot.p, sizeof(c), hipMemcpyDeviceToHost, s));
+        LLG_HIP(hipMemcpyAsync(ctx->readback, hist.p, sizeof(c), hipMemcpyDeviceToHost, s));
         LLG_HIP(hipStreamSynchronize(s));
         std::memcpy(c, ctx->readback, sizeof(c));
-        for (unsigned i = kBins - 1; i > 0; i--) c[i] -= c[i - 1];  // prefix -> per bin
         uint64_t below_last = 0;
         for (unsigned i = 0; i + 1 < kBins; i++) below_last += c[i];
         if (below_last > 0 || c[kBins - 1] == 0) break;
         // everything lies past the histogram: restart it at the smallest distance
         float mf;
-        const uint32_t mb = uint32_t(c[kBins]);
-        std::memcpy(&mf, &mb, 4);
+        std::memcpy(&mf, &c[kBins], 4);
         T = std::max(T, double(mf));
+        k_hist_zero<<<1, kBins + 1, 0, s>>>(hist.as<uint32_t>());
       }
       // from the first non-empty bin on, enough bins to hold min_queue
       // vertices (in the tail only), never past the last non-empty one
@@ -507,16 +654,16 @@ int ll_gpu_sssp(ll_gpu_graph* g, int level, int64_t root, float* dist_out, uint6
         }
       if (first < 0) break;  // the far pile is empty: done
       const uint64_t want = work_done * 2 >= out.E ? min_queue : 0;
-      uint32_t k = uint32_t(first);
-      uint64_t take = c[k];
-      while (int(k) < last && take < want) take += c[++k];
-      k_far_offsets<<<1, kBlock, 0, s>>>(h_bins, k, h_offs);
-      k_far_scatter<<<kSplitBlocks, kBlock, 0, s>>>(far.as<uint8_t>(), V, k, h_offs,
-                                                    q[cur].as<uint32_t>());
+      uint32_t kb = uint32_t(first);
+      uint64_t take = c[kb];
+      while (int(kb) < last && take < want) take += c[++kb];
+      r++;  // slot r may still hold the small queue; the next one is empty
+      k_far_scatter<<<far_grid, kBlock, 0, s>>>(a.far, V, kb, outdeg, a.relaxed, a.qs.q[r & 1],
+                                                a.qs.big[r & 1], a.slots + r % kSlots,
+                                                hist.as<uint32_t>());
       LLG_HIP(hipGetLastError());
-      T = k + 1 < kBins ? T + double(k + 1) * delta : double(kUnreachedDist);
-      t_bits = bits_of(T);
-      nq = take;
+      T = kb + 1 < kBins ? T + double(kb + 1) * delta : double(kUnreachedDist);
+      a.t_bits = bits_of(T);
       force = true;
     }
     k_sssp_summary_init<<<1, 1, 0, s>>>(cnt.as<unsigned long long>(),
@@ -535,7 +682,7 @@ int ll_gpu_sssp(ll_gpu_graph* g, int level, int64_t root, float* dist_out, uint6
       std::memcpy(&f, &bits, 4);
       *max_dist = double(f);
     }
-    if (rounds) *rounds = nrounds;
+    if (rounds) *rounds = std::max<uint64_t>(nrounds, 1);  // a root without out-edges: one, empty
     return LL_GPU_OK;
   } catch (const Error& e) {
     g->ctx->err = e.msg;
