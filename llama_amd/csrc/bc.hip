@@ -90,12 +90,38 @@ __device__ inline void finish(const BcArgs& a, uint32_t r, float S) {
   }
 }
 
+// v[lo] + v[lo + 1] + ... in that order, one lane.  Each addition waits for
+// the one before it; the LDS reads are kept kAhead terms ahead, so a row waits
+// for its additions alone and not for an LDS read at each.
+__device__ inline float ordered_sum(const float* v, uint32_t lo, uint32_t hi) {
+  constexpr uint32_t kAhead = 8;
+  float S = 0.0f;
+  uint32_t j = lo;
+  if (hi - lo >= 2 * kAhead) {
+    float cur[kAhead];
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; k++) cur[k] = v[j + k];
+    for (j += kAhead; j + kAhead <= hi; j += kAhead) {
+      float nxt[kAhead];
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) nxt[k] = v[j + k];
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) S = S + cur[k];
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; k++) cur[k] = nxt[k];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; k++) S = S + cur[k];
+  }
+  for (; j < hi; j++) S = S + v[j];
+  return S;
+}
+
 // One work item of a pass (all threads of the workgroup call it).
 template <bool kFwd>
 __device__ inline void bc_item(const BcArgs& a, uint64_t item) {
   __shared__ uint64_t rofs[kRowsPerItem + 1];
   __shared__ __align__(16) float vals[2][kMaxEdges];
-  __shared__ uint8_t rowof[kMaxEdges];
   __shared__ float srow[kRowsPerItem];
   __shared__ uint8_t onf[kRowsPerItem];
   __shared__ float red[kBlock / 64];
@@ -114,26 +140,28 @@ __device__ inline void bc_item(const BcArgs& a, uint64_t item) {
     if (threadIdx.x < nrows) {
       onf[threadIdx.x] = on ? 1 : 0;
       srow[threadIdx.x] = on && !kFwd ? a.st[r].sigma : 0.0f;
-      if (on)
-        for (uint32_t j = lo; j < hi; j++) rowof[j] = uint8_t(threadIdx.x);
     }
     __syncthreads();
-    // entries of rows off the level are neither loaded nor staged (rowof is
-    // written for rows on the level only, so the row's range is checked too);
-    // all neighbour IDs first, then their states, so the loads overlap
+    // entries of rows off the level are neither loaded nor staged; all
+    // neighbour IDs first, then their states, so the loads overlap
     uint32_t nb[kPer], rr[kPer];
     VState w[kPer];
     bool need[kPer];
 #pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) rr[k] = 0;
+    // an entry's row: the last row that starts at or before it
+#pragma unroll
+    for (uint32_t step = kRowsPerItem / 2; step > 0; step >>= 1) {
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; k++) {
+        const uint32_t m = rr[k] + step;
+        if (m < nrows && uint32_t(rofs[m] - e0) <= k * kBlock + threadIdx.x) rr[k] = m;
+      }
+    }
+#pragma unroll
     for (uint32_t k = 0; k < kPer; k++) {
       const uint32_t i = k * kBlock + threadIdx.x;
-      need[k] = false;
-      rr[k] = 0;
-      if (i < ne) {
-        rr[k] = rowof[i];
-        need[k] = rr[k] < nrows && onf[rr[k]] && i >= uint32_t(rofs[rr[k]] - e0) &&
-                  i < uint32_t(rofs[rr[k] + 1] - e0);
-      }
+      need[k] = i < ne && onf[rr[k]];
       nb[k] = need[k] ? a.adj[e0 + i] : 0u;
     }
 #pragma unroll
@@ -144,9 +172,7 @@ __device__ inline void bc_item(const BcArgs& a, uint64_t item) {
     __syncthreads();
     if (on) {
       // the row's terms in edge order, as the reference's loop adds them
-      float S = 0.0f;
-      for (uint32_t j = lo; j < hi; j++) S = S + vals[0][j];
-      finish<kFwd>(a, r, S);
+      finish<kFwd>(a, r, ordered_sum(vals[0], lo, hi));
     }
   } else if (!kFwd) {
     // Reverse pass, long row: k_bc_hub_terms has written the row's terms
