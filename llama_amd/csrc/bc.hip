@@ -11,13 +11,13 @@
 //                          for r != source,
 // in FP32 as the generated task code computes them.  Per source, each row
 // block item gets a mask of the levels its rows are on, and per level a list
-// of the items with a row there (long rows' pieces first); a pass launches one
+// of the items with a row there (long rows' pieces apart); a pass launches one
 // workgroup per item of its level's list.  Within an item only the edges of
-// rows on the level are loaded (an LDS map from entry to row masks the rest),
+// rows on the level are loaded (an entry finds its row by search over the item's offsets),
 // their terms staged in LDS, and each row sums its own terms sequentially in
 // edge order, so the reference's sums are reproduced bit for bit.  Long rows:
 // the forward pass reduces pieces in parallel (path counts are whole numbers,
-// exact in any order below 2^24) and joins them in piece order; for the
+// exact in any order below 2^24) and a wave joins them; for the
 // reverse pass their terms are computed piece-parallel into a buffer by edge
 // position first, then one lane adds them in edge order while the other waves
 // stage the next chunk.
@@ -34,6 +34,11 @@ namespace {
 constexpr int kBlock = 256;
 constexpr uint32_t kCap = 1024;  // row-block capacity of the path-count and dependency passes
 constexpr uint32_t kMaxEdges = kCap + kCap / 2;
+// Entries of one piece of a long row: one load per thread and entry slot, so a
+// piece has no loop of dependent chunks (pieces of 8192 entries took 15.6 us a
+// level for the reverse terms on 131101 vertices, a workgroup walking six
+// chunks while most of the chip was idle; these take 5.2).
+constexpr uint32_t kBcPiece = kMaxEdges;
 
 // Per-vertex Brandes state in one 16-byte record, so visiting a neighbour is
 // one load (level, path count and dependency together) instead of a level
@@ -78,6 +83,22 @@ __device__ inline VState load_state(const BcArgs& a, bool need, uint32_t nb) {
   v.delta = 0.0f;
   v.pad = 0.0f;
   return v;
+}
+
+// The states of the neighbours of a long row's piece, entry k * kBlock +
+// threadIdx.x in w[k]; past the piece the off-level placeholder.
+__device__ inline void load_piece(const BcArgs& a, uint32_t r, uint32_t piece, VState (&w)[kPer]) {
+  const uint64_t lo = a.ofs[r] + uint64_t(piece) * kBcPiece;
+  const uint64_t hi = min(a.ofs[r + 1], lo + kBcPiece);
+  uint32_t nb[kPer];
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    const uint64_t e = lo + k * kBlock + threadIdx.x;
+    nb[k] = e < hi ? a.adj[e] : 0u;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; k++)
+    w[k] = load_state(a, lo + k * kBlock + threadIdx.x < hi, nb[k]);
 }
 
 template <bool kFwd>
@@ -236,23 +257,11 @@ __device__ inline void bc_item(const BcArgs& a, uint64_t item) {
     // order below 2^24; pieces reduce in parallel, k_bc_fixup joins them.
     const uint32_t r = it.row_begin;
     if (a.st[r].lv != a.d) return;  // uniform over the workgroup
-    const uint64_t lo = a.ofs[r] + uint64_t(it.piece) * kPiece;
-    const uint64_t hi = min(a.ofs[r + 1], lo + kPiece);
+    VState w[kPer];
+    load_piece(a, r, it.piece, w);
     float S = 0.0f;
-    for (uint64_t c0 = lo; c0 < hi; c0 += kMaxEdges) {
-      uint32_t nb[kPer];
-      VState w[kPer];
 #pragma unroll
-      for (uint32_t k = 0; k < kPer; k++) {
-        const uint64_t e = c0 + k * kBlock + threadIdx.x;
-        nb[k] = e < hi ? a.adj[e] : 0u;
-      }
-#pragma unroll
-      for (uint32_t k = 0; k < kPer; k++)
-        w[k] = load_state(a, c0 + k * kBlock + threadIdx.x < hi, nb[k]);
-#pragma unroll
-      for (uint32_t k = 0; k < kPer; k++) S = S + term<true>(a, w[k], 0.0f);
-    }
+    for (uint32_t k = 0; k < kPer; k++) S = S + term<true>(a, w[k], 0.0f);
     for (int o = 32; o > 0; o >>= 1) S = S + __shfl_down(S, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = S;
     __syncthreads();
@@ -265,94 +274,92 @@ __device__ inline void bc_item(const BcArgs& a, uint64_t item) {
   }
 }
 
+// A level's items: long rows' pieces from the front of its list, the other
+// items from the back, so one launch fills both and each part's count bounds
+// the launch that reads it.
+struct LevelList {
+  const uint32_t* list;
+  uint32_t n;        // capacity (items of the direction)
+  uint32_t nlong;    // entries at the front
+  __device__ uint32_t at(uint32_t i) const {
+    return i < nlong ? list[i] : list[n - 1 - (i - nlong)];
+  }
+};
+
 // A pass: one workgroup per item of the level's list.
 template <bool kFwd>
-__global__ __launch_bounds__(kBlock) void k_bc_pass(BcArgs a, const uint32_t* list) {
-  bc_item<kFwd>(a, list[blockIdx.x]);
+__global__ __launch_bounds__(kBlock) void k_bc_pass(BcArgs a, LevelList l) {
+  bc_item<kFwd>(a, l.at(blockIdx.x));
 }
 
 // Reverse pass, long rows on the level: each piece writes its edges' terms
-// to a.hub at their out-edge positions (the list's first items are the long
-// rows' pieces).
-__global__ __launch_bounds__(kBlock) void k_bc_hub_terms(BcArgs a, const uint32_t* list) {
-  const RowItem it = a.items[list[blockIdx.x]];
+// to a.hub at their out-edge positions.
+__global__ __launch_bounds__(kBlock) void k_bc_hub_terms(BcArgs a, LevelList l) {
+  const RowItem it = a.items[l.list[blockIdx.x]];
   const uint32_t r = it.row_begin;
   if (a.st[r].lv != a.d) return;
-  const uint64_t lo = a.ofs[r] + uint64_t(it.piece) * kPiece;
-  const uint64_t hi = min(a.ofs[r + 1], lo + kPiece);
+  const uint64_t lo = a.ofs[r] + uint64_t(it.piece) * kBcPiece;
+  const uint64_t hi = min(a.ofs[r + 1], lo + kBcPiece);
   const float sr = a.st[r].sigma;
-  for (uint64_t c0 = lo; c0 < hi; c0 += kMaxEdges) {
-    uint32_t nb[kPer];
-    VState w[kPer];
+  VState w[kPer];
+  load_piece(a, r, it.piece, w);
 #pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) {
-      const uint64_t e = c0 + k * kBlock + threadIdx.x;
-      nb[k] = e < hi ? a.adj[e] : 0u;
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) w[k] = load_state(a, c0 + k * kBlock + threadIdx.x < hi, nb[k]);
-#pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) {
-      const uint64_t e = c0 + k * kBlock + threadIdx.x;
-      if (e < hi) a.hub[e] = term<false>(a, w[k], sr);
-    }
+  for (uint32_t k = 0; k < kPer; k++) {
+    const uint64_t e = lo + k * kBlock + threadIdx.x;
+    if (e < hi) a.hub[e] = term<false>(a, w[k], sr);
   }
 }
 
-// Level lists: list[l * n + j] = the j-th item with a row on level l (levels
-// >= 31 share list 31), counts in cnt[l].  Called for the long rows' pieces
-// first and then for the other items, so each list starts with its long rows.
-// Positions come from one global atomic per workgroup and level (the waves
-// take their slots in the workgroup's share from an LDS counter).
-constexpr unsigned kListBlock = 1024;  // workgroup of k_level_lists
-
-__global__ __launch_bounds__(kListBlock) void k_level_lists(const RowItem* items, uint64_t n,
-                                                            const uint32_t* mask, bool long_rows,
-                                                            uint32_t* list, uint32_t* cnt) {
-  constexpr uint32_t kWaves = kListBlock / 64;
-  __shared__ uint32_t bcount[32], bbase[32], woff[kWaves][32];
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t m = 0;
-  if (i < n && (items[i].npieces != 0) == long_rows) m = mask[i];
-  if (threadIdx.x < 32) bcount[threadIdx.x] = 0;
-  __syncthreads();
-  uint32_t wm = m;
-  for (int o = 32; o > 0; o >>= 1) wm |= __shfl_xor(wm, o, 64);
-  // the wave's slot in the workgroup's share of each level's list
-  for (uint32_t x = wm; x;) {
-    const uint32_t l = uint32_t(__builtin_ctz(x));
-    x &= x - 1;
-    const uint64_t b = __ballot((m >> l) & 1u);
-    if (lane == uint32_t(__builtin_ctzll(b))) woff[wave][l] = atomicAdd(&bcount[l], uint32_t(__popcll(b)));
-  }
-  __syncthreads();
-  // one global atomic per workgroup and level
-  if (threadIdx.x < 32 && bcount[threadIdx.x])
-    bbase[threadIdx.x] = atomicAdd(&cnt[threadIdx.x], bcount[threadIdx.x]);
-  __syncthreads();
-  for (uint32_t x = wm; x;) {
-    const uint32_t l = uint32_t(__builtin_ctz(x));
-    x &= x - 1;
-    const uint64_t b = __ballot((m >> l) & 1u);
-    if ((m >> l) & 1u) {
-      const uint64_t below = lane ? (b & (~0ull >> (64 - lane))) : 0ull;
-      list[uint64_t(l) * n + bbase[l] + woff[wave][l] + uint32_t(__popcll(below))] = uint32_t(i);
-    }
-  }
-}
-
-__global__ void k_copy_u32(const uint32_t* src, uint32_t* dst, uint32_t n) {
-  if (threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
-}
-
-// Per item, the levels its rows are on (bit min(level, 31)), one wave per item.
-__global__ void k_item_levels(const RowItem* items, uint64_t n, const int32_t* lv,
-                              uint32_t* mask) {
+// Forward pass, rows split over several pieces: combine the partials, one
+// wave per listed piece (the first piece of a row joins them); launched for
+// the levels with long rows only, over their pieces.
+__global__ __launch_bounds__(kBlock) void k_bc_fixup(BcArgs a, LevelList l) {
   const uint32_t lane = threadIdx.x & 63;
-  const uint64_t nw = (uint64_t(gridDim.x) * blockDim.x) >> 6;
-  for (uint64_t i = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6; i < n; i += nw) {
-    const RowItem it = items[i];
+  const uint32_t i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (i >= l.nlong) return;
+  const uint32_t item = l.list[i];
+  const RowItem it = a.items[item];
+  if (it.npieces <= 1 || it.piece != 0 || a.st[it.row_begin].lv != a.d) return;
+  float t = 0.0f;
+  for (uint32_t p = lane; p < it.npieces; p += 64) t = t + a.part[item + p];
+  for (int o = 32; o > 0; o >>= 1) t = t + __shfl_down(t, o, 64);
+  if (lane == 0) finish<true>(a, it.row_begin, t);
+}
+
+// One direction's items and what a source's lists need of them.
+struct LevelItems {
+  const RowItem* items;
+  uint64_t n;
+  uint32_t* mask;   // per item, the levels its rows are on (bit min(level, 31))
+  uint32_t* list;   // 32 x n
+  uint32_t* nlong;  // 32 counts: long rows' pieces
+  uint32_t* nshort; // 32 counts: the other items
+};
+
+// Start of a source, one launch (a source's state, masks and lists in ten
+// launches cost about 80 us of a 500 us source, most of it between them; two
+// launches take about 12): the state from the BFS levels (one path to
+// the source, no dependency), the level masks of both directions' items (one
+// wave per item), the list counts cleared.
+__global__ __launch_bounds__(kBlock) void k_bc_source(const int32_t* lv, VState* st, uint64_t V,
+                                                      uint32_t src, LevelItems in, LevelItems out,
+                                                      uint32_t* cnt) {
+  const uint64_t t0 = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const uint64_t nt = uint64_t(gridDim.x) * blockDim.x;
+  if (blockIdx.x == 0 && threadIdx.x < 128) cnt[threadIdx.x] = 0;
+  for (uint64_t v = t0; v < V; v += nt) {
+    VState x;
+    x.lv = lv[v];
+    x.sigma = v == src ? 1.0f : 0.0f;
+    x.delta = 0.0f;
+    x.pad = 0.0f;
+    st[v] = x;
+  }
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint64_t i = t0 >> 6; i < in.n + out.n; i += nt >> 6) {
+    const bool first = i < in.n;
+    const uint64_t j = first ? i : i - in.n;
+    const RowItem it = first ? in.items[j] : out.items[j];
     const uint32_t re = it.npieces == 0 ? it.row_end : it.row_begin + 1;
     uint32_t m = 0;
     for (uint32_t r = it.row_begin + lane; r < re; r += 64) {
@@ -360,39 +367,65 @@ __global__ void k_item_levels(const RowItem* items, uint64_t n, const int32_t* l
       if (l != kUnreachedLevel) m |= 1u << min(l, 31);
     }
     for (int o = 32; o > 0; o >>= 1) m |= __shfl_xor(m, o, 64);
-    if (lane == 0) mask[i] = m;
+    if (lane == 0) (first ? in.mask : out.mask)[j] = m;
   }
 }
 
-// Forward pass, rows split over several pieces: combine the partials in
-// piece order.
-__global__ void k_bc_fixup(BcArgs a, uint64_t nitems) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= nitems) return;
-  const RowItem it = a.items[i];
-  if (it.npieces > 1 && it.piece == 0 && a.st[it.row_begin].lv == a.d) {
-    float t = a.part[i];
-    for (uint32_t p = 1; p < it.npieces; p++) t = t + a.part[i + p];
-    finish<true>(a, it.row_begin, t);
-  }
-}
+// Level lists of both directions, one launch: the first `in_blocks` workgroups
+// list the in-direction's items, the others the out-direction's.  An item is
+// listed on every level it has a row on (levels >= 31 share list 31).
+// Positions come from one global atomic per workgroup, level and kind (the
+// waves take their slots in the workgroup's share from an LDS counter).
+constexpr unsigned kListBlock = 1024;  // workgroup of k_level_lists
 
-// A source's state: the BFS levels, one path to the source, no dependency.
-__global__ void k_bc_source_init(const int32_t* lv, VState* st, uint64_t V, uint32_t s) {
-  const uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (v < V) {
-    VState x;
-    x.lv = lv[v];
-    x.sigma = v == s ? 1.0f : 0.0f;
-    x.delta = 0.0f;
-    x.pad = 0.0f;
-    st[v] = x;
+__global__ __launch_bounds__(kListBlock) void k_level_lists(LevelItems in, LevelItems out,
+                                                            uint32_t in_blocks) {
+  constexpr uint32_t kWaves = kListBlock / 64;
+  __shared__ uint32_t bcount[2][32], bbase[2][32], woff[2][kWaves][32];
+  const bool first = blockIdx.x < in_blocks;
+  const LevelItems& d = first ? in : out;
+  const uint64_t i =
+      uint64_t(first ? blockIdx.x : blockIdx.x - in_blocks) * kListBlock + threadIdx.x;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t mk[2] = {0, 0}, wm[2];
+  if (i < d.n) {
+    const uint32_t m = d.mask[i];
+    const bool is_long = d.items[i].npieces != 0;
+    mk[0] = is_long ? m : 0;
+    mk[1] = is_long ? 0 : m;
   }
-}
-
-__global__ void k_fill_u64(unsigned long long* p, uint64_t n) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
+  if (threadIdx.x < 64) bcount[threadIdx.x >> 5][threadIdx.x & 31] = 0;
+  __syncthreads();
+  // the wave's slot in the workgroup's share of each level's list
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    wm[k] = mk[k];
+    for (int o = 32; o > 0; o >>= 1) wm[k] |= __shfl_xor(wm[k], o, 64);
+    for (uint32_t x = wm[k]; x; x &= x - 1) {
+      const uint32_t l = uint32_t(__builtin_ctz(x));
+      const uint64_t b = __ballot((mk[k] >> l) & 1u);
+      if (lane == uint32_t(__builtin_ctzll(b)))
+        woff[k][wave][l] = atomicAdd(&bcount[k][l], uint32_t(__popcll(b)));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const uint32_t k = threadIdx.x >> 5, l = threadIdx.x & 31;
+    if (bcount[k][l]) bbase[k][l] = atomicAdd(&(k ? d.nshort : d.nlong)[l], bcount[k][l]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    for (uint32_t x = wm[k]; x; x &= x - 1) {
+      const uint32_t l = uint32_t(__builtin_ctz(x));
+      const uint64_t b = __ballot((mk[k] >> l) & 1u);
+      if ((mk[k] >> l) & 1u) {
+        const uint64_t below = lane ? (b & (~0ull >> (64 - lane))) : 0ull;
+        const uint64_t p = bbase[k][l] + woff[k][wave][l] + uint32_t(__popcll(below));
+        d.list[uint64_t(l) * d.n + (k ? d.n - 1 - p : p)] = uint32_t(i);
+      }
+    }
+  }
 }
 
 __global__ void k_fill_f32(float* p, uint64_t n, float x) {
@@ -422,8 +455,8 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
     const BfsPrepared bfs = bfs_prepare(g, level);
     const Csr& out = *bfs.out;
     const Csr& in = *bfs.in;
-    const RowBlocks& in_rb = ensure_rowblocks(g, LL_GPU_DIR_IN, level, kCap, kPiece);
-    const RowBlocks& out_rb = ensure_rowblocks(g, LL_GPU_DIR_OUT, level, kCap, kPiece);
+    const RowBlocks& in_rb = ensure_rowblocks(g, LL_GPU_DIR_IN, level, kCap, kBcPiece);
+    const RowBlocks& out_rb = ensure_rowblocks(g, LL_GPU_DIR_OUT, level, kCap, kBcPiece);
     const uint64_t nin = std::max<uint64_t>(in_rb.n, 1), nout = std::max<uint64_t>(out_rb.n, 1);
     DevBuf lv, bfs_ws, st, bc, part, in_mask, out_mask, in_list, out_list, cnt, hub;
     lv.alloc(V * 4, s);
@@ -435,44 +468,34 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
     out_mask.alloc(nout * 4, s);
     in_list.alloc(32 * nin * 4, s);
     out_list.alloc(32 * nout * 4, s);
-    cnt.alloc(3 * 32 * 4, s);  // in, out, out long rows
-    const unsigned mask_grid = 4u * unsigned(ctx->num_cus);
+    cnt.alloc(4 * 32 * 4, s);  // in and out, each long rows' pieces and others
     k_fill_f32<<<grid_for(V, 256), 256, 0, s>>>(bc.as<float>(), V, 0.0f);
-    uint32_t* c_in = cnt.as<uint32_t>();
-    uint32_t* c_out = c_in + 32;
-    uint32_t* c_long = c_in + 64;
+    uint32_t* c = cnt.as<uint32_t>();
+    const LevelItems li{in_rb.items.as<RowItem>(), in_rb.n, in_mask.as<uint32_t>(),
+                        in_list.as<uint32_t>(), c, c + 32};
+    const LevelItems lo{out_rb.items.as<RowItem>(), out_rb.n, out_mask.as<uint32_t>(),
+                        out_list.as<uint32_t>(), c + 64, c + 96};
+    const unsigned source_grid = unsigned(std::min<uint64_t>(
+        grid_for((li.n + lo.n) * 64, kBlock), 8u * unsigned(ctx->num_cus)));
+    const unsigned in_blocks = unsigned(grid_for(li.n, kListBlock));
+    const unsigned out_blocks = unsigned(grid_for(lo.n, kListBlock));
     for (int64_t i = 0; i < ns; i++) {
       const uint32_t src = uint32_t(sources ? sources[i] : i);
       // the search's step count bounds the deepest level (a last step may
       // find nothing): a level without rows has an empty list
       const int32_t D = bfs_single_ws(g, bfs, src, bfs_ws.p, lv.as<int32_t>(), true).levels;
-      k_bc_source_init<<<grid_for(V, 256), 256, 0, s>>>(lv.as<int32_t>(), st.as<VState>(), V,
-                                                        src);
-      k_fill_u64<<<1, 64, 0, s>>>(reinterpret_cast<unsigned long long*>(c_in), 48);
-      k_item_levels<<<mask_grid, 256, 0, s>>>(in_rb.items.as<RowItem>(), in_rb.n,
-                                              lv.as<int32_t>(), in_mask.as<uint32_t>());
-      k_item_levels<<<mask_grid, 256, 0, s>>>(out_rb.items.as<RowItem>(), out_rb.n,
-                                              lv.as<int32_t>(), out_mask.as<uint32_t>());
-      for (bool long_rows : {true, false})
-        k_level_lists<<<grid_for(in_rb.n, kListBlock), kListBlock, 0, s>>>(
-            in_rb.items.as<RowItem>(), in_rb.n, in_mask.as<uint32_t>(), long_rows,
-            in_list.as<uint32_t>(), c_in);
-      k_level_lists<<<grid_for(out_rb.n, kListBlock), kListBlock, 0, s>>>(
-          out_rb.items.as<RowItem>(), out_rb.n, out_mask.as<uint32_t>(), true,
-          out_list.as<uint32_t>(), c_out);
-      k_copy_u32<<<1, 32, 0, s>>>(c_out, c_long, 32);
-      k_level_lists<<<grid_for(out_rb.n, kListBlock), kListBlock, 0, s>>>(
-          out_rb.items.as<RowItem>(), out_rb.n, out_mask.as<uint32_t>(), false,
-          out_list.as<uint32_t>(), c_out);
+      k_bc_source<<<source_grid, kBlock, 0, s>>>(lv.as<int32_t>(), st.as<VState>(), V, src, li,
+                                                 lo, c);
+      k_level_lists<<<in_blocks + out_blocks, kListBlock, 0, s>>>(li, lo, in_blocks);
       LLG_HIP(hipGetLastError());
-      LLG_HIP(hipMemcpyAsync(ctx->readback, c_in, 96 * 4, hipMemcpyDeviceToHost, s));
+      LLG_HIP(hipMemcpyAsync(ctx->readback, c, 4 * 32 * 4, hipMemcpyDeviceToHost, s));
       LLG_HIP(hipStreamSynchronize(s));
-      uint32_t h[96];
+      uint32_t h[4][32];
       std::memcpy(h, ctx->readback, sizeof(h));
       // long rows' terms by out-edge position, allocated when a source first
       // reaches one
       for (int l = 0; l < 32 && !hub.p; l++)
-        if (h[64 + l]) hub.alloc(out.E * 4, s);
+        if (h[2][l]) hub.alloc(out.E * 4, s);
       BcArgs a;
       a.st = st.as<VState>();
       a.bc = bc.as<float>();
@@ -484,13 +507,15 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
       a.adj = in.adj.as<uint32_t>();
       for (int32_t d = 1; d <= D; d++) {
         const uint32_t l = uint32_t(std::min(d, 31));
-        if (!h[l]) continue;
+        const LevelList lst{li.list + l * li.n, uint32_t(li.n), h[0][l]};
+        if (h[0][l] + h[1][l] == 0) continue;
         a.d = d;
         {
           TimedLaunch t(ctx, "k_bc_pass");
-          k_bc_pass<true><<<h[l], kBlock, 0, s>>>(a, in_list.as<uint32_t>() + l * nin);
+          k_bc_pass<true><<<h[0][l] + h[1][l], kBlock, 0, s>>>(a, lst);
         }
-        if (in_rb.nsplit) k_bc_fixup<<<grid_for(in_rb.n, 256), 256, 0, s>>>(a, in_rb.n);
+        if (h[0][l] && in_rb.nsplit)
+          k_bc_fixup<<<grid_for(h[0][l], kBlock / 64), kBlock, 0, s>>>(a, lst);
       }
       a.items = out_rb.items.as<RowItem>();
       a.ofs = out.ofs.as<uint64_t>();
@@ -498,15 +523,15 @@ int ll_gpu_bc(ll_gpu_graph* g, int level, const int64_t* sources, int64_t n, flo
       // level 0 is the source alone, whose dependency is never added
       for (int32_t d = D - 1; d >= 1; d--) {
         const uint32_t l = uint32_t(std::min(d, 31));
-        if (!h[32 + l]) continue;
+        const LevelList lst{lo.list + l * lo.n, uint32_t(lo.n), h[2][l]};
+        if (h[2][l] + h[3][l] == 0) continue;
         a.d = d;
-        const uint32_t* lst = out_list.as<uint32_t>() + l * nout;
-        if (h[64 + l]) {
+        if (h[2][l]) {
           TimedLaunch t(ctx, "k_bc_hub_terms");
-          k_bc_hub_terms<<<h[64 + l], kBlock, 0, s>>>(a, lst);
+          k_bc_hub_terms<<<h[2][l], kBlock, 0, s>>>(a, lst);
         }
         TimedLaunch t(ctx, "k_bc_pass");
-        k_bc_pass<false><<<h[32 + l], kBlock, 0, s>>>(a, lst);
+        k_bc_pass<false><<<h[2][l] + h[3][l], kBlock, 0, s>>>(a, lst);
       }
       LLG_HIP(hipGetLastError());
     }
