@@ -343,27 +343,52 @@ __global__ void k_fill_i32(int32_t* p, uint64_t n, int32_t x) {
 // The roots' lanes; the first frontier: the roots with out-edges, listed
 // once each, their count into stripe 0's word kListCount and their out-edges
 // into word 2.
+// One workgroup, a thread a lane: roots may repeat across lanes, so the first
+// lane of a root writes the words of all of its lanes (one thread walking the
+// lanes took 58 us for 64 roots, a chain of loads and stores a root).
+constexpr unsigned kRootBlock = 128;
+
 template <typename W>
-__global__ void k_ms_roots(W* vis, W* fr, const int64_t* roots, int n, int32_t* lv, uint64_t V,
-                           int src_base, const uint32_t* outdeg, uint32_t* lst,
-                           unsigned long long* flags) {
-  // one thread: roots may repeat across lanes
-  unsigned long long nl = 0, work = 0;
-  for (int s = 0; s < n; s++) {
-    const uint64_t r = uint64_t(roots[s]);
-    W bit = Lane<W>::low(s + 1) & ~Lane<W>::low(s);
-    vis[r] = vis[r] | bit;
-    if (lv) lv[uint64_t(src_base + s) * V + r] = 0;
-    const uint32_t od = outdeg[r];
-    if (od == 0) continue;
-    if (fr[r] == Lane<W>::zero()) {
-      lst[nl++] = uint32_t(r);
-      work += od;
-    }
-    fr[r] = fr[r] | bit;
+__global__ __launch_bounds__(kRootBlock) void k_ms_roots(W* vis, W* fr, const int64_t* roots, int n,
+                                                         int32_t* lv, uint64_t V, int src_base,
+                                                         const uint32_t* outdeg, uint32_t* lst,
+                                                         unsigned long long* flags) {
+  static_assert(Lane<W>::kBits <= int(kRootBlock), "a thread per lane");
+  __shared__ uint32_t root[kRootBlock];
+  __shared__ uint32_t listed;
+  __shared__ unsigned long long work;
+  const int s = int(threadIdx.x);
+  if (s == 0) {
+    listed = 0;
+    work = 0;
   }
-  flags[kListCount] = nl;
-  flags[2] = work;
+  if (s < n) root[s] = uint32_t(roots[s]);
+  __syncthreads();
+  if (s < n) {
+    const uint32_t r = root[s];
+    if (lv) lv[uint64_t(src_base + s) * V + r] = 0;
+    bool first = true;
+    W lanes = Lane<W>::zero();
+    for (int t = 0; t < n; t++) {
+      if (root[t] != r) continue;
+      first = first && t >= s;
+      lanes = lanes | (Lane<W>::low(t + 1) & ~Lane<W>::low(t));
+    }
+    if (first) {
+      vis[r] = vis[r] | lanes;
+      const uint32_t od = outdeg[r];
+      if (od) {
+        fr[r] = lanes;
+        lst[atomicAdd(&listed, 1u)] = r;
+        atomicAdd(&work, (unsigned long long)od);
+      }
+    }
+  }
+  __syncthreads();
+  if (s == 0) {
+    flags[kListCount] = listed;
+    flags[2] = work;
+  }
 }
 
 __global__ void k_zero_ull(unsigned long long* p) { *p = 0; }
@@ -760,7 +785,7 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
   k_ms_init<W><<<grid_for(V, 256), 256, 0, s>>>(vis.as<W>(), fr.as<W>(), nx.as<W>(), V,
                                                 full & ~used);
   k_zero_flags<<<1, kFlagStripes, 0, s>>>(found.as<unsigned long long>());
-  k_ms_roots<W><<<1, 1, 0, s>>>(vis.as<W>(), fr.as<W>(), d_roots + src_base, n, d_lv, V, src_base,
+  k_ms_roots<W><<<1, kRootBlock, 0, s>>>(vis.as<W>(), fr.as<W>(), d_roots + src_base, n, d_lv, V, src_base,
                                 outdeg, lst[0].as<uint32_t>(), found.as<unsigned long long>());
   LLG_HIP(hipGetLastError());
   static_assert(kFlagStripes * kFlagStride * 8 <= kReadbackBytes, "flags fit the read-back buffer");
