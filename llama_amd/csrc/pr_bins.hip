@@ -17,10 +17,11 @@
 //      rank/outdeg (FP32), kept in LDS;
 //   C. as the same vertices are the sources of chunks (b', b) for every b',
 //      writes the next iteration's values into those chunks (each slot names
-//      its source's offset in the bin, u16): a wave takes the chunks kGroupC
-//      at a time, their first 128 slots loaded together, so its writes are
-//      contiguous runs and several loads are in flight.  Neighbouring bins
-//      run on one XCD, whose L2 merges the partial lines at chunk ends.
+//      its source's offset in the bin, u16): the chunks are dealt to the
+//      waves by slots, a wave keeps kGroupC pieces of 64 slots in flight
+//      whatever the chunks' lengths, and its writes are contiguous runs.
+//      Neighbouring bins run on one XCD, whose L2 merges the partial lines
+//      at chunk ends.
 // Integer addition is associative, so a row sum does not depend on the order
 // its slots are added in: every run gives the same bits, whatever the
 // schedule or bin size.  Each term is the FP32 contribution truncated to a

@@ -412,11 +412,6 @@ size_t scan_tmp_bytes(uint64_t n) {
   return w * 8;
 }
 
-void scan_u32_to_u64_ws(const uint32_t* in, uint64_t* out, uint64_t n, void* tmp,
-                        hipStream_t s) {
-  scan_rec(SrcU32{in}, n, out, static_cast<uint64_t*>(tmp), s);
-}
-
 void scan_gather_u32_to_u64_ws(const uint32_t* idx, const uint32_t* val, uint64_t* out,
                                uint64_t n, void* tmp, hipStream_t s) {
   scan_rec(SrcGatherU32{idx, val}, n, out, static_cast<uint64_t*>(tmp), s);
@@ -428,11 +423,6 @@ void scan_u32_to_u64(const uint32_t* in, uint64_t* out, uint64_t n, hipStream_t 
 
 void scan_u64(const uint64_t* in, uint64_t* out, uint64_t n, hipStream_t s) {
   scan_alloc(SrcU64{in}, n, out, s);
-}
-
-void sort_pairs_u64_u32(const uint64_t* keys_in, uint64_t* keys_out, const uint32_t* vals_in,
-                        uint32_t* vals_out, uint64_t n, int end_bit, hipStream_t s) {
-  radix_sort<uint64_t, true>(keys_in, keys_out, vals_in, vals_out, n, end_bit, s);
 }
 
 void sort_pairs_u32_u32(const uint32_t* keys_in, uint32_t* keys_out, const uint32_t* vals_in,
