@@ -108,6 +108,106 @@ __device__ inline void accumulate_rows(const PprArgs& a, uint64_t lo, uint64_t h
   }
 }
 
+__device__ inline uint32_t lane_u32(uint32_t x, uint32_t lane) {
+  return uint32_t(__builtin_amdgcn_readlane(int(x), int(lane)));
+}
+__device__ inline float lane_f32(float x, uint32_t lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), int(lane)));
+}
+
+// A wave's walk over n <= 2^32 entries first, first + stride, ... of the
+// in-edges, for rows as wide as the wave: 64 source IDs and their 1/outdeg are
+// loaded a lane each (the next 64 before this chunk's rows), then the rows of
+// kRowsAhead sources are requested together, their addresses wave-uniform.
+// at(i, x) takes entry i's values already scaled, in order.
+//
+// Bound by the row gathers (Infinity Cache on graphs past the L2s).  With a
+// row at a time, four sources ahead and every lane loading the same source ID
+// and 1/outdeg, an iteration of 64 columns over 200003 vertices and 3.2 M
+// edges took 217 us (3.8 TB/s of rows); with the ID loads shared by the wave
+// and the gathers running across row ends 165 us.  Widths under 64 keep the
+// form above: their rows are narrower than a wave, whose lane groups work on
+// different rows.
+constexpr uint32_t kRowsAhead = 8;
+
+template <int B, typename F>
+__device__ inline void walk_entries(const PprArgs& a, uint64_t first, uint32_t n, uint32_t stride,
+                                    uint32_t lane, F at) {
+  constexpr int EPL = Geo<B>::EPL;
+  uint32_t w_next = lane < n ? a.adj[first + uint64_t(lane) * stride] : 0u;
+  for (uint32_t c = 0; c < n; c += 64) {
+    const uint32_t m = min(64u, n - c);
+    const uint32_t w = w_next;
+    const float f = a.invdeg[w];
+    const uint64_t nx = uint64_t(c) + 64 + lane;
+    w_next = nx < n ? a.adj[first + nx * stride] : 0u;
+    for (uint32_t j = 0; j < m; j += kRowsAhead) {
+      // past the chunk's end: vertex 0 or a repeated lane, loaded and not used
+      float x[kRowsAhead][EPL];
+#pragma unroll
+      for (uint32_t u = 0; u < kRowsAhead; u++) {
+        const float* row = a.rin + uint64_t(lane_u32(w, (j + u) & 63)) * B;
+#pragma unroll
+        for (int k = 0; k < EPL; k++) x[u][k] = row[lane * EPL + k];
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kRowsAhead; u++) {
+        if (j + u < m) {
+          const float fu = lane_f32(f, j + u);
+#pragma unroll
+          for (int k = 0; k < EPL; k++) x[u][k] *= fu;
+          at(c + j + u, x[u]);
+        }
+      }
+    }
+  }
+}
+
+// Rows [r0, r1) of a stream item by one wave, 64 row ends held in the lanes at
+// a time.  The rows' entries are one run, so the walk's loads do not stop at a
+// row's end; a row's old rank is requested when the row before it ends.
+template <int B>
+__device__ inline void wave_rows(const PprArgs& a, uint32_t r0, uint32_t r1, uint32_t lane,
+                                 const uint32_t* seed, float* dsum) {
+  constexpr int EPL = Geo<B>::EPL;
+  for (uint32_t rb = r0; rb < r1; rb += 64) {
+    const uint32_t nr = min(64u, r1 - rb);
+    const uint64_t base = a.ofs[rb];
+    const uint32_t end = uint32_t(a.ofs[rb + min(lane, nr - 1) + 1] - base);
+    uint32_t row = 0, row_end = lane_u32(end, 0);
+    float old[EPL];
+    Neu acc[EPL];
+    auto open_row = [&]() {
+#pragma unroll
+      for (int k = 0; k < EPL; k++) {
+        old[k] = a.rin[uint64_t(rb + row) * B + lane * EPL + k];
+        acc[k] = Neu::zero();
+      }
+    };
+    auto close_row = [&]() {
+#pragma unroll
+      for (int k = 0; k < EPL; k++) {
+        float v = a.d * acc[k].value();
+        if (seed[k] == rb + row) v += a.one_minus_d;
+        dsum[k] += fabsf(v - old[k]);
+        a.rout[uint64_t(rb + row) * B + lane * EPL + k] = v;
+      }
+      row++;
+      if (row < nr) {
+        row_end = lane_u32(end, row);
+        open_row();
+      }
+    };
+    open_row();
+    walk_entries<B>(a, base, lane_u32(end, nr - 1), 1, lane, [&](uint32_t i, const float* x) {
+      while (i >= row_end) close_row();
+#pragma unroll
+      for (int k = 0; k < EPL; k++) acc[k].add(x[k]);
+    });
+    while (row < nr) close_row();
+  }
+}
+
 template <int B>
 __global__ __launch_bounds__(kBlock) void k_ppr_iter(PprArgs a) {
   if (a.st->converged) return;
@@ -119,11 +219,33 @@ __global__ __launch_bounds__(kBlock) void k_ppr_iter(PprArgs a) {
   const int li = lane % LPR, sr = lane / LPR;
   const int slot = wave * RPW + sr;
   float dsum[EPL];
+  uint32_t seed[EPL];
 #pragma unroll
-  for (int k = 0; k < EPL; k++) dsum[k] = 0.f;
+  for (int k = 0; k < EPL; k++) {
+    dsum[k] = 0.f;
+    seed[k] = a.seeds[li * EPL + k];
+  }
   for (uint64_t i = blockIdx.x; i < a.nitems; i += gridDim.x) {
     const RowItem it = a.items[i];
-    if (it.npieces == 0) {
+    if (it.npieces == 0 && LPR == 64) {
+      // the rows cut into one run per wave by their entries: the rows that
+      // start before the run's first entry, counted over the item's offsets
+      const uint32_t nr = it.row_end - it.row_begin;
+      const uint64_t e0 = a.ofs[it.row_begin];
+      const uint32_t ne = uint32_t(a.ofs[it.row_end] - e0);
+      uint32_t lo = 0, hi = 0;
+      for (uint32_t q = 0; q < nr; q += 64) {
+        const uint32_t t = q + lane;
+        const uint32_t st =
+            t < nr ? uint32_t(a.ofs[it.row_begin + t] - e0) * SLOTS : 0xffffffffu;
+        lo += uint32_t(__popcll(__ballot(st < ne * uint32_t(wave))));
+        hi += uint32_t(__popcll(__ballot(st < ne * uint32_t(wave + 1))));
+      }
+      if (wave + 1 == SLOTS) hi = nr;
+      const uint32_t r0 = uint32_t(__builtin_amdgcn_readfirstlane(int(it.row_begin + lo)));
+      const uint32_t r1 = uint32_t(__builtin_amdgcn_readfirstlane(int(it.row_begin + hi)));
+      wave_rows<B>(a, r0, r1, uint32_t(lane), seed, dsum);
+    } else if (it.npieces == 0) {
       for (uint32_t t = it.row_begin + slot; t < it.row_end; t += SLOTS) {
         Neu acc[EPL];
 #pragma unroll
@@ -138,7 +260,17 @@ __global__ __launch_bounds__(kBlock) void k_ppr_iter(PprArgs a) {
       Neu acc[EPL];
 #pragma unroll
       for (int k = 0; k < EPL; k++) acc[k] = Neu::zero();
-      accumulate_rows<B>(a, lo + slot, hi, SLOTS, li, acc);
+      if (LPR == 64) {
+        const uint32_t uw = uint32_t(__builtin_amdgcn_readfirstlane(wave));
+        const uint32_t n = uint32_t(hi - lo);
+        walk_entries<B>(a, lo + uw, n > uw ? (n - uw + SLOTS - 1) / SLOTS : 0u, SLOTS,
+                        uint32_t(lane), [&](uint32_t, const float* x) {
+#pragma unroll
+                          for (int k = 0; k < EPL; k++) acc[k].add(x[k]);
+                        });
+      } else {
+        accumulate_rows<B>(a, lo + slot, hi, SLOTS, li, acc);
+      }
 #pragma unroll
       for (int k = 0; k < EPL; k++) {
         ls[slot][li * EPL + k] = acc[k].s;
