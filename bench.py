@@ -674,11 +674,11 @@ def bench_large(args) -> int:
     info = dg.snapshot_info()
     E, V = int(info.live_edges), g.num_nodes
     ctx.sync()
-    # PageRank: bins of 2^13 (the automatic choice) and 2^14 destinations; a
+    # PageRank: bins of 2^14 (the automatic choice here) and 2^13 destinations; a
     # first call materialises the snapshot and builds the layout, the second
     # is timed with the layout in place
     by_bins = {}
-    for bb in (-1, 14):
+    for bb in (-1, 13):
         ctx.set_option("pr_bin_bits", bb)
         dg.drop_snapshots()
         ctx.sync()
