@@ -523,7 +523,7 @@ def measured_traffic(args, V: int, E: int, used: list) -> dict | None:
     counter reads for a 1 GiB device copy in the same run), when this run is
     the workload and PageRank variant they were measured on; else None."""
     if used == ["k_pb_iter"]:
-        kernel, variant = "k_pb_iter", args.bin_bits in (-1, 13)
+        kernel, variant = "k_pb_iter", args.bin_bits in (-1, 14)
     elif used == ["k_pr_pull", "k_pr_fixup"]:
         kernel = "k_pr_pull"
         variant = (args.reorder == 1 and args.seg_bits in (-1, 0) and args.hot_bits in (-1, 0)
