@@ -51,3 +51,26 @@ def test_counts(ctx, V, per, skew):
     assert dg.triangles() == n  # again, over the DAG already built
     assert dg.tc_i() >= n
     assert dg.triangles() == n
+
+
+@pytest.mark.parametrize("outside", [0.60, 0.68, 0.74])
+def test_hubs_beside_many_small_vertices(ctx, outside):
+    """A core of hubs 16 times the mean degree or more with most edge ends
+    outside it: on either side of, and between, the two limits of the share."""
+    V, E, hubs = 2_200_000, 600_000, 32_768
+    gpu_case(f"tc core hubs, {outside} of the ends outside")
+    rng = np.random.default_rng(int(outside * 100))
+    n = int(E * outside)
+    top = rng.choice(V, hubs, replace=False)
+    m = (E - n) // 2
+    a, b = top[rng.integers(0, hubs, m)], top[(hubs * rng.random(m) ** 2).astype(np.int64)]
+    s = rng.integers(0, V, n // 2)
+    d = rng.integers(0, V, n // 2)
+    src = np.concatenate([a, a, s, s])
+    dst = np.concatenate([b, top[rng.integers(0, 300, m)], d, (s + 1) % V])
+    g = HostGraph(V)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    n, arcs, work = dg.triangles(stats=True)
+    assert n == oracle.OracleGraph.from_host(g).triangles()
+    assert (arcs, work) == dag_stats(V, src, dst)
