@@ -263,6 +263,17 @@ __global__ void k_edge_tails(const uint64_t* ofs, uint64_t V, uint32_t* tail) {
     for (uint64_t e = ofs[u] + lane, end = ofs[u + 1]; e < end; e += 64) tail[e] = uint32_t(u);
 }
 
+// In-degrees counted over the out-edges' heads.
+__global__ void k_count_heads(const uint32_t* adj, uint64_t n, uint32_t* deg) {
+  const uint64_t e = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e < n) atomicAdd(&deg[adj[e]], 1u);
+}
+
+__global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
+  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = v;
+}
+
 // Edge e's row (its number in `slot` when given) as the sort key, e as the value.
 __global__ void k_row_keys(const uint32_t* row, const uint32_t* slot, uint32_t* key,
                            uint32_t* pos, uint64_t n) {
@@ -384,8 +395,22 @@ const WprMatrix& ensure_wpr_matrix(ll_gpu_graph* g, int level, bool forward) {
     m.level = level;
     return m;
   }
-  if (renumber)
-    degree_slots(ctx, ensure_degrees(g, forward ? LL_GPU_DIR_OUT : LL_GPU_DIR_IN, level), V, m.slot);
+  if (renumber) {
+    DevBuf counted;
+    const uint32_t* deg;
+    if (!forward && g->slcsr && !g->sl[LL_GPU_DIR_IN].valid) {
+      // a single-level CSR may hold the out-edges alone
+      counted.alloc(V * 4, s);
+      k_fill_u32<<<grid_for(V, 256), 256, 0, s>>>(counted.as<uint32_t>(), V, 0u);
+      k_count_heads<<<grid_for(E, 256), 256, 0, s>>>(out.adj.as<uint32_t>(), E,
+                                                     counted.as<uint32_t>());
+      LLG_HIP(hipGetLastError());
+      deg = counted.as<uint32_t>();
+    } else {
+      deg = ensure_degrees(g, forward ? LL_GPU_DIR_OUT : LL_GPU_DIR_IN, level);
+    }
+    degree_slots(ctx, deg, V, m.slot);
+  }
   const uint32_t* slot = m.slot.as<uint32_t>();
   const uint64_t n = std::max<uint64_t>(E, 1);
   DevBuf tail, key, pos, rows;

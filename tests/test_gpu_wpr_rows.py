@@ -56,3 +56,24 @@ def test_rows_of_every_length(ctx, V):
     assert np.all(np.abs(wt.grad.cpu().numpy() - ref) <= 2 * TOL * ref + 1e-30)
     again = weighted_pagerank(wt, pt, dg, K, D)
     assert torch.equal(again, r)  # the sums do not depend on the schedule
+
+
+@pytest.mark.parametrize("V", [24576, 24577, 60001])
+def test_out_edges_alone(ctx, V):
+    """A single-level CSR without its in-edges gives the same forward and
+    adjoint, bit for bit."""
+    gpu_case(f"wpr out-edges alone V={V}")
+    rng = np.random.default_rng(V)
+    src = rng.integers(0, V, 6 * V)
+    dst = (V * rng.random(6 * V) ** 3).astype(np.int64)
+    w = (rng.random(src.size) / 8).astype(np.float32)
+    p = (rng.random(V) / V).astype(np.float32)
+    got = []
+    for in_csr in (csr_of(V, dst, src), None):
+        dg = SlcsrGraph(ctx, V, csr_of(V, src, dst), in_csr)
+        wt = torch.tensor(w, device="cuda", requires_grad=True)
+        pt = torch.tensor(p, device="cuda", requires_grad=True)
+        r = weighted_pagerank(wt, pt, dg, K, D)
+        r.backward(torch.ones(V, device="cuda"))
+        got.append((r.detach(), wt.grad, pt.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
