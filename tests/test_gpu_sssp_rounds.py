@@ -122,3 +122,25 @@ def test_fixed_point_on_a_skewed_graph(ctx, min_queue):
             assert n == int((d < UNREACHED).sum())
     finally:
         ctx.set_option("sssp_min_queue", -1)
+
+
+@pytest.mark.parametrize("V,E", [(64, 400_000), (2000, 3_000_000)])
+def test_few_vertices_many_edges(ctx, V, E):
+    """The edges of few vertices are spread over the chip: a round moves at most
+    12 bytes an edge (1 to 8 us at the rate of a large copy) and a launch takes
+    about 10 us, so 100 us a launch is several times what it needs."""
+    rng = np.random.default_rng(V)
+    src, dst = rng.integers(0, V, E), rng.integers(0, V, E)
+    w = rng.random(E).astype(np.float32)
+    g = HostGraph(V)
+    g.add_level(src, dst, weights=w)
+    dg = DeviceGraph(ctx, g)
+    gpu_case(f"sssp few vertices V={V} E={E}")
+    assert np.array_equal(dg.sssp(0)[0], bellman_ford(V, src, dst, w, 0))
+    ctx.profile(True)
+    try:
+        dg.sssp(0)
+        n, ms = ctx.kernel_time("k_relax")
+    finally:
+        ctx.profile(False)
+    assert n > 0 and ms / n < 0.1
