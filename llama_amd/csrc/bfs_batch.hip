@@ -695,7 +695,7 @@ template <uint32_t BB, typename W>
 void launch_binned(const PrBins& pb, const W* fr, W* sv, const MsArgs<W>& a,
                    const uint32_t* indeg, hipStream_t s) {
   if constexpr (bins_fit<W>(BB)) {
-      k_msb_scatter<BB, W><<<pb.nbins, kBinBlock, 0, s>>>(fr, a.V, pb.nbins, pb.ct.as<uint2>(),
+    k_msb_scatter<BB, W><<<pb.nbins, kBinBlock, 0, s>>>(fr, a.V, pb.nbins, pb.ct.as<uint2>(),
                                                         pb.sidx.as<uint16_t>(), sv);
     k_msb_gather<BB, W><<<pb.nbins, kBinBlock, 0, s>>>(a, sv, pb.ldst.as<uint16_t>(),
                                                        pb.bstart.as<uint64_t>(), indeg);
@@ -755,6 +755,25 @@ __global__ __launch_bounds__(kReachBlock) void k_ms_reached(const W* vis, uint64
 }
 
 }  // namespace
+
+long option_or(const ll_gpu_ctx* ctx, const char* name, long fallback) {
+  const auto it = ctx->options.find(name);
+  return it == ctx->options.end() ? fallback : it->second;
+}
+
+// The binned layout the sweeps of this lane width take, built on first use;
+// nullptr when they have none.
+template <typename W>
+const PrBins* batch_bins(ll_gpu_graph* g, int level) {
+  const long bins_opt = option_or(g->ctx, "bfs_batch_bins", -1);
+  if (bins_opt == 0) return nullptr;
+  const long bb = option_or(g->ctx, "pr_bin_bits", -1);
+  uint32_t max_bb = kMaxBinBits;  // the largest bins this lane width can gather
+  while (!bins_fit<W>(max_bb)) max_bb--;
+  const PrBins* p = ensure_lane_bins(g, level, bb, max_bb);
+  if (!p && bins_opt == 1 && pr_bin_bits(g, level, bb) == 0) p = ensure_pr_bins(g, level, 12);
+  return p && bins_fit<W>(p->bb) ? p : nullptr;
+}
 
 template <typename W>
 void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int src_base,
@@ -817,23 +836,11 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
   // kBinOpen of the in-edges (a pull skips the other rows; the binned sweep
   // streams every edge at about half a full pull's cost), else a pull.
   constexpr uint64_t kPushRatio = 16;
-  const long bins_opt = ctx->options.count("bfs_batch_bins") ? ctx->options["bfs_batch_bins"] : -1;
-  const long open_opt =
-      ctx->options.count("bfs_batch_bin_open") ? ctx->options["bfs_batch_bin_open"] : -1;
+  const long bins_opt = option_or(ctx, "bfs_batch_bins", -1);
+  const long open_opt = option_or(ctx, "bfs_batch_bin_open", -1);
   const double kBinOpen = open_opt >= 0 ? double(open_opt) / 100.0 : 0.4;
-  const PrBins* pb = nullptr;
-  const uint32_t* indeg = nullptr;
-  if (bins_opt != 0) {
-    const long bb = ctx->options.count("pr_bin_bits") ? ctx->options["pr_bin_bits"] : -1;
-    uint32_t max_bb = kMaxBinBits;  // the largest bins this lane width can gather
-    while (!bins_fit<W>(max_bb)) max_bb--;
-    PrBins* p = ensure_lane_bins(g, level, bb, max_bb);
-    if (!p && bins_opt == 1 && bb == 0) p = ensure_pr_bins(g, level, 12);
-    if (p && bins_fit<W>(p->bb)) {
-      pb = p;
-      indeg = ensure_degrees(g, LL_GPU_DIR_IN, level);
-    }
-  }
+  const PrBins* pb = batch_bins<W>(g, level);
+  const uint32_t* indeg = pb ? ensure_degrees(g, LL_GPU_DIR_IN, level) : nullptr;
   uint64_t open_in = in.E;  // in-edges of the rows a searching lane has not reached
   DevBuf sv;                // binned sweeps: the slots' lane words
   const Csr* out = nullptr;

@@ -448,6 +448,8 @@ void build_pr_bins(ll_gpu_graph* g, const Csr& out, uint32_t bb, PrBins& pb);
 // (12..14), built on first use; -1 = automatic (8..14 by the snapshot's size
 // while E < 2^32 and the bins of 2^14 number at most 16384; otherwise none);
 // nullptr when there are none (0 or the automatic rule's "none").
+// pr_bin_bits answers the size alone (0 = none) and builds nothing.
+uint32_t pr_bin_bits(ll_gpu_graph* g, int level, long bin_bits);
 PrBins* ensure_pr_bins(ll_gpu_graph* g, int level, long bin_bits);
 // The same for a sweep whose LDS holds bins of at most 2^max_bb vertices: the
 // PageRank layout where it fits, else (automatic bins only) one of its own

@@ -428,37 +428,39 @@ uint32_t auto_bin_bits(uint64_t V, uint64_t E) {
   return bb;
 }
 
-}  // namespace
-
-PrBins* ensure_pr_bins(ll_gpu_graph* g, int level, long bin_bits) {
-  const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
-  const uint64_t V = g->V;
-  if (bin_bits < 0) {
-    bin_bits = auto_bin_bits(V, out.E);
-    if (bin_bits == 0) return nullptr;
-  } else {
-    if (bin_bits == 0) return nullptr;
-    LLG_CHECK(bin_bits >= 12 && bin_bits <= 14, LL_GPU_EINVAL, "bin bits must be 0 or 12..14");
-  }
-  PrBins& pb = g->pr_bins;
-  if (!(pb.valid && pb.level == out.level && pb.bb == uint32_t(bin_bits)))
-    build_pr_bins(g, out, uint32_t(bin_bits), pb);
+// The layout of the out-CSR in bins of 2^bb vertices, in `pb`.
+PrBins* bins_in(ll_gpu_graph* g, const Csr& out, uint32_t bb, PrBins& pb) {
+  if (!(pb.valid && pb.level == out.level && pb.bb == bb)) build_pr_bins(g, out, bb, pb);
   return &pb;
 }
 
+}  // namespace
+
+uint32_t pr_bin_bits(ll_gpu_graph* g, int level, long bin_bits) {
+  if (bin_bits < 0) return auto_bin_bits(g->V, ensure_csr(g, LL_GPU_DIR_OUT, level).E);
+  LLG_CHECK(bin_bits == 0 || (bin_bits >= 12 && bin_bits <= 14), LL_GPU_EINVAL,
+            "bin bits must be 0 or 12..14");
+  return uint32_t(bin_bits);
+}
+
+PrBins* ensure_pr_bins(ll_gpu_graph* g, int level, long bin_bits) {
+  const uint32_t bb = pr_bin_bits(g, level, bin_bits);
+  if (bb == 0) return nullptr;
+  return bins_in(g, ensure_csr(g, LL_GPU_DIR_OUT, level), bb, g->pr_bins);
+}
+
 PrBins* ensure_lane_bins(ll_gpu_graph* g, int level, long bin_bits, uint32_t max_bb) {
-  PrBins* p = ensure_pr_bins(g, level, bin_bits);
-  if (!p || p->bb <= max_bb) return p;
+  const uint32_t bb = pr_bin_bits(g, level, bin_bits);
+  if (bb == 0) return nullptr;
+  const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
+  if (bb <= max_bb) return bins_in(g, out, bb, g->pr_bins);
   // the PageRank bins are too large for this lane width: a layout of their
   // own for the sweeps, while its chunks hold 32 slots on average (at 8.6 the
-  // binned sweep loses to the pull)
+  // binned sweep loses to the pull); the PageRank layout is not needed for it
   if (bin_bits >= 0) return nullptr;
-  const Csr& out = ensure_csr(g, LL_GPU_DIR_OUT, level);
   const uint64_t nb = bins_of(g->V, max_bb);
   if (nb > 16384 || out.E < 32 * nb * nb) return nullptr;
-  PrBins& pb = g->lane_bins;
-  if (!(pb.valid && pb.level == out.level && pb.bb == max_bb)) build_pr_bins(g, out, max_bb, pb);
-  return &pb;
+  return bins_in(g, out, max_bb, g->lane_bins);
 }
 
 void pagerank_bins(ll_gpu_graph* g, const Csr& out, const uint32_t* outdeg, PrBins& pb,

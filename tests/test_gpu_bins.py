@@ -56,3 +56,35 @@ def test_every_bin_size(ctx, V, per):
                 assert np.array_equal(lv[j], one) and reached[j] == n
     finally:
         ctx.set_option("bfs_batch_bins", -1)
+
+
+# one bin of any size holds every slot: from 40 edges on PageRank takes 2^8,
+# below 2^14, whose 128-lane words do not fit a workgroup's LDS; those sweeps
+# take 2^13 down to 32 edges, and none below
+@pytest.mark.parametrize("E,lane_layout", [(31, False), (32, True), (39, True), (40, True)])
+def test_wide_lanes_build_their_own_layout_alone(ctx, E, lane_layout):
+    """A 128-lane sweep builds the one layout it reads, whatever PageRank's
+    would be, and takes its levels from it."""
+    V = 100
+    rng = np.random.default_rng(E)
+    pairs = rng.choice(V * (V - 1), E, replace=False)
+    src, dst = pairs // (V - 1), pairs % (V - 1)
+    dst = dst + (dst >= src)
+    g = HostGraph(V)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    roots = np.concatenate([src, rng.integers(0, V, 128 - E)])
+    gpu_case(f"lane layout E={E}")
+    ctx.set_option("bfs_batch_bins", 1)
+    ctx.profile(True)
+    try:
+        lv, reached, _ = dg.bfs_batch(roots, lane_width=128)
+        builds, _ = ctx.kernel_time("pr_bins_build")
+        sweeps, _ = ctx.kernel_time("k_msb_sweep")
+    finally:
+        ctx.profile(False)
+        ctx.set_option("bfs_batch_bins", -1)
+    assert (builds, sweeps > 0) == ((1, True) if lane_layout else (0, False))
+    for j, root in enumerate(roots):
+        one, n, _ = dg.bfs(int(root))
+        assert np.array_equal(lv[j], one) and reached[j] == n
