@@ -775,29 +775,61 @@ const PrBins* batch_bins(ll_gpu_graph* g, int level) {
   return p && bins_fit<W>(p->bb) ? p : nullptr;
 }
 
+// Push sweeps run while the frontier's out-edges are under 1/kPushRatio of the
+// edges.
+constexpr uint64_t kPushRatio = 16;
+
+// Device memory of a batch, which the batches of one call share: allocated by
+// the first, each batch clears what it reads.
+struct MsWork {
+  DevBuf vis, fr, nx, part, found;
+  // vertex lists of the frontiers (two, alternating), the vertices a push
+  // reaches and its touched bits (all clear between sweeps)
+  DevBuf lst[2], tl, touched;
+  DevBuf qdeg, qofs, qn, blk;  // push sweeps
+  DevBuf sv;                   // binned sweeps: the slots' lane words
+
+  template <typename W>
+  void alloc(uint64_t V, const RowBlocks& rb, hipStream_t s) {
+    if (vis.p) return;
+    vis.alloc(V * sizeof(W), s);
+    fr.alloc(V * sizeof(W) + 16, s);  // padded: 16-bit lanes are OR-ed through 32-bit words
+    nx.alloc(V * sizeof(W) + 16, s);
+    part.alloc(std::max<uint64_t>(rb.n, 1) * sizeof(W), s);
+    found.alloc(kFlagStripes * kFlagStride * 8, s);
+    lst[0].alloc(V * 4, s);
+    lst[1].alloc(V * 4, s);
+    tl.alloc(V * 4, s);
+    touched.alloc((V + 31) / 32 * 4, s);
+  }
+  // a push sweep's frontier holds under E / kPushRatio out-edges
+  void alloc_push(uint64_t V, uint64_t E, hipStream_t s) {
+    if (qdeg.p) return;
+    qdeg.alloc(V * 4, s);
+    qofs.alloc((V + 1) * 8, s);
+    qn.alloc(8, s);
+    blk.alloc((E / kPushRatio / kPushEdges + 1) * 16, s);
+  }
+  template <typename W>
+  void alloc_slots(uint64_t E, hipStream_t s) {
+    if (!sv.p) sv.alloc(std::max<uint64_t>(E, 1) * sizeof(W), s);
+  }
+};
+
 template <typename W>
 void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int src_base,
-                 int32_t* d_lv, unsigned long long* d_reached, uint64_t* levels_run) {
+                 int32_t* d_lv, unsigned long long* d_reached, uint64_t* levels_run, MsWork& mem) {
   ll_gpu_ctx* ctx = g->ctx;
   hipStream_t s = ctx->stream;
   const uint64_t V = g->V;
   const Csr& in = ensure_csr(g, LL_GPU_DIR_IN, level);
   const RowBlocks& rb = ensure_rowblocks(g, LL_GPU_DIR_IN, level, kCap, kPiece);
   const uint32_t* outdeg = ensure_degrees(g, LL_GPU_DIR_OUT, level);
-  DevBuf vis, fr, nx, part, found;
-  vis.alloc(V * sizeof(W), s);
-  fr.alloc(V * sizeof(W) + 16, s);  // padded: 16-bit lanes are OR-ed through 32-bit words
-  nx.alloc(V * sizeof(W) + 16, s);
-  part.alloc(std::max<uint64_t>(rb.n, 1) * sizeof(W), s);
-  found.alloc(kFlagStripes * kFlagStride * 8, s);
-  // vertex lists of the frontiers (two, alternating), the vertices a push
-  // reaches and its touched bits (all clear between sweeps)
-  DevBuf lst[2], tl, touched;
-  lst[0].alloc(V * 4, s);
-  lst[1].alloc(V * 4, s);
-  tl.alloc(V * 4, s);
+  mem.alloc<W>(V, rb, s);
+  DevBuf &vis = mem.vis, &fr = mem.fr, &nx = mem.nx, &part = mem.part, &found = mem.found;
+  DevBuf &tl = mem.tl, &touched = mem.touched;
+  DevBuf(&lst)[2] = mem.lst;
   const uint64_t tw = (V + 31) / 32;
-  touched.alloc(tw * 4, s);
   k_fill_i32<<<grid_for(tw, 256), 256, 0, s>>>(touched.as<int32_t>(), tw, 0);
   const W full = Lane<W>::low(Lane<W>::kBits);
   const W used = Lane<W>::low(n);
@@ -835,16 +867,13 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
   // while the rows some searching lane has not reached hold at least
   // kBinOpen of the in-edges (a pull skips the other rows; the binned sweep
   // streams every edge at about half a full pull's cost), else a pull.
-  constexpr uint64_t kPushRatio = 16;
   const long bins_opt = option_or(ctx, "bfs_batch_bins", -1);
   const long open_opt = option_or(ctx, "bfs_batch_bin_open", -1);
   const double kBinOpen = open_opt >= 0 ? double(open_opt) / 100.0 : 0.4;
   const PrBins* pb = batch_bins<W>(g, level);
   const uint32_t* indeg = pb ? ensure_degrees(g, LL_GPU_DIR_IN, level) : nullptr;
   uint64_t open_in = in.E;  // in-edges of the rows a searching lane has not reached
-  DevBuf sv;                // binned sweeps: the slots' lane words
   const Csr* out = nullptr;
-  DevBuf qdeg, qofs, qn, blk;
   uint64_t lv_count = 0;
   W done = full & ~used;  // lanes not searching (unused); later also finished ones
   for (int32_t l = 1;; l++) {
@@ -873,9 +902,7 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
     if (push) {
       if (!out) {
         out = &ensure_csr(g, LL_GPU_DIR_OUT, level);
-        qdeg.alloc(V * 4, s);
-        qofs.alloc((V + 1) * 8, s);
-        qn.alloc(8, s);
+        mem.alloc_push(V, in.E, s);
       }
       // the output words start at zero: clear the listed vertices, or all
       if (nx_list == kUnlisted || (nx_list >= 0 && nx_n > V / 16)) {
@@ -886,10 +913,10 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
       }
       if (fr_list == kUnlisted) {
         // the list buffers are free: the output's list (if any) was read above
-        k_zero_ull<<<1, 1, 0, s>>>(qn.as<unsigned long long>());
+        k_zero_ull<<<1, 1, 0, s>>>(mem.qn.as<unsigned long long>());
         k_ms_queue<W><<<std::min(grid_for(V, kBlock), 4u * unsigned(ctx->num_cus)), kBlock, 0,
-                        s>>>(fr.as<W>(), V, lst[0].as<uint32_t>(), qn.as<unsigned long long>());
-        LLG_HIP(hipMemcpyAsync(ctx->readback, qn.p, 8, hipMemcpyDeviceToHost, s));
+                        s>>>(fr.as<W>(), V, lst[0].as<uint32_t>(), mem.qn.as<unsigned long long>());
+        LLG_HIP(hipMemcpyAsync(ctx->readback, mem.qn.p, 8, hipMemcpyDeviceToHost, s));
         LLG_HIP(hipStreamSynchronize(s));
         fr_list = 0;
         fr_n = *static_cast<const uint64_t*>(ctx->readback);
@@ -900,24 +927,23 @@ void msbfs_batch(ll_gpu_graph* g, int level, const int64_t* d_roots, int n, int 
       // out-degree of every vertex it discovers, once)
       const uint64_t nblk = (m_f + kPushEdges - 1) / kPushEdges;
       if (fr_n > 0 && nblk > 0) {
-        k_queue_deg<<<grid_for(fr_n, 256), 256, 0, s>>>(q, fr_n, outdeg, qdeg.as<uint32_t>());
-        scan_u32_to_u64(qdeg.as<uint32_t>(), qofs.as<uint64_t>(), fr_n, s);
-        blk.alloc(nblk * 16, s);
-        k_push_blocks<<<grid_for(nblk, 256), 256, 0, s>>>(qofs.as<uint64_t>(), fr_n, m_f, nblk,
-                                                          blk.as<uint64_t>());
+        k_queue_deg<<<grid_for(fr_n, 256), 256, 0, s>>>(q, fr_n, outdeg, mem.qdeg.as<uint32_t>());
+        scan_u32_to_u64(mem.qdeg.as<uint32_t>(), mem.qofs.as<uint64_t>(), fr_n, s);
+        k_push_blocks<<<grid_for(nblk, 256), 256, 0, s>>>(mem.qofs.as<uint64_t>(), fr_n, m_f, nblk,
+                                                          mem.blk.as<uint64_t>());
         TimedLaunch t(ctx, "k_ms_push");
         k_ms_push<W><<<unsigned(nblk), kBlock, 0, s>>>(
-            q, qofs.as<uint64_t>(), blk.as<uint64_t>(), m_f, out->ofs.as<uint64_t>(),
+            q, mem.qofs.as<uint64_t>(), mem.blk.as<uint64_t>(), m_f, out->ofs.as<uint64_t>(),
             out->adj.as<uint32_t>(), fr.as<W>(), vis.as<W>(), nx.as<W>(), touched.as<uint32_t>(),
             tl.as<uint32_t>(), a.found);
       }
       k_ms_settle<W><<<std::min(grid_for(V, kBlock), 4u * unsigned(ctx->num_cus)), kBlock, 0, s>>>(
           a, tl.as<uint32_t>(), touched.as<uint32_t>(), lst[out_list].as<uint32_t>());
     } else if (binned) {
-      if (!sv.p) sv.alloc(std::max<uint64_t>(in.E, 1) * sizeof(W), s);
+      mem.alloc_slots<W>(in.E, s);
       TimedLaunch t(ctx, "k_msb_sweep");
       with_bin_bits(pb->bb, [&](auto k) {
-        launch_binned<k(), W>(*pb, fr.as<W>(), sv.as<W>(), a, indeg, s);
+        launch_binned<k(), W>(*pb, fr.as<W>(), mem.sv.as<W>(), a, indeg, s);
       });
     } else {
       {
@@ -968,18 +994,37 @@ int autotune_lanes(ll_gpu_graph* g, int level, const int64_t* roots, int n) {
   LLG_HIP(hipMemcpyAsync(d_roots.p, roots, size_t(m) * 8, hipMemcpyHostToDevice, s));
   llgpu::EventPair ev;
   hipEvent_t e0 = ev.a, e1 = ev.b;
+  // What a snapshot builds once comes before any trial, a trial's memory before
+  // its first event and its release after the second, so that no width is
+  // charged for them: the sort behind a layout takes 3.7 ms at 2^24 vertices
+  // (a batch of 64 lanes 4.1), allocating and releasing a batch's buffers 3.6 ms
+  // at 2^22 (a batch 0.9), whichever width comes first.
+  const RowBlocks& rb = ensure_rowblocks(g, LL_GPU_DIR_IN, level, kCap, kPiece);
+  ensure_csr(g, LL_GPU_DIR_OUT, level);
+  for (uint32_t d : {LL_GPU_DIR_OUT, LL_GPU_DIR_IN}) ensure_degrees(g, d, level);
   int best = 64;
   double best_t = 1e300;
   for (int w : {16, 32, 64, 128}) {
     const int k = std::min(m, w);
-    LLG_HIP(hipEventRecord(e0, s));
+    auto batch = [&](auto lane) {
+      using W = decltype(lane);
+      MsWork mem;
+      mem.alloc<W>(g->V, rb, s);
+      mem.alloc_push(g->V, in.E, s);
+      try {
+        if (batch_bins<W>(g, level)) mem.alloc_slots<W>(in.E, s);
+      } catch (const Error&) {  // a batch without binned sweeps does without
+      }
+      LLG_HIP(hipEventRecord(e0, s));
+      msbfs_batch<W>(g, level, d_roots.as<int64_t>(), k, 0, nullptr, nullptr, nullptr, mem);
+      LLG_HIP(hipEventRecord(e1, s));
+    };
     switch (w) {
-      case 16: msbfs_batch<uint16_t>(g, level, d_roots.as<int64_t>(), k, 0, nullptr, nullptr, nullptr); break;
-      case 32: msbfs_batch<uint32_t>(g, level, d_roots.as<int64_t>(), k, 0, nullptr, nullptr, nullptr); break;
-      case 64: msbfs_batch<uint64_t>(g, level, d_roots.as<int64_t>(), k, 0, nullptr, nullptr, nullptr); break;
-      default: msbfs_batch<W128>(g, level, d_roots.as<int64_t>(), k, 0, nullptr, nullptr, nullptr); break;
+      case 16: batch(uint16_t{}); break;
+      case 32: batch(uint32_t{}); break;
+      case 64: batch(uint64_t{}); break;
+      default: batch(W128{}); break;
     }
-    LLG_HIP(hipEventRecord(e1, s));
     LLG_HIP(hipEventSynchronize(e1));
     float ms = 0;
     LLG_HIP(hipEventElapsedTime(&ms, e0, e1));
@@ -1025,15 +1070,19 @@ int ll_gpu_bfs_batch_ex(ll_gpu_graph* g, int level, const int64_t* roots, int n,
     d_reached.alloc(size_t(n) * 8, s);
     k_fill_i32<<<grid_for(uint64_t(n) * 2, 256), 256, 0, s>>>(d_reached.as<int32_t>(),
                                                             uint64_t(n) * 2, 0);
+    MsWork mem;
     for (int b = 0; b < n; b += lane_width) {
       const int m = std::min(lane_width, n - b);
       int32_t* lvp = levels_out ? d_lv.as<int32_t>() : nullptr;
       unsigned long long* rp = d_reached.as<unsigned long long>();
+      auto batch = [&](auto lane) {
+        msbfs_batch<decltype(lane)>(g, level, d_roots.as<int64_t>(), m, b, lvp, rp, sweeps, mem);
+      };
       switch (lane_width) {
-        case 16: msbfs_batch<uint16_t>(g, level, d_roots.as<int64_t>(), m, b, lvp, rp, sweeps); break;
-        case 32: msbfs_batch<uint32_t>(g, level, d_roots.as<int64_t>(), m, b, lvp, rp, sweeps); break;
-        case 64: msbfs_batch<uint64_t>(g, level, d_roots.as<int64_t>(), m, b, lvp, rp, sweeps); break;
-        default: msbfs_batch<W128>(g, level, d_roots.as<int64_t>(), m, b, lvp, rp, sweeps); break;
+        case 16: batch(uint16_t{}); break;
+        case 32: batch(uint32_t{}); break;
+        case 64: batch(uint64_t{}); break;
+        default: batch(W128{}); break;
       }
     }
     if (levels_out) copy_to_host(g->ctx, levels_out, d_lv.p, size_t(n) * V * 4);

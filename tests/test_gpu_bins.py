@@ -2,12 +2,14 @@
 are bit-identical to those over explicit bins of 2^12 vertices (row sums are
 integers) and within 1e-6 L1 of the FP64 oracle, and multi-source sweeps over
 it give every lane its single-source levels."""
+import time
+
 import numpy as np
 import pytest
 
 import oracle
 from conftest import gpu_case
-from llama_amd.graph import DeviceGraph, HostGraph
+from llama_amd.graph import DeviceGraph, GpuContext, HostGraph, SlcsrGraph, csr_of
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +90,32 @@ def test_wide_lanes_build_their_own_layout_alone(ctx, E, lane_layout):
     for j, root in enumerate(roots):
         one, n, _ = dg.bfs(int(root))
         assert np.array_equal(lv[j], one) and reached[j] == n
+
+
+def test_autotuned_width_is_a_fast_one():
+    """The width chosen on a new snapshot costs no more than the best explicit
+    one (a fifth allowed; runs differ by 5%): what a width's trial finds
+    unbuilt or unallocated is not held against it."""
+    V, E, n = 1 << 22, 9_600_000, 512
+    rng = np.random.default_rng(8)
+    src, dst = np.zeros(E, np.int64), np.zeros(E, np.int64)
+    for _ in range(22):  # R-MAT
+        r = rng.random(E)
+        src = 2 * src + (r >= 0.76)
+        dst = 2 * dst + (((r >= 0.57) & (r < 0.76)) | (r >= 0.95))
+    ids = rng.permutation(V)
+    src, dst = ids[src], ids[dst]
+    roots = src[rng.integers(0, E, n)]
+    own = GpuContext(0)
+    try:
+        dg = SlcsrGraph(own, V, csr_of(V, src, dst), csr_of(V, dst, src))
+        took = {}
+        for w in (0, 16, 32, 64, 128):
+            gpu_case(f"autotuned width, {w} lanes")
+            for _ in range(4):
+                t0 = time.perf_counter()
+                dg.bfs_batch(roots, w, want_levels=False)
+                took[w] = min(took.get(w, 1e9), time.perf_counter() - t0)
+        assert took[0] <= 1.2 * min(took[w] for w in (16, 32, 64, 128)), took
+    finally:
+        own.close()
