@@ -167,8 +167,11 @@ void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
                              hipMemcpyDeviceToHost, c->stream));
       LLG_HIP(hipEventRecord(c->chunk_ev[i], c->stream));
     }
-    std::atomic<size_t> ready{0};  // chunks in the staging; n + 1 = given up
-    hipError_t err = hipSuccess;
+    // the threads wake with the first chunk, not before: the work queued ahead
+    // of the copy may take as long as it likes, and they spin for a chunk
+    hipError_t err = hipEventSynchronize(c->chunk_ev[0]);
+    LLG_HIP(err);
+    std::atomic<size_t> ready{1};  // chunks in the staging; n + 1 = given up
     c->copies.run((m + slice - 1) / slice,
                   [&](size_t i) {
                     const size_t o = i * slice;
@@ -178,7 +181,7 @@ void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
                     if (r <= n) std::memcpy(d + off + o, stage + o, std::min(slice, m - o));
                   },
                   [&] {
-                    for (size_t i = 0; i < n && err == hipSuccess; i++) {
+                    for (size_t i = 1; i < n && err == hipSuccess; i++) {
                       err = hipEventSynchronize(c->chunk_ev[i]);
                       ready.store(err == hipSuccess ? i + 1 : n + 1, std::memory_order_release);
                     }

@@ -2,12 +2,13 @@
 changes: the read-back buffer (64 KiB), one chunk (1 MiB), chunks of 512 KiB
 and 2 MiB (8 MiB), and more than the staging holds (64 MiB)."""
 import threading
+import time
 
 import numpy as np
 import pytest
 
 from conftest import gpu_case
-from llama_amd.graph import DIR_IN, DIR_OUT, GpuContext, SlcsrGraph
+from llama_amd.graph import DIR_IN, DIR_OUT, GpuContext, SlcsrGraph, csr_of
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +58,20 @@ def test_contexts_on_threads():
     for t in ts:
         t.join()
     assert not bad
+
+
+def test_no_thread_spins_while_kernels_run(ctx):
+    """A result whose kernels are still queued is awaited by the caller alone:
+    push PageRank queues all its iterations and then copies 8 MiB.  One thread
+    waiting costs at most the wall time; half as much again is left for the
+    copy itself."""
+    V = 1 << 20
+    rng = np.random.default_rng(2)
+    src, dst = rng.integers(0, V, 8 * V), rng.integers(0, V, 8 * V)
+    dg = SlcsrGraph(ctx, V, csr_of(V, src, dst), csr_of(V, dst, src))
+    dg.pagerank_push(2)
+    gpu_case("push PageRank, CPU time")
+    wall, cpu = time.perf_counter(), time.process_time()
+    dg.pagerank_push(200)
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert wall > 0.05 and cpu <= 1.5 * wall, (wall, cpu)
