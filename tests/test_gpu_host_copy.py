@@ -1,11 +1,13 @@
 """Results and uploads through the staging buffer, at the sizes where the path
 changes: the read-back buffer (64 KiB), one chunk (1 MiB), chunks of 512 KiB
 and 2 MiB (8 MiB), and more than the staging holds (64 MiB)."""
+import ctypes
 import threading
 import time
 
 import numpy as np
 import pytest
+import torch
 
 from conftest import gpu_case
 from llama_amd.graph import DIR_IN, DIR_OUT, GpuContext, SlcsrGraph, csr_of
@@ -75,3 +77,29 @@ def test_no_thread_spins_while_kernels_run(ctx):
     dg.pagerank_push(200)
     wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
     assert wall > 0.05 and cpu <= 1.5 * wall, (wall, cpu)
+
+
+def test_pinned_destination(ctx):
+    """A caller's pinned array is filled by the device itself, at the rate of a
+    plain copy into it (through the staging: 1.6 times as long)."""
+    V, E = 1000, 48_000_000
+    dg, _, vals = graph(ctx, V, E, 5)
+    buf = torch.zeros(E, dtype=torch.int32, pin_memory=True)
+    out = buf.numpy().view(np.uint32)
+    ptr = out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32))
+    dev = torch.ones(E, dtype=torch.int32, device="cuda")
+
+    def best(f):
+        times = []
+        for _ in range(6):
+            t0 = time.perf_counter()
+            f()
+            times.append(time.perf_counter() - t0)
+        return min(times)
+
+    gpu_case("pinned destination")
+    plain = best(lambda: buf.copy_(dev))
+    ours = best(lambda: ctx.check(
+        dg.lib.ll_gpu_snapshot_adjacency(dg._h, -1, DIR_OUT, None, ptr)))
+    assert np.array_equal(out, vals.astype(np.uint32))
+    assert ours <= 1.25 * plain, (ours, plain)
