@@ -1,6 +1,8 @@
 """Weighted PageRank sweeps at the edges of the sweep items: rows of 0, 1, 8,
 32, 33, 255..257, 511..513, 767..769 and thousands of entries, graphs whose x
 fits the LDS table and one that does not, against FP64."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -77,3 +79,37 @@ def test_out_edges_alone(ctx, V):
         r.backward(torch.ones(V, device="cuda"))
         got.append((r.detach(), wt.grad, pt.grad))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_isolated_vertices_cost_little(ctx):
+    """A few connected vertices among 4 M isolated ones: the first call on the
+    snapshot writes 34 MB of row offsets per direction (10 us at the copy rate)
+    and sorts nearly nothing; 20 ms are many times what it needs."""
+    V, n, m = 1 << 22, 2000, 20_000
+    rng = np.random.default_rng(3)
+    ids = rng.permutation(V)[:n]
+    src, dst = ids[rng.integers(0, n, m)], ids[rng.integers(0, n, m)]
+    src, dst = np.concatenate([src, dst]), np.concatenate([dst, src])
+    ofs, adj = csr_of(V, src, dst)
+    tail = np.repeat(np.arange(V), np.diff(ofs))
+    dg = SlcsrGraph(ctx, V, (ofs, adj), csr_of(V, dst, src))
+    w = (rng.random(adj.size) / 30).astype(np.float32)
+    p = np.ones(V, np.float32)
+    wt = torch.tensor(w, device="cuda", requires_grad=True)
+    pt = torch.tensor(p, device="cuda", requires_grad=True)
+    grad = torch.ones(V, device="cuda")
+    gpu_case("wpr, isolated vertices")
+    best = 1e9
+    for _ in range(3):
+        dg.drop_snapshots()
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        r = weighted_pagerank(wt, pt, dg, K, D)
+        r.backward(grad)
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t0)
+    w64, x = w.astype(np.float64), p.astype(np.float64)
+    for _ in range(K):
+        x = (1 - D) * p + D * np.bincount(adj, w64 * x[tail], V)
+    assert np.all(np.abs(r.detach().cpu().numpy() - x) <= TOL * x)
+    assert best < 0.02, best
