@@ -280,6 +280,7 @@ struct PrBins {
 // One direction of the weighted PageRank sweeps (built by wpr.hip).
 struct WprMatrix {
   int level = -1;
+  bool table = false;  // hot entries of x in LDS, rows and columns numbered by `slot`
   DevBuf slot;      // uint32_t[V]: number of each vertex's row and column (empty: its ID)
   DevBuf perm;      // uint32_t[E]: entry -> out-edge position (empty: its own)
   Csr csr;          // not valid: the snapshot's out-CSR
@@ -432,6 +433,10 @@ void drop_snapshots(ll_gpu_graph* g);
 void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes);
 // inv[v] = position of v by descending `deg` (ties by ID).
 void degree_slots(ll_gpu_ctx* ctx, const uint32_t* deg, uint64_t V, DevBuf& inv);
+// Sum of the k largest a[v] + b[v] (b may be null); a lower bound of it when
+// more than k vertices have 4095 or more.
+uint64_t top_degree_sum(ll_gpu_ctx* ctx, const uint32_t* a, const uint32_t* b, uint64_t V,
+                        uint64_t k);
 // Column segments of `in` (source IDs mapped through `inv` when given) with
 // segments of 2^zb slots (zb raised until at most kMaxSegments segments).
 void build_pr_segments(ll_gpu_graph* g, const Csr& in, const uint32_t* inv, uint32_t zb,

@@ -219,6 +219,33 @@ __global__ void k_max_u32(const uint32_t* x, uint64_t n, uint32_t* out) {
     atomicMax(out, m);
   }
 }
+// Vertices by degree a + b (b may be null), the last bin holding all past the
+// others; out[kDegBins] = the degree sum of the last bin.
+constexpr uint32_t kDegBins = 4096;
+constexpr uint32_t kDegWords = kDegBins + 1;
+__global__ __launch_bounds__(1024) void k_degree_hist(const uint32_t* a, const uint32_t* b,
+                                                      uint64_t V, unsigned long long* out) {
+  __shared__ uint32_t h[kDegBins];
+  for (uint32_t i = threadIdx.x; i < kDegBins; i += blockDim.x) h[i] = 0;
+  __syncthreads();
+  unsigned long long over = 0;
+  for (uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < V;
+       v += uint64_t(gridDim.x) * blockDim.x) {
+    const uint64_t d = uint64_t(a[v]) + (b ? b[v] : 0u);
+    const uint32_t bin = uint32_t(min(d, uint64_t(kDegBins - 1)));
+    if (bin == kDegBins - 1) over += d;
+    atomicAdd(&h[bin], 1u);
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < kDegBins; i += blockDim.x)
+    if (h[i]) atomicAdd(&out[i], (unsigned long long)h[i]);
+  for (int o = 32; o > 0; o >>= 1) over += __shfl_down(over, o, 64);
+  if ((threadIdx.x & 63) == 0 && over) atomicAdd(&out[kDegBins], over);
+}
+__global__ void k_fill_u64(unsigned long long* p, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
 __global__ void k_deg_keys(const uint32_t* outdeg, uint32_t maxdeg, uint32_t* keys, uint32_t* ids,
                            uint64_t V) {
   uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -331,6 +358,31 @@ void degree_slots(ll_gpu_ctx* ctx, const uint32_t* deg, uint64_t V, DevBuf& inv)
   inv.alloc(V * 4, s);
   k_inv_from_sorted<<<grid_for(V, 256), 256, 0, s>>>(sids.as<uint32_t>(), inv.as<uint32_t>(), V);
   LLG_HIP(hipGetLastError());
+}
+
+uint64_t top_degree_sum(ll_gpu_ctx* ctx, const uint32_t* a, const uint32_t* b, uint64_t V,
+                        uint64_t k) {
+  hipStream_t s = ctx->stream;
+  DevBuf hist;
+  hist.alloc(kDegWords * 8, s);
+  k_fill_u64<<<grid_for(kDegWords, 256), 256, 0, s>>>(hist.as<unsigned long long>(), kDegWords);
+  k_degree_hist<<<std::min(grid_for(V, 1024), unsigned(ctx->num_cus)), 1024, 0, s>>>(
+      a, b, V, hist.as<unsigned long long>());
+  LLG_HIP(hipGetLastError());
+  uint64_t h[kDegWords];
+  copy_to_host(ctx, h, hist.p, sizeof h);
+  // from the highest degree down; the last bin holds all past the others, of
+  // which the k-th part is a lower bound
+  const uint64_t over = h[kDegBins - 1];
+  if (over > k) return uint64_t(double(h[kDegBins]) * double(k) / double(over));
+  uint64_t sum = h[kDegBins];
+  k -= over;
+  for (uint32_t d = kDegBins - 1; d-- > 0 && k > 0;) {
+    const uint64_t n = std::min<uint64_t>(h[d], k);
+    sum += n * d;
+    k -= n;
+  }
+  return sum;
 }
 
 // Run `iters` pull iterations; leaves FP32 ranks in rank_final (device).

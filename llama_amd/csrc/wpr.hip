@@ -87,11 +87,13 @@ __device__ inline void wave_sync() {
 // with workgroup-wide items and the same LDS table.  Lanes per row 8 / rows of
 // 32 by a lane: 7.94 ms for 100 sweeps, 16 / 16: 8.22, 8 / 8: 8.14; a table of
 // 8192 entries: 8.87.
-__global__ __launch_bounds__(kSpBlock) void k_wspmv(SpArgs a) {
+template <bool kTable>
+__global__ __launch_bounds__(kTable ? kSpBlock : kBlock) void k_wspmv(SpArgs a) {
   constexpr uint32_t kPer = kEnt / 64;
-  constexpr uint32_t kWaves = kSpBlock / 64;
+  constexpr uint32_t kThreads = kTable ? kSpBlock : kBlock;
+  constexpr uint32_t kWaves = kThreads / 64;
   constexpr uint32_t kRowPer = kRowsPerItem / 64;
-  __shared__ float hot[kHot];
+  __shared__ float hot[kTable ? kHot : 1];
   __shared__ float s_vals[kWaves][kEnt];
   __shared__ uint16_t s_rofs[kWaves][kRowsPerItem + 1];
   __shared__ uint16_t s_list[kWaves][kEnt / kThreadRow];  // rows left to lane groups
@@ -130,18 +132,22 @@ __global__ __launch_bounds__(kSpBlock) void k_wspmv(SpArgs a) {
   };
   SpItem cur = uniform(fetch(i)), nxt = uniform(fetch(i + stride));
   load(cur);
-  for (uint32_t q = threadIdx.x; q < kHot; q += kSpBlock) hot[q] = q < a.nx ? a.x[q] : 0.f;
-  __syncthreads();
+  if (kTable) {
+    for (uint32_t q = threadIdx.x; q < kHot; q += kThreads) hot[q] = q < a.nx ? a.x[q] : 0.f;
+    __syncthreads();
+  }
   for (; i < a.nitems; i += stride) {
     const uint32_t ne = cur.meta & 0xfffu, nrows = (cur.meta >> 12) & 0xfffu;
     const uint32_t kind = cur.meta >> 24;
     const SpItem after = fetch(i + 2 * stride);
     float xv[kPer];
 #pragma unroll
-    for (uint32_t k = 0; k < kPer; k++) xv[k] = idx[k] >= kHot ? a.x[idx[k]] : 0.f;
+    for (uint32_t k = 0; k < kPer; k++) xv[k] = !kTable || idx[k] >= kHot ? a.x[idx[k]] : 0.f;
+    if (kTable) {
 #pragma unroll
-    for (uint32_t k = 0; k < kPer; k++)
-      if (idx[k] < kHot) xv[k] = hot[idx[k]];
+      for (uint32_t k = 0; k < kPer; k++)
+        if (idx[k] < kHot) xv[k] = hot[idx[k]];
+    }
     if (kind == kRun) {
 #pragma unroll
       for (uint32_t k = 0; k < kPer; k++)
@@ -307,6 +313,27 @@ __global__ void k_columns(const uint32_t* perm, const uint32_t* column, const ui
   col[i] = slot ? slot[c] : c;
 }
 
+// Length of every row by its number.
+__global__ void k_row_lengths(const uint64_t* ofs, const uint32_t* slot, uint64_t V,
+                              uint32_t* len) {
+  const uint64_t u = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (u < V) len[slot[u]] = uint32_t(ofs[u + 1] - ofs[u]);
+}
+
+// Every edge to its row's new place, its column numbered; perm names its old
+// position.  A thread per edge: a wave per row spent 80 ms on one row of 7.6 M
+// edges.
+__global__ void k_move_entries(const uint64_t* ofs, const uint32_t* adj, const uint32_t* tail,
+                               const uint32_t* slot, const uint64_t* new_ofs, uint32_t* perm,
+                               uint32_t* col, uint64_t n) {
+  const uint64_t e = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const uint32_t u = tail[e];
+  const uint64_t to = new_ofs[slot[u]] + (e - ofs[u]);
+  perm[to] = uint32_t(e);
+  col[to] = slot[adj[e]];
+}
+
 // xs[slot[v]] = x[v].
 __global__ void k_to_slots(const float* x, const uint32_t* slot, float* xs, uint64_t n) {
   const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -371,19 +398,33 @@ void build_sweep_items(ll_gpu_ctx* ctx, const Csr& c, WprMatrix& m) {
       rb.items.as<RowItem>(), rb.slots.as<uint32_t>(), rb.n, c.ofs.as<uint64_t>(),
       m.items.as<SpItem>(), m.splits.as<SpSplit>(), cnt.as<uint32_t>());
   LLG_HIP(hipGetLastError());
-  LLG_HIP(hipMemcpyAsync(ctx->readback, cnt.p, 4, hipMemcpyDeviceToHost, s));
-  LLG_HIP(hipStreamSynchronize(s));
-  m.nsplits = *static_cast<const uint32_t*>(ctx->readback);
+  if (rb.nsplit) {
+    LLG_HIP(hipMemcpyAsync(ctx->readback, cnt.p, 4, hipMemcpyDeviceToHost, s));
+    LLG_HIP(hipStreamSynchronize(s));
+    m.nsplits = *static_cast<const uint32_t*>(ctx->readback);
+  }
   m.n = rb.n;
   m.nparts = rb.nsplit;
 }
 
+// Whether x's hottest entries are worth an LDS table: they hold kHotShare of
+// the columns, and the graph is large enough, and its rows long enough, for 96
+// KiB copied per workgroup and rows numbered anew.  50 iterations forward and back, ms with table /
+// plain (first call on a snapshot in brackets): R-MAT of 16 edges a vertex
+// (share) 24576 vertices 1.8 / 1.1; 200003 (0.85) 2.54 / 2.48 [5.9 / 4.7];
+// 400000 (0.75) 3.5 / 4.1; 2^20 (0.65) 7.7 / 10.6 [17.5 / 16.0]; 2^22 (0.47)
+// 39 / 69 [55 / 78].  Even degrees: 2^20 (0.04) 12.5 / 10.7 [21.6 / 16.2], 24577
+// 1.5 / 0.8.  Power laws whose IDs already ascend by degree: 2^20 (0.29) 10.8 /
+// 10.4, (0.39) 10.3 / 9.8, (0.59) 9.6 / 9.1, 2^22 (0.36) 57 / 53: there the
+// table loses 5%, with IDs in any order it wins as on R-MAT.
+constexpr uint64_t kTableV = uint64_t(1) << 18;
+constexpr double kHotShare = 0.3;
+
 // The matrix of one direction of the sweeps.  forward: rows = heads, columns =
 // tails; adjoint: rows = tails, columns = heads.  Entries of a row in out-edge
-// order.  Rows and columns are numbered by descending degree on the column
-// side, unless all of x fits the LDS table anyway.  The adjoint's rows are the
-// out-CSR's own when they keep their numbers (also past 2^32 edges, where no
-// u32 permutation exists).
+// order.  With a table, rows and columns are numbered by descending degree on
+// the column side; else they keep their IDs, and the adjoint's matrix is the
+// out-CSR itself (also past 2^32 edges, where no u32 permutation exists).
 const WprMatrix& ensure_wpr_matrix(ll_gpu_graph* g, int level, bool forward) {
   level = resolve_level(g, level);
   WprMatrix& m = g->wpr[forward ? 0 : 1];
@@ -395,13 +436,7 @@ const WprMatrix& ensure_wpr_matrix(ll_gpu_graph* g, int level, bool forward) {
   const bool fits = E < (uint64_t(1) << 32);
   LLG_CHECK(fits || !forward, LL_GPU_ERANGE, "weighted PageRank needs E < 2^32");
   m = WprMatrix();
-  const bool renumber = V > kHot && fits;
-  if (!forward && !renumber) {
-    build_sweep_items(ctx, out, m);
-    m.level = level;
-    return m;
-  }
-  if (renumber) {
+  if (fits && V >= kTableV && E / 4 >= V) {
     DevBuf counted;
     const uint32_t* deg;
     if (!forward && g->slcsr && !g->sl[LL_GPU_DIR_IN].valid) {
@@ -415,33 +450,54 @@ const WprMatrix& ensure_wpr_matrix(ll_gpu_graph* g, int level, bool forward) {
     } else {
       deg = ensure_degrees(g, forward ? LL_GPU_DIR_OUT : LL_GPU_DIR_IN, level);
     }
-    degree_slots(ctx, deg, V, m.slot);
+    m.table = double(top_degree_sum(ctx, deg, nullptr, V, kHot)) >= kHotShare * double(E);
+    if (m.table) degree_slots(ctx, deg, V, m.slot);
+  }
+  if (!forward && !m.table) {
+    build_sweep_items(ctx, out, m);
+    m.level = level;
+    return m;
   }
   const uint32_t* slot = m.slot.as<uint32_t>();
-  const uint64_t n = std::max<uint64_t>(E, 1);
-  DevBuf tail, key, pos, rows;
-  tail.alloc(n * 4, s);
-  key.alloc(n * 4, s);
-  pos.alloc(n * 4, s);
-  rows.alloc(n * 4, s);
-  m.perm.alloc(n * 4, s);
-  k_edge_tails<<<unsigned(std::min<uint64_t>((V + 3) / 4, uint64_t(ctx->num_cus) * 32)), 256, 0,
-                 s>>>(out.ofs.as<uint64_t>(), V, tail.as<uint32_t>());
   const uint32_t* heads = out.adj.as<uint32_t>();
-  k_row_keys<<<grid_for(E, 256), 256, 0, s>>>(forward ? heads : tail.as<uint32_t>(), slot,
-                                              key.as<uint32_t>(), pos.as<uint32_t>(), E);
-  LLG_HIP(hipGetLastError());
-  int bits = 1;
-  while (bits < 32 && ((V - 1) >> bits) != 0) bits++;
-  sort_pairs_u32_u32(key.as<uint32_t>(), rows.as<uint32_t>(), pos.as<uint32_t>(),
-                     m.perm.as<uint32_t>(), E, bits, s, false);
+  const uint64_t n = std::max<uint64_t>(E, 1);
+  m.perm.alloc(n * 4, s);
   m.csr.ofs.alloc((V + 1) * 8, s);
   m.csr.adj.alloc(n * 4, s);
-  k_row_offsets<<<grid_for(V + 1, 256), 256, 0, s>>>(rows.as<uint32_t>(), E, V,
-                                                     m.csr.ofs.as<uint64_t>());
-  k_columns<<<grid_for(E, 256), 256, 0, s>>>(m.perm.as<uint32_t>(),
-                                             forward ? tail.as<uint32_t>() : heads, slot,
-                                             m.csr.adj.as<uint32_t>(), E);
+  DevBuf tail;  // the forward's sort keys first
+  tail.alloc(n * 4, s);
+  auto edge_tails = [&]() {
+    k_edge_tails<<<unsigned(std::min<uint64_t>((V + 3) / 4, uint64_t(ctx->num_cus) * 32)), 256, 0,
+                   s>>>(out.ofs.as<uint64_t>(), V, tail.as<uint32_t>());
+  };
+  if (forward) {
+    DevBuf pos, rows;
+    pos.alloc(n * 4, s);
+    rows.alloc(n * 4, s);
+    k_row_keys<<<grid_for(E, 256), 256, 0, s>>>(heads, slot, tail.as<uint32_t>(),
+                                                pos.as<uint32_t>(), E);
+    LLG_HIP(hipGetLastError());
+    int bits = 1;
+    while (bits < 32 && ((V - 1) >> bits) != 0) bits++;
+    sort_pairs_u32_u32(tail.as<uint32_t>(), rows.as<uint32_t>(), pos.as<uint32_t>(),
+                       m.perm.as<uint32_t>(), E, bits, s, false);
+    edge_tails();
+    k_row_offsets<<<grid_for(V + 1, 256), 256, 0, s>>>(rows.as<uint32_t>(), E, V,
+                                                       m.csr.ofs.as<uint64_t>());
+    k_columns<<<grid_for(E, 256), 256, 0, s>>>(m.perm.as<uint32_t>(), tail.as<uint32_t>(), slot,
+                                               m.csr.adj.as<uint32_t>(), E);
+  } else {
+    // the rows are the out-CSR's, whole, in another order: nothing to sort
+    DevBuf len;
+    len.alloc(V * 4, s);
+    edge_tails();
+    k_row_lengths<<<grid_for(V, 256), 256, 0, s>>>(out.ofs.as<uint64_t>(), slot, V,
+                                                   len.as<uint32_t>());
+    scan_u32_to_u64(len.as<uint32_t>(), m.csr.ofs.as<uint64_t>(), V, s);
+    k_move_entries<<<grid_for(E, 256), 256, 0, s>>>(
+        out.ofs.as<uint64_t>(), heads, tail.as<uint32_t>(), slot, m.csr.ofs.as<uint64_t>(),
+        m.perm.as<uint32_t>(), m.csr.adj.as<uint32_t>(), E);
+  }
   LLG_HIP(hipGetLastError());
   m.csr.valid = true;
   m.csr.level = level;
@@ -491,14 +547,17 @@ void wpr_sweeps(ll_gpu_graph* g, int level, bool forward, const float* w, const 
   a.base_scale = base_scale;
   a.d = d;
   a.part = part.as<double>();
-  constexpr uint64_t kWaves = kSpBlock / 64;
-  const unsigned grid =
-      unsigned(std::min<uint64_t>((m.n + kWaves - 1) / kWaves, uint64_t(ctx->num_cus)));
+  const uint64_t per = (m.table ? kSpBlock : kBlock) / 64;  // waves of a workgroup
+  // with a table one workgroup fits a CU and its copy is to be shared by many
+  // items; else as many as there are items, up to many a CU (8 a CU: 5% slower)
+  const unsigned grid = unsigned(std::min<uint64_t>(
+      (m.n + per - 1) / per, uint64_t(ctx->num_cus) * (m.table ? 1 : 64)));
   for (int it = 0; it < iters; it++) {
     a.y = it == iters - 1 && !slot ? out : buf[it & 1].as<float>();
     {
       TimedLaunch t(ctx, name);
-      k_wspmv<<<grid, kSpBlock, 0, s>>>(a);
+      if (m.table) k_wspmv<true><<<grid, kSpBlock, 0, s>>>(a);
+      else k_wspmv<false><<<grid, kBlock, 0, s>>>(a);
     }
     if (a.nsplits) k_wspmv_split<<<grid_for(uint64_t(a.nsplits) * kSplitLanes, 64), 64, 0, s>>>(a);
     LLG_HIP(hipGetLastError());
