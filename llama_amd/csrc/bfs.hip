@@ -187,17 +187,29 @@ __device__ inline bool claim(uint32_t v, uint64_t* visited, int32_t* lv, int32_t
   return true;
 }
 
+// Whether a level goes bottom-up: the frontier's out-edges exceed the
+// unexplored edges / alpha.
+__host__ __device__ inline bool goes_bottom_up(uint64_t m_f, uint64_t m_visited, uint64_t E,
+                                               uint64_t alpha) {
+  return m_f > (E > m_visited ? E - m_visited : 0) / alpha;
+}
+
 // Level 1, before the host has seen the root's degree: the root's out-edges
-// in blocks of kEdgesPerBlock over a fixed grid.
+// in blocks of kEdgesPerBlock over a fixed grid.  A root that goes bottom-up
+// at once is left to the host (`start`: the root's counters; E, e_reach: the
+// edges a search can reach without and with the reach set).
 __global__ __launch_bounds__(kBlock) void k_root_expand(uint32_t root, const uint64_t* ofs,
                                                         const uint32_t* adj,
                                                         const uint32_t* outdeg,
                                                         uint64_t* visited, int32_t* lv,
-                                                        uint32_t* q_next, Counters* c) {
+                                                        uint32_t* q_next, Counters* c,
+                                                        const Counters* start, uint64_t E,
+                                                        uint64_t e_reach, uint64_t alpha) {
   __shared__ uint32_t l_q[kEdgesPerBlock];
   __shared__ uint32_t l_qn;
   __shared__ unsigned long long l_qbase;
   const uint64_t e0 = ofs[root], e1 = ofs[root + 1];
+  if (goes_bottom_up(e1 - e0, e1 - e0, start->aux ? e_reach : E, alpha)) return;
   for (uint64_t x0 = e0 + uint64_t(blockIdx.x) * kEdgesPerBlock; x0 < e1;
        x0 += uint64_t(gridDim.x) * kEdgesPerBlock) {
     const uint64_t x1 = min(e1, x0 + kEdgesPerBlock);
@@ -739,8 +751,7 @@ __global__ __launch_bounds__(kTinyBlock) void k_bfs_tiny(
   int32_t lvl = 0;
   int cur = 0;
   while (n_f > 0 && m_f > 0) {
-    const uint64_t m_u = E > m_vis ? E - m_vis : 0;
-    const bool bottom_up = nq > kTinyQueue || m_f > m_u / alpha;
+    const bool bottom_up = nq > kTinyQueue || goes_bottom_up(m_f, m_vis, E, alpha);
     __syncthreads();  // the level before is read
     for (uint32_t i = tid; i < words; i += kTinyBlock) nx[i] = 0;
     if (tid == 0) {
@@ -934,32 +945,42 @@ BfsResult bfs_core_ws(ll_gpu_graph* g, const Csr& fwd, const Csr& rev, const uin
                                    w.cnt, 3);
   k_bfs_init<<<grid_for(std::max(V, words), 256), 256, 0, s>>>(
       lv, w.visited, excluded, notr, w.cnt, V, words, root, fdeg, w.q[0]);
-  k_root_expand<<<64, kBlock, 0, s>>>(root, fwd.ofs.as<uint64_t>(), fwd.adj.as<uint32_t>(), fdeg,
-                                      w.visited, lv, w.q[1], w.cnt + kStripes);
+  // a root that is expanded here has at most E / (alpha + 1) out-edges (a search
+  // of 4 M vertices from a root with a million: 0.62 ms with 64 workgroups for
+  // them, 0.54 with 512; from one with 4 M, left to the bottom-up level, 0.25
+  // against 1.07)
+  const unsigned root_grid =
+      std::min(std::max(grid_for(std::min(V, fwd.E / (alpha + 1)), kEdgesPerBlock), 64u),
+               2u * unsigned(ctx->num_cus));
+  k_root_expand<<<root_grid, kBlock, 0, s>>>(root, fwd.ofs.as<uint64_t>(), fwd.adj.as<uint32_t>(),
+                                             fdeg, w.visited, lv, w.q[1], w.cnt + kStripes, w.cnt,
+                                             fwd.E, e_reach, alpha);
   LLG_HIP(hipGetLastError());
   Counters h0[2];
   read_counter_sets(ctx, w.cnt, 2, h0);
-  Counters h = h0[1];
   const unsigned bu_grid = std::min(grid_for(V, kBlock), 8u * unsigned(ctx->num_cus));
   const uint32_t open_per = open_words_per_wave(words);
   const unsigned open_grid = grid_for(words, uint32_t(kOpenWaves) * open_per);
-  uint64_t nq = h.n_next;       // queue entries (vertices with out-edges)
-  uint64_t n_f = h.found;       // frontier vertices
-  uint64_t m_f = h.m_next;      // frontier out-edges
-  uint64_t m_visited = h0[0].m_next + h.m_next;
-  r.reached = 1 + h.found;
-  r.examined = h.examined;
-  bool bottom_up = false;
-  int td = 2;   // counter set of the next top-down level (zeroed)
-  int cur = 1;
-  int32_t lvl = h0[0].m_next > 0 ? 1 : 0;
   // out-edges a search can still reach: those inside R when R excludes the rest
   const uint64_t E = h0[0].aux ? e_reach : fwd.E;
+  // the frontier: level 1, or the root where its level goes bottom-up
+  const uint64_t m_root = h0[0].m_next;
+  const bool expanded = m_root > 0 && !goes_bottom_up(m_root, m_root, E, alpha);
+  Counters h = h0[expanded ? 1 : 0];
+  uint64_t nq = h.n_next;                        // queue entries (vertices with out-edges)
+  uint64_t n_f = expanded ? h.found : 1;         // frontier vertices
+  uint64_t m_f = h.m_next;                       // frontier out-edges
+  uint64_t m_visited = expanded ? m_root + h.m_next : m_root;
+  r.reached = expanded ? 1 + h.found : 1;
+  r.examined = h.examined;
+  bool bottom_up = false;
+  int td = expanded ? 2 : 1;  // counter set of the next top-down level (zeroed)
+  int cur = expanded ? 1 : 0;
+  int32_t lvl = expanded ? 1 : 0;
   // beta 0: no return to top-down
   const uint64_t beta = b_opt > 0 ? uint64_t(b_opt) : (h0[0].aux ? 0 : 24);
   while (n_f > 0 && m_f > 0) {
-    const uint64_t m_u = E > m_visited ? E - m_visited : 0;
-    if (!bottom_up && m_f > m_u / alpha) {
+    if (!bottom_up && goes_bottom_up(m_f, m_visited, E, alpha)) {
       bottom_up = true;
       k_fill_u64<<<grid_for(words, 256), 256, 0, s>>>(fbm, words, 0);
       k_queue_to_bitmap<<<grid_for(nq, 256), 256, 0, s>>>(w.q[cur], nq,

@@ -84,3 +84,42 @@ def test_levels(ctx, name, V):
             finally:
                 ctx.set_option(opt, 1 if opt == "bfs_reach" else -1)
             assert np.array_equal(lv2, ref) and reached2 == reached
+
+
+def forms(ctx, search):
+    """The forms a search ran: launches of the one-workgroup search, of
+    top-down levels past the first and of bottom-up levels."""
+    ctx.profile(True)
+    try:
+        out = search()
+        return out, [ctx.kernel_time(k)[0] for k in ("k_bfs_tiny", "k_td_expand", "k_bu_step")]
+    finally:
+        ctx.profile(False)
+
+
+# 45400 edges among the others: 4540 are at most a tenth of them
+@pytest.mark.parametrize("hub_edges,bottom_up", [(1, False), (4540, False), (4541, True),
+                                                 (40000, True)])
+def test_first_level_of_a_hub(ctx, hub_edges, bottom_up):
+    """A root whose out-edges exceed the unexplored ones / alpha starts
+    bottom-up, others top-down; the leaves lead nowhere, so level 1 is the
+    last one."""
+    V = 40001
+    rng = np.random.default_rng(hub_edges)
+    leaf = 1 + rng.choice(V - 1, hub_edges, replace=False)
+    ring = np.arange(V, V + 100)  # edges the search never sees
+    src = np.concatenate([np.zeros(hub_edges, np.int64), np.repeat(ring, 454)])
+    dst = np.concatenate([leaf, np.tile(ring, 454)])
+    g = HostGraph(V + 100)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    ctx.set_option("bfs_reach", 0)
+    try:
+        dg.bfs(0)
+        gpu_case(f"bfs hub of {hub_edges} edges")
+        (lv, reached, _), (tiny, _, bu) = forms(ctx, lambda: dg.bfs(0))
+    finally:
+        ctx.set_option("bfs_reach", 1)
+    assert np.array_equal(lv, levels_of(V + 100, src, dst, 0)) and reached == 1 + hub_edges
+    assert dg.last_bfs_traversed == hub_edges
+    assert (tiny, bu > 0) == (0, bottom_up)
