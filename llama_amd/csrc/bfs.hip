@@ -697,17 +697,21 @@ __global__ void k_dead_rows(const uint64_t* ofs, uint64_t V, uint64_t words, uin
 // launches and host round trips of the level-by-level form: visited, frontier
 // and next-frontier bitmaps and the frontier queues in LDS.  A level goes
 // top-down from the queue (the workgroup over one vertex's edges while the
-// queue is short, else a wave per vertex) until the frontier's out-edges
+// queue is short or the row long, else a wave per vertex) until the frontier's out-edges
 // exceed the unexplored edges / alpha or a level finds more than kTinyQueue
 // vertices, bottom-up then (a thread per open row).  The counts go straight
 // to the host's read-back buffer.  Bound by the latency of one CU's loads, so
 // it stops where the whole chip catches up; us per search, counts only, this
 // form / level by level: 5000 vertices, 80000 edges 70 / 147; 20000, 320000
 // 119 / 215; 32000, 512000 137 / 153; 65000, 520000 262 / 180; 65000, 1.04 M
-// 263 / 156.
+// 263 / 156.  A row of 25000 out-edges among twenty short ones: 256 us by one
+// wave, 99 by the workgroup.  Bottom-up rows stay with a thread each, also the
+// long ones: a hub of 15000 in-edges reached last, the worst for them, 4.6 ms
+// against 25.7 level by level (2000: 1.0 / 5.3).
 constexpr uint64_t kTinyV = 32768;
 constexpr uint64_t kTinyE = 600000;
 constexpr uint32_t kTinyQueue = 4096;
+constexpr uint32_t kTinyLong = 4096;  // out-edges past which a queued row takes the workgroup
 constexpr int kTinyBlock = 1024;
 struct TinyResult {
   unsigned long long reached, examined, traversed, levels;
@@ -721,7 +725,8 @@ __global__ __launch_bounds__(kTinyBlock) void k_bfs_tiny(
   constexpr uint32_t kWords = uint32_t(kTinyV / 64);
   __shared__ unsigned long long vis[kWords], fr[kWords], nx[kWords];
   __shared__ uint32_t q[2][kTinyQueue];
-  __shared__ uint32_t qn, found;
+  __shared__ uint32_t longq[kTinyE / kTinyLong];
+  __shared__ uint32_t qn, found, nlong;
   __shared__ unsigned long long m_next, exam;
   __shared__ int bad;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -758,6 +763,7 @@ __global__ __launch_bounds__(kTinyBlock) void k_bfs_tiny(
       qn = 0;
       found = 0;
       m_next = 0;
+      nlong = 0;
     }
     __syncthreads();
     uint32_t my_found = 0;
@@ -774,10 +780,7 @@ __global__ __launch_bounds__(kTinyBlock) void k_bfs_tiny(
       }
     };
     if (!bottom_up) {
-      const bool all = nq < kTinyBlock / 64;  // the workgroup takes one vertex at a time
-      const uint32_t step = all ? kTinyBlock : 64, at = all ? tid : lane;
-      for (uint32_t k = all ? 0 : wave; k < nq; k += all ? 1 : kTinyBlock / 64) {
-        const uint32_t u = q[cur][k];
+      auto row = [&](uint32_t u, uint32_t at, uint32_t step) {
         const uint64_t e1 = fofs[u + 1];
         for (uint64_t e = fofs[u] + at; e < e1; e += step) {
           const uint32_t v = fadj[e];
@@ -785,6 +788,17 @@ __global__ __launch_bounds__(kTinyBlock) void k_bfs_tiny(
           my_exam++;
           if (!(vis[v >> 6] & bit) && !(atomicOr(&vis[v >> 6], bit) & bit)) take(v);
         }
+      };
+      if (nq < kTinyBlock / 64) {
+        for (uint32_t k = 0; k < nq; k++) row(q[cur][k], tid, kTinyBlock);
+      } else {
+        for (uint32_t k = wave; k < nq; k += kTinyBlock / 64) {
+          const uint32_t u = q[cur][k];
+          if (fdeg[u] <= kTinyLong) row(u, lane, 64);
+          else if (lane == 0) longq[atomicAdd(&nlong, 1u)] = u;
+        }
+        __syncthreads();
+        for (uint32_t k = 0; k < nlong; k++) row(longq[k], tid, kTinyBlock);
       }
     } else {
       for (uint32_t r = tid; r < V; r += kTinyBlock) {

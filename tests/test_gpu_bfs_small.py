@@ -123,3 +123,22 @@ def test_first_level_of_a_hub(ctx, hub_edges, bottom_up):
     assert np.array_equal(lv, levels_of(V + 100, src, dst, 0)) and reached == 1 + hub_edges
     assert dg.last_bfs_traversed == hub_edges
     assert (tiny, bu > 0) == (0, bottom_up)
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 25_000])
+def test_long_rows_of_a_wide_level(ctx, n):
+    """Twenty vertices queued together, three of them with n out-edges: at most
+    a tenth of the edges, so their level goes top-down."""
+    V = 32768
+    rng = np.random.default_rng(n)
+    mid = np.arange(1, 21)
+    src = np.concatenate([np.zeros(20, np.int64), mid, np.repeat(mid[:3], n // 3 if n > 9000 else n),
+                          rng.integers(21, V, 500_000)])
+    dst = np.concatenate([mid, 21 + rng.integers(0, V - 21, src.size - 20)])
+    g = HostGraph(V)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    dg.bfs(0)
+    gpu_case(f"bfs long rows of {n}")
+    (lv, _, _), (tiny, _, _) = forms(ctx, lambda: dg.bfs(0))
+    assert tiny == 1 and np.array_equal(lv, levels_of(V, src, dst, 0))
