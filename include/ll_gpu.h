@@ -316,7 +316,9 @@ int ll_gpu_tuned(ll_gpu_ctx* ctx, const char* prefix, int* value);
  * out-edges exceed the unexplored edges / alpha, back to top-down when a
  * shrinking frontier holds under max_nodes / beta vertices; <= 0 = defaults:
  * alpha 10; beta 24, or no return to top-down for a search that treats the
- * rows outside the snapshot's reach set as visited), "bfs_batch_bins"
+ * rows outside the snapshot's reach set as visited; snapshots of at most
+ * 32768 vertices and 600000 edges are searched by one workgroup, which reads
+ * alpha alone), "bfs_batch_bins"
  * (multi-source BFS sweeps over the binned out-edge layout of "pr_bin_bits":
  * -1 = automatic = where that layout exists and fits the lane width in LDS,
  * for the sweeps that do not push while the rows some search has not reached

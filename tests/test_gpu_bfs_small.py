@@ -1,7 +1,9 @@
 """Searches on both sides of the one-workgroup form's limits (32768 vertices,
-600000 edges): shapes with one level per vertex, a level past the in-LDS
-queue (4096), no out-edges, several components, rows of every length around
-the long-row bound, against a plain queue search."""
+600000 edges) and the form each of them runs: shapes with one level per vertex,
+a level past the in-LDS queue (4096), no out-edges, several components, rows
+around the length that takes the whole workgroup (4096 out-edges), hubs whose
+first level goes either way, and a search that returns to top-down, against a
+plain queue search."""
 from collections import deque
 
 import numpy as np
@@ -76,7 +78,8 @@ def test_levels(ctx, name, V):
         assert np.array_equal(lv, ref)
         assert reached == int((ref != UNREACHED).sum())
         assert dg.last_bfs_traversed == int(deg[ref != UNREACHED].sum())
-        # the same without the reach set, and with a return to top-down
+        # the same without the reach set, and (past the limits) with the option
+        # that lets a search return to top-down
         for opt, val in (("bfs_reach", 0), ("bfs_beta", 8)):
             ctx.set_option(opt, val)
             try:
@@ -123,6 +126,50 @@ def test_first_level_of_a_hub(ctx, hub_edges, bottom_up):
     assert np.array_equal(lv, levels_of(V + 100, src, dst, 0)) and reached == 1 + hub_edges
     assert dg.last_bfs_traversed == hub_edges
     assert (tiny, bu > 0) == (0, bottom_up)
+
+
+@pytest.mark.parametrize("V,E,one_workgroup", [
+    (32768, 599_999, True), (32768, 600_000, True), (32768, 600_001, False), (1000, 600_001, False),
+    (32769, 600_000, False), (32769, 1000, False), (32768, 1000, True)])
+def test_form_limits(ctx, V, E, one_workgroup):
+    rng = np.random.default_rng(E)
+    src, dst = rng.integers(0, V, E), (V * rng.random(E) ** 2).astype(np.int64)
+    g = HostGraph(V)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    root = int(src[0])
+    dg.bfs(root)
+    gpu_case(f"bfs limits V={V} E={E}")
+    (lv, _, _), (tiny, td, bu) = forms(ctx, lambda: dg.bfs(root))
+    assert np.array_equal(lv, levels_of(V, src, dst, root))
+    assert tiny == (1 if one_workgroup else 0)
+    assert not one_workgroup or td + bu == 0
+
+
+def test_return_to_top_down(ctx):
+    """A dense part, which goes bottom-up, and a tail of one vertex a level:
+    with bfs_beta the search returns to top-down for the tail, without it
+    stays bottom-up (the whole graph is the reach set)."""
+    n, tail = 40_000, 60
+    V = n + tail
+    rng = np.random.default_rng(4)
+    t = np.arange(n, V)
+    src = np.concatenate([rng.integers(0, n, 8 * n), [0], t])
+    dst = np.concatenate([rng.integers(0, n, 8 * n), [n], t[1:], [0]])
+    g = HostGraph(V)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    ref = levels_of(V, src, dst, 1)
+    dg.bfs(1)
+    for beta, returns in ((8, True), (-1, False)):
+        gpu_case(f"bfs return to top-down, beta {beta}")
+        ctx.set_option("bfs_beta", beta)
+        try:
+            (lv, _, _), (_, td, bu) = forms(ctx, lambda: dg.bfs(1))
+        finally:
+            ctx.set_option("bfs_beta", -1)
+        assert np.array_equal(lv, ref)
+        assert bu > 0 and (td >= tail // 2) == returns  # the dense part ends within ten levels
 
 
 @pytest.mark.parametrize("n", [4095, 4096, 4097, 25_000])
