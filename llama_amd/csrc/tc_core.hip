@@ -51,16 +51,6 @@ __global__ void k_zero_ull(unsigned long long* p, uint32_t n) {
   if (threadIdx.x < n) p[threadIdx.x] = 0;
 }
 
-// Degree sum of the vertices numbered from `first` on.
-__global__ __launch_bounds__(256) void k_core_degrees(const uint32_t* sorted_deg, uint64_t first,
-                                                      uint64_t V, unsigned long long* sum) {
-  unsigned long long t = 0;
-  for (uint64_t i = first + uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < V;
-       i += uint64_t(gridDim.x) * blockDim.x)
-    t += sorted_deg[i];
-  block_atomic_add(sum, t);
-}
-
 // The key of a self-loop: all ones, past every arc's.
 __host__ __device__ inline uint64_t no_arc(uint32_t vb) {
   return vb >= 32 ? ~uint64_t(0) : (uint64_t(1) << (2 * vb)) - 1;
@@ -291,8 +281,34 @@ bool ensure_tc_core(ll_gpu_graph* g, int level) {
   t = TcCore();
   DevBuf num;
   const uint32_t core0 = uint32_t(V > kCore ? V - kCore : 0);
+  if (core0) {
+    // Entries outside the core cost several times a bit test.  With a share
+    // x of the edge ends outside, x^2 of the arcs lie wholly outside (and
+    // fewer of the list entries, the more skewed the graph).  Milliseconds of
+    // a count, this form / by vertex ID, at x^2, [first call on a snapshot]:
+    // R-MAT of 16 edges a vertex 2^20 vertices (0.10) 2.2 / 10.8 [8.2 / 16.2],
+    // 2^22 (0.23) 11.8 / 55 [22 / 67], 2^24 123 / 308; even degrees 90000
+    // vertices, 64 edges (0.36) 0.67 / 0.67 [2.8 / 3.7], 100000 (0.41) 0.80 /
+    // 0.72 [2.9 / 3.8], 120000 (0.49) 1.18 / 0.79 [3.3 / 4.0].
+    // With hubs among many small vertices the lists end in the core all the
+    // same: R-MAT 2^20 and uniform edges, half as many (0.28) 3.1 / 11.4, as
+    // many (0.41) 4.1 / 11.9, twice (0.56) 8.3 / 13.4, four times (0.70) 29 /
+    // 17.9; 2^22 half (0.42) 16 / 58, as many (0.54) 22 / 60, twice (0.67) 45 /
+    // 67, four times (0.79) 142 / 87.  So the limit is higher where the core's
+    // vertices have 16 times the mean degree (2^22: 23 to 67), and not as high
+    // as it could be.  The share comes from a histogram of the degrees, before
+    // any sort (a rejected graph of 4 M vertices paid 2.1 ms for one).
+    const double in_core = double(top_degree_sum(ctx, dout, din, V, kCore));
+    const double x = E ? 1.0 - in_core / (2.0 * double(E)) : 0.0;
+    const double hub = (1.0 - x) * double(V) / kCore;  // mean degree of the core over all
+    if (x * x > (hub >= 16 ? 0.5 : 0.42)) {
+      t.level = level;
+      t.usable = false;
+      return false;
+    }
+  }
   {
-    DevBuf key, id, skey, sid, sum;
+    DevBuf key, id, skey, sid;
     key.alloc(V * 4, s);
     id.alloc(V * 4, s);
     skey.alloc(V * 4, s);
@@ -304,31 +320,6 @@ bool ensure_tc_core(ll_gpu_graph* g, int level) {
                        sid.as<uint32_t>(), V, 32, s);
     k_number<<<grid_for(V, 256), 256, 0, s>>>(sid.as<uint32_t>(), num.as<uint32_t>(), V);
     LLG_HIP(hipGetLastError());
-    if (core0) {
-      // Entries outside the core cost several times a bit test.  With a share
-      // x of the edge ends outside, x^2 of the arcs lie wholly outside (and
-      // fewer of the list entries, the more skewed the graph).  Count only,
-      // this form / by vertex ID: R-MAT 2^20 vertices 2.2 / 10.8 ms, 2^22 11.8
-      // / 55, 2^24 123 / 308 (16 edges per vertex); even degrees 90000 vertices
-      // (x^2 0.40) 0.16 / 0.18 ms, 100000 with 64 edges (0.45) 0.83 / 0.76.
-      // Where the core's vertices have 16 times the mean degree or more the
-      // lists end in it all the same: R-MAT 2^24 with 10% of uniform edges
-      // inserted (x^2 between 0.42 and 0.5) 124 / 304.
-      sum.alloc(8, s);
-      k_zero_ull<<<1, 64, 0, s>>>(sum.as<unsigned long long>(), 1);
-      k_core_degrees<<<256, 256, 0, s>>>(skey.as<uint32_t>(), core0, V,
-                                         sum.as<unsigned long long>());
-      LLG_HIP(hipGetLastError());
-      uint64_t in_core = 0;
-      copy_to_host(ctx, &in_core, sum.p, 8);
-      const double x = E ? 1.0 - double(in_core) / (2.0 * double(E)) : 0.0;
-      const double hub = (1.0 - x) * double(V) / kCore;  // mean degree of the core over all
-      if (x * x > (hub >= 16 ? 0.5 : 0.42)) {
-        t.level = level;
-        t.usable = false;
-        return false;
-      }
-    }
   }
   uint32_t vb = 1;
   while (vb < 32 && ((V - 1) >> vb) != 0) vb++;

@@ -3,12 +3,14 @@ vertices), past it with hubs (most lists in the core), past it with even
 degrees (many entries outside: the filter and its confirmation), and too even
 for it (the form by vertex ID), against the CPU count; W and the arcs equal
 the definition."""
+import time
+
 import numpy as np
 import pytest
 
 import oracle
 from conftest import gpu_case
-from llama_amd.graph import DeviceGraph, HostGraph
+from llama_amd.graph import DIR_IN, DIR_OUT, DeviceGraph, HostGraph, SlcsrGraph, csr_of
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +76,29 @@ def test_hubs_beside_many_small_vertices(ctx, outside):
     n, arcs, work = dg.triangles(stats=True)
     assert n == oracle.OracleGraph.from_host(g).triangles()
     assert (arcs, work) == dag_stats(V, src, dst)
+
+
+def test_rejected_graph_pays_no_sort(ctx):
+    """Even degrees far past the core: the rule answers from a histogram and no
+    vertex is numbered, so the first call is the DAG by vertex ID and a scan of
+    the degrees (32 MB: 7 us at the copy rate; half a millisecond allowed)."""
+    V = 4_000_000
+    rng = np.random.default_rng(5)
+    src, dst = rng.integers(0, V, 2 * V), rng.integers(0, V, 2 * V)
+    dg = SlcsrGraph(ctx, V, csr_of(V, src, dst), csr_of(V, dst, src))
+
+    def best(f):
+        times = []
+        for _ in range(6):
+            dg.drop_snapshots()
+            dg.degrees(DIR_OUT)
+            dg.degrees(DIR_IN)
+            dg.adjacency(DIR_OUT)
+            t0 = time.perf_counter()
+            f()
+            times.append(time.perf_counter() - t0)
+        return min(times)
+
+    gpu_case("tc rejected graph")
+    # tc_i builds the same DAG without the rule, and its count is the slower one
+    assert best(dg.triangles) <= best(dg.tc_i) + 0.0005
