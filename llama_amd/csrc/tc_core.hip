@@ -3,7 +3,7 @@
 // Arcs go from lower to higher (degree, ID), as in tc.hip; here that order is
 // the numbering itself, so the neighbours of a list are its hubs-to-be and the
 // kCore highest numbers (the core) hold nearly every list entry of a skewed
-// graph.  A row a sets the bits of N+(a) within the core in an LDS bitmap (8
+// graph.  A row a sets the bits of N+(a) within the core in an LDS bitmap (4
 // KiB a wave); the core part of every N+(b), b in N+(a), is then streamed as
 // 16-bit offsets and each entry costs one LDS bit test.  Entries outside the
 // core -- only neighbours of a b that is itself outside -- pass a hashed bit
@@ -369,10 +369,14 @@ void tc_core_count(ll_gpu_graph* g, uint64_t* triangles, uint64_t* work, uint64_
   k_zero_ull<<<1, 64, 0, s>>>(out.as<unsigned long long>(), 3);
   {
     TimedLaunch tl(ctx, "k_tc_core");
-    // four workgroups fit a CU; more of them even out the rows of a large graph
-    const unsigned grid = unsigned(std::min<uint64_t>(
-        (g->V + kWaves - 1) / kWaves,
-        uint64_t(ctx->num_cus) * (g->V > (uint64_t(1) << 20) ? 32 : 8)));
+    // four workgroups fit a CU; more of them even out the rows of a large graph,
+    // and each clears its bitmaps once more.  us a count by workgroups a CU 8 /
+    // 16 / 32, R-MAT of 16 edges a vertex: 100000 vertices 167 / 220 / 351,
+    // 300000 442 / 411 / 471, 700000 1210 / 1133 / 1113, 2^20 2214 / 2020 /
+    // 1981, 2^22 13191 / 12253 / 11800; 64: 1964 and 11699 at the last two
+    const uint64_t per_cu = g->V > (uint64_t(1) << 19) ? 32 : g->V > (uint64_t(1) << 17) ? 16 : 8;
+    const unsigned grid = unsigned(std::min<uint64_t>((g->V + kWaves - 1) / kWaves,
+                                                      uint64_t(ctx->num_cus) * per_cu));
     const TcCoreArgs a{t.ofs.as<uint64_t>(), t.nbr.as<uint32_t>(), t.nbc.as<uint16_t>(),
                        t.nout.as<uint32_t>(), g->V, out.as<unsigned long long>()};
     if (t.arcs < (uint64_t(1) << 32)) k_tc_core<uint32_t><<<grid, kWaves * 64, 0, s>>>(a);
