@@ -1,9 +1,11 @@
 """Betweenness around one hub whose in-edges and out-edges are split into
 pieces of 1536 entries that one wave joins 64 at a time: the path counts and
-the terms are whole numbers, so the expected values are exact."""
+the terms are whole numbers, so the expected values are exact.  And rows whose
+starts lie around the words of 64 entries that name an entry's row."""
 import numpy as np
 import pytest
 
+import oracle
 from conftest import gpu_case
 from llama_amd.graph import DeviceGraph, HostGraph
 
@@ -30,3 +32,23 @@ def test_hub_split_into_pieces(ctx, mids, leaves):
     want[hub] = leaves
     want[mid] = np.float32(1) / np.float32(mids) * (np.float32(1) + np.float32(leaves))
     assert np.array_equal(b, want)
+
+
+@pytest.mark.parametrize("empty", [0, 1, 63, 200, 300])
+def test_row_starts(ctx, empty):
+    """Rows of 0, 1, 63, 64, 65, 127..129 and 511 entries in any order, with
+    runs of empty rows between them, bit for bit as the oracle adds them."""
+    gpu_case(f"bc row starts, runs of {empty} empty rows")
+    rng = np.random.default_rng(empty)
+    lengths = []
+    for n in rng.permutation([0, 1, 2, 63, 64, 65, 127, 128, 129, 511] * 4):
+        lengths += [n] + [0] * (empty if rng.random() < 0.2 else 0)
+    V = max(len(lengths), 2000)
+    rows = np.repeat(np.arange(len(lengths)), lengths)
+    ends = rng.integers(0, V, rows.size)
+    extra = rng.integers(0, V, (2, 3 * V))
+    g = HostGraph(V)
+    g.add_level(np.concatenate([rows, ends, extra[0]]), np.concatenate([ends, rows, extra[1]]))
+    sources = rng.integers(0, V, 5)
+    assert np.array_equal(DeviceGraph(ctx, g).bc(sources),
+                          oracle.OracleGraph.from_host(g).bc(sources))
