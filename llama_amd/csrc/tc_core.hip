@@ -138,7 +138,7 @@ struct TcCoreArgs {
 // ones: 2.3; workgroups of 8 waves instead of 4: 2.2.
 // I: type of an arc position.
 template <typename I>
-__global__ __launch_bounds__(kWaves * 64) void k_tc_core(TcCoreArgs a) {
+__global__ __launch_bounds__(kWaves * 64, 8) void k_tc_core(TcCoreArgs a) {
   __shared__ uint32_t s_bits[kWaves][kCore / 32 + 1];
   __shared__ uint32_t s_filter[kWaves][kFilterBits / 32];
   __shared__ unsigned long long red[3][kWaves];
@@ -151,98 +151,118 @@ __global__ __launch_bounds__(kWaves * 64) void k_tc_core(TcCoreArgs a) {
   wave_sync();
   unsigned long long count = 0, work = 0, maxrow = 0;
   const uint64_t nw = uint64_t(gridDim.x) * kWaves;
-  for (uint64_t r = uint64_t(blockIdx.x) * kWaves + wave; r < a.V; r += nw) {
-    const uint64_t row = a.V - 1 - r;
-    const uint64_t a0 = a.ofs[row], a1 = a.ofs[row + 1];
-    const uint64_t na = a1 - a0;
-    if (na == 0) continue;
-    const uint32_t outside = a.nout[row];
-    const uint64_t c0 = a0 + outside;
-    for (uint64_t e = c0 + lane; e < a1; e += 64) {
-      const uint32_t x = a.nbc[e];
-      atomicOr(&bits[x >> 5], 1u << (x & 31));
-    }
-    for (uint64_t e = a0 + lane; e < c0; e += 64) {
-      const uint32_t h = filter_bit(a.nbr[e]);
-      atomicOr(&filter[h >> 5], 1u << (h & 31));
-    }
-    wave_sync();
-    uint32_t c = 0;
-    unsigned long long el = 0;
-    for (uint64_t i0 = 0; i0 < na; i0 += 64) {
-      const uint64_t i = i0 + lane;
-      I start = 0, ostart = 0;
-      uint32_t len = 0, olen = 0;
-      if (i < na) {
-        const uint32_t b = a.nbr[a0 + i];
-        const uint64_t b0 = a.ofs[b], b1 = a.ofs[b + 1];
-        const uint32_t bo = a.nout[b];
-        el += b1 - b0;
-        start = I(b0 + bo);
-        len = uint32_t(b1 - b0) - bo;
-        if (i < outside && outside > 1) {
-          ostart = I(b0);
-          olen = bo;
-        }
+  for (uint64_t r0 = uint64_t(blockIdx.x) * kWaves + wave; r0 < a.V; r0 += 64 * nw) {
+    // the wave's next 64 rows, a lane each; those of one arc close no triangle
+    // and are done there
+    const uint64_t mine = r0 + lane * nw;
+    uint64_t mine_a0 = 0;
+    uint32_t mine_na = 0, mine_out = 0;
+    if (mine < a.V) {
+      const uint64_t row = a.V - 1 - mine;
+      mine_a0 = a.ofs[row];
+      mine_na = uint32_t(a.ofs[row + 1] - mine_a0);
+      if (mine_na == 1) {
+        const uint32_t b = a.nbr[mine_a0];
+        const unsigned long long el = a.ofs[b + 1] - a.ofs[b];
+        work += el + 1;
+        maxrow = el > maxrow ? el : maxrow;
+      } else if (mine_na > 1) {
+        mine_out = a.nout[row];
       }
-      if (na < 2) break;  // one arc closes no triangle
-      // the core parts of the 64 lists, in pieces of 64 entries
-      uint64_t todo = __ballot(len != 0);
-      I at = 0;
-      uint32_t left = 0;
-      while (todo || left) {
-        uint32_t n[kGroup];
-        uint16_t w[kGroup];
-#pragma unroll
-        for (int q = 0; q < kGroup; q++) {
-          if (left == 0 && todo) {
-            const int j = __ffsll((long long)todo) - 1;
-            todo &= todo - 1;
-            at = lane_val(start, j);
-            left = lane_val(len, j);
+    }
+    for (uint64_t todo_rows = __ballot(mine_na > 1); todo_rows; todo_rows &= todo_rows - 1) {
+      const int rj = __ffsll((long long)todo_rows) - 1;
+      const uint64_t a0 = lane_val(mine_a0, rj);
+      const uint64_t na = lane_val(mine_na, rj), a1 = a0 + na;
+      const uint32_t outside = lane_val(mine_out, rj);
+      const uint64_t c0 = a0 + outside;
+      for (uint64_t e = c0 + lane; e < a1; e += 64) {
+        const uint32_t x = a.nbc[e];
+        atomicOr(&bits[x >> 5], 1u << (x & 31));
+      }
+      for (uint64_t e = a0 + lane; e < c0; e += 64) {
+        const uint32_t h = filter_bit(a.nbr[e]);
+        atomicOr(&filter[h >> 5], 1u << (h & 31));
+      }
+      wave_sync();
+      uint32_t c = 0;
+      unsigned long long el = 0;
+      for (uint64_t i0 = 0; i0 < na; i0 += 64) {
+        const uint64_t i = i0 + lane;
+        I start = 0, ostart = 0;
+        uint32_t len = 0, olen = 0;
+        if (i < na) {
+          const uint32_t b = a.nbr[a0 + i];
+          const uint64_t b0 = a.ofs[b], b1 = a.ofs[b + 1];
+          const uint32_t bo = a.nout[b];
+          el += b1 - b0;
+          start = I(b0 + bo);
+          len = uint32_t(b1 - b0) - bo;
+          if (i < outside && outside > 1) {
+            ostart = I(b0);
+            olen = bo;
           }
-          n[q] = min(left, 64u);
-          w[q] = (a.nbc + at)[lane];  // past the piece: other entries, or the padding
-          at += n[q];
-          left -= n[q];
         }
+        // the core parts of the 64 lists, in pieces of 64 entries
+        uint64_t todo = __ballot(len != 0);
+        I at = 0;
+        uint32_t left = 0;
+        while (todo || left) {
+          uint32_t n[kGroup];
+          uint16_t w[kGroup];
 #pragma unroll
-        for (int q = 0; q < kGroup; q++) {
-          const uint32_t x = lane < n[q] ? uint32_t(w[q]) : kNone;
-          c += (bits[x >> 5] >> (x & 31)) & 1u;
-        }
-      }
-      // the entries outside the core of the lists of vertices outside it
-      for (uint64_t om = __ballot(olen != 0); om; om &= om - 1) {
-        const int j = __ffsll((long long)om) - 1;
-        const I s0 = lane_val(ostart, j);
-        const uint32_t n = lane_val(olen, j);
-        for (uint32_t t = lane; t < n; t += 64) {
-          const uint32_t w = a.nbr[s0 + t];
-          const uint32_t h = filter_bit(w);
-          if (!((filter[h >> 5] >> (h & 31)) & 1u)) continue;
-          uint64_t lo = a0, hi = c0;
-          while (lo < hi) {
-            const uint64_t mid = (lo + hi) >> 1;
-            if (a.nbr[mid] < w) lo = mid + 1;
-            else hi = mid;
+          for (int q = 0; q < kGroup; q++) {
+            if (left == 0 && todo) {
+              const int j = __ffsll((long long)todo) - 1;
+              todo &= todo - 1;
+              at = lane_val(start, j);
+              left = lane_val(len, j);
+            }
+            n[q] = min(left, 64u);
+            w[q] = (a.nbc + at)[lane];  // past the piece: other entries, or the padding
+            at += n[q];
+            left -= n[q];
           }
-          c += lo < c0 && a.nbr[lo] == w ? 1u : 0u;
+#pragma unroll
+          for (int q = 0; q < kGroup; q++) {
+            const uint32_t x = lane < n[q] ? uint32_t(w[q]) : kNone;
+            c += (bits[x >> 5] >> (x & 31)) & 1u;
+          }
+        }
+        // the entries outside the core of the lists of vertices outside it
+        for (uint64_t om = __ballot(olen != 0); om; om &= om - 1) {
+          const int j = __ffsll((long long)om) - 1;
+          const I s0 = lane_val(ostart, j);
+          const uint32_t n = lane_val(olen, j);
+          for (uint32_t t = lane; t < n; t += 64) {
+            const uint32_t w = a.nbr[s0 + t];
+            const uint32_t h = filter_bit(w);
+            if (!((filter[h >> 5] >> (h & 31)) & 1u)) continue;
+            uint64_t lo = a0, hi = c0;
+            while (lo < hi) {
+              const uint64_t mid = (lo + hi) >> 1;
+              if (a.nbr[mid] < w) lo = mid + 1;
+              else hi = mid;
+            }
+            c += lo < c0 && a.nbr[lo] == w ? 1u : 0u;
+          }
         }
       }
+      wave_sync();
+      for (uint64_t e = c0 + lane; e < a1; e += 64) bits[a.nbc[e] >> 5] = 0;
+      for (uint64_t e = a0 + lane; e < c0; e += 64) filter[filter_bit(a.nbr[e]) >> 5] = 0;
+      wave_sync();
+      count += c;
+      work += el + (lane == 0 ? na * na : 0);  // na arcs of d+(a) each, and every d+(b)
+      for (int o = 32; o > 0; o >>= 1) el += __shfl_xor(el, o, 64);
+      maxrow = el > maxrow ? el : maxrow;
     }
-    wave_sync();
-    for (uint64_t e = c0 + lane; e < a1; e += 64) bits[a.nbc[e] >> 5] = 0;
-    for (uint64_t e = a0 + lane; e < c0; e += 64) filter[filter_bit(a.nbr[e]) >> 5] = 0;
-    wave_sync();
-    count += c;
-    work += el + (lane == 0 ? na * na : 0);  // na arcs of d+(a) each, and every d+(b)
-    for (int o = 32; o > 0; o >>= 1) el += __shfl_xor(el, o, 64);
-    maxrow = el > maxrow ? el : maxrow;
   }
   for (int o = 32; o > 0; o >>= 1) {
     count += __shfl_down(count, o, 64);
     work += __shfl_down(work, o, 64);
+    const unsigned long long m = __shfl_down(maxrow, o, 64);
+    maxrow = m > maxrow ? m : maxrow;
   }
   if (lane == 0) {
     red[0][wave] = count;

@@ -102,3 +102,42 @@ def test_rejected_graph_pays_no_sort(ctx):
     gpu_case("tc rejected graph")
     # tc_i builds the same DAG without the rule, and its count is the slower one
     assert best(dg.triangles) <= best(dg.tc_i) + 0.0005
+
+
+def test_rows_of_one_arc(ctx):
+    """A star: every row has one arc and closes nothing.  24 bytes a row are 12
+    MB, 2.5 us at the copy rate; 25 times that is allowed."""
+    V = 500_001
+    leaf = np.arange(1, V)
+    g = HostGraph(V)
+    g.add_level(np.zeros(V - 1, np.int64), leaf)
+    dg = DeviceGraph(ctx, g)
+    gpu_case("tc star")
+    n, arcs, work = dg.triangles(stats=True)
+    # a leaf's row: its own d+ of 1 and the hub's of 0
+    assert (n, arcs, work) == (0, V - 1, V - 1)
+    ctx.profile(True)
+    try:
+        for _ in range(10):
+            dg.triangles()
+        k, ms = ctx.kernel_time("k_tc_core")
+    finally:
+        ctx.profile(False)
+    assert k == 10 and ms / k < 0.0625, ms / k
+
+
+def test_many_row_lengths(ctx):
+    """Rows of no, one, two, 63..65 and more arcs beside each other, more rows
+    than the waves' first 64, against the CPU count."""
+    V = 300_000
+    rng = np.random.default_rng(6)
+    src = np.repeat(np.arange(V), rng.choice([0, 1, 1, 2, 3, 63, 64, 65], V,
+                                             p=[.5, .2, .1, .1, .07, .01, .01, .01]))
+    dst = (V * rng.random(src.size) ** 3).astype(np.int64)
+    g = HostGraph(V)
+    g.add_level(src, dst)
+    dg = DeviceGraph(ctx, g)
+    gpu_case("tc row lengths")
+    n, arcs, work = dg.triangles(stats=True)
+    assert n == oracle.OracleGraph.from_host(g).triangles()
+    assert (arcs, work) == dag_stats(V, src, dst)
