@@ -514,8 +514,33 @@ __global__ __launch_bounds__(256) void k_count_nonzero(const uint32_t* x, uint64
   block_atomic_add(out, c);
 }
 
+// The same by one workgroup, straight to the host's read-back buffer.
+__global__ __launch_bounds__(1024) void k_count_small(const uint32_t* x, uint32_t n,
+                                                      unsigned long long* out) {
+  __shared__ uint32_t part[16];
+  uint32_t c = 0;
+  for (uint32_t i = threadIdx.x; i < n; i += 1024) c += x[i] > 0 ? 1u : 0u;
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 16; i++) c += part[i];
+    *out = c;
+  }
+}
+
 uint64_t count_nonzero(ll_gpu_ctx* ctx, const uint32_t* x, uint64_t n) {
   hipStream_t s = ctx->stream;
+  // one launch and no copy while one workgroup walks the degrees faster than
+  // the others cost: a call over 16384 vertices 15 us, 65536 20 (35 with two
+  // launches and a copy, 12 to 29 when the host read every degree)
+  if (n <= 65536) {
+    auto* out = static_cast<unsigned long long*>(ctx->readback);
+    k_count_small<<<1, 1024, 0, s>>>(x, uint32_t(n), out);
+    LLG_HIP(hipGetLastError());
+    LLG_HIP(hipStreamSynchronize(s));
+    return *out;
+  }
   DevBuf cnt;
   cnt.alloc(8, s);
   k_zero_count<<<1, 1, 0, s>>>(cnt.as<unsigned long long>());
