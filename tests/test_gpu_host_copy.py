@@ -1,6 +1,7 @@
 """Results and uploads through the staging buffer, at the sizes where the path
-changes: the read-back buffer (64 KiB), one chunk (1 MiB), chunks of 512 KiB
-and 2 MiB (8 MiB), and more than the staging holds (64 MiB)."""
+changes: the read-back buffer (64 KiB), one piece (under 1 MiB), chunks of 2
+MiB moved on in slices of 256 KiB, and more than the staging holds (64 MiB);
+pinned destinations; what the copies cost the host."""
 import ctypes
 import threading
 import time
@@ -27,7 +28,8 @@ def graph(ctx, V, E, seed):
 
 
 # bytes of the neighbour array
-@pytest.mark.parametrize("nbytes", [4, 65532, 65536, 65540, MB - 4, MB, MB + 4, 8 * MB - 4,
+@pytest.mark.parametrize("nbytes", [4, 65532, 65536, 65540, MB - 4, MB, MB + 4, 2 * MB - 4,
+                                    2 * MB, 2 * MB + 4, 2 * MB + MB // 4 + 4, 8 * MB - 4,
                                     8 * MB + 4, 64 * MB, 64 * MB + 4, 133 * MB])
 def test_round_trip(ctx, nbytes):
     gpu_case(f"host copy {nbytes} bytes")
