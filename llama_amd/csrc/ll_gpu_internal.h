@@ -433,8 +433,8 @@ void drop_snapshots(ll_gpu_graph* g);
 void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes);
 // inv[v] = position of v by descending `deg` (ties by ID).
 void degree_slots(ll_gpu_ctx* ctx, const uint32_t* deg, uint64_t V, DevBuf& inv);
-// Sum of the k largest a[v] + b[v] (b may be null); a lower bound of it when
-// more than k vertices have 4095 or more.
+// Sum of the k largest a[v] + b[v] (b may be null), within 1/128 of the last
+// ones where they are 2048 or more.
 uint64_t top_degree_sum(ll_gpu_ctx* ctx, const uint32_t* a, const uint32_t* b, uint64_t V,
                         uint64_t k);
 // Column segments of `in` (source IDs mapped through `inv` when given) with

@@ -219,28 +219,39 @@ __global__ void k_max_u32(const uint32_t* x, uint64_t n, uint32_t* out) {
     atomicMax(out, m);
   }
 }
-// Vertices by degree a + b (b may be null), the last bin holding all past the
-// others; out[kDegBins] = the degree sum of the last bin.
-constexpr uint32_t kDegBins = 4096;
-constexpr uint32_t kDegWords = kDegBins + 1;
+// Vertices by degree a + b (b may be null): a bin per degree below 2048, then
+// 128 bins an octave, whose degree sums are kept too.
+constexpr uint32_t kExactDeg = 2048;
+constexpr uint32_t kWideBins = 22 * 128;  // degrees below 2^33
+constexpr uint32_t kDegBins = kExactDeg + kWideBins;
+constexpr uint32_t kDegWords = kDegBins + kWideBins;  // counts, then sums
+static_assert(kDegWords * 8 <= kReadbackBytes, "the histogram fits the read-back buffer");
+
+__device__ inline uint32_t degree_bin(uint64_t d) {
+  if (d < kExactDeg) return uint32_t(d);
+  const uint32_t e = 63 - uint32_t(__clzll((long long)d));
+  return kExactDeg + (e - 11) * 128 + (uint32_t(d >> (e - 7)) & 127u);
+}
+
 __global__ __launch_bounds__(1024) void k_degree_hist(const uint32_t* a, const uint32_t* b,
                                                       uint64_t V, unsigned long long* out) {
-  __shared__ uint32_t h[kDegBins];
-  for (uint32_t i = threadIdx.x; i < kDegBins; i += blockDim.x) h[i] = 0;
+  __shared__ unsigned long long sum[kWideBins];
+  __shared__ uint32_t cnt[kDegBins];
+  for (uint32_t i = threadIdx.x; i < kDegBins; i += blockDim.x) cnt[i] = 0;
+  for (uint32_t i = threadIdx.x; i < kWideBins; i += blockDim.x) sum[i] = 0;
   __syncthreads();
-  unsigned long long over = 0;
   for (uint64_t v = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; v < V;
        v += uint64_t(gridDim.x) * blockDim.x) {
     const uint64_t d = uint64_t(a[v]) + (b ? b[v] : 0u);
-    const uint32_t bin = uint32_t(min(d, uint64_t(kDegBins - 1)));
-    if (bin == kDegBins - 1) over += d;
-    atomicAdd(&h[bin], 1u);
+    const uint32_t bin = degree_bin(d);
+    atomicAdd(&cnt[bin], 1u);
+    if (bin >= kExactDeg) atomicAdd(&sum[bin - kExactDeg], (unsigned long long)d);
   }
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < kDegBins; i += blockDim.x)
-    if (h[i]) atomicAdd(&out[i], (unsigned long long)h[i]);
-  for (int o = 32; o > 0; o >>= 1) over += __shfl_down(over, o, 64);
-  if ((threadIdx.x & 63) == 0 && over) atomicAdd(&out[kDegBins], over);
+    if (cnt[i]) atomicAdd(&out[i], (unsigned long long)cnt[i]);
+  for (uint32_t i = threadIdx.x; i < kWideBins; i += blockDim.x)
+    if (sum[i]) atomicAdd(&out[kDegBins + i], sum[i]);
 }
 __global__ void k_fill_u64(unsigned long long* p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -371,15 +382,14 @@ uint64_t top_degree_sum(ll_gpu_ctx* ctx, const uint32_t* a, const uint32_t* b, u
   LLG_HIP(hipGetLastError());
   uint64_t h[kDegWords];
   copy_to_host(ctx, h, hist.p, sizeof h);
-  // from the highest degree down; the last bin holds all past the others, of
-  // which the k-th part is a lower bound
-  const uint64_t over = h[kDegBins - 1];
-  if (over > k) return uint64_t(double(h[kDegBins]) * double(k) / double(over));
-  uint64_t sum = h[kDegBins];
-  k -= over;
-  for (uint32_t d = kDegBins - 1; d-- > 0 && k > 0;) {
-    const uint64_t n = std::min<uint64_t>(h[d], k);
-    sum += n * d;
+  // from the highest degree down; of a wide bin that is not taken whole, its mean
+  uint64_t sum = 0;
+  for (uint32_t i = kDegBins; i-- > 0 && k > 0;) {
+    const uint64_t n = std::min<uint64_t>(h[i], k);
+    if (n == 0) continue;
+    if (i < kExactDeg) sum += n * i;
+    else if (n == h[i]) sum += h[kDegBins + i - kExactDeg];
+    else sum += uint64_t(double(h[kDegBins + i - kExactDeg]) * double(n) / double(h[i]));
     k -= n;
   }
   return sum;
