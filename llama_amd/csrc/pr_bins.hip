@@ -18,8 +18,9 @@
 //   C. as the same vertices are the sources of chunks (b', b) for every b',
 //      writes the next iteration's values into those chunks (each slot names
 //      its source's offset in the bin, u16): the chunks are dealt to the
-//      waves by slots, a wave keeps kGroupC pieces of 64 slots in flight
-//      whatever the chunks' lengths, and its writes are contiguous runs.
+//      waves by number (each cut into equal parts where they are fewer than
+//      the waves), a wave keeps kGroupC pieces of 64 slots in flight whatever
+//      the chunks' lengths, and its writes are contiguous runs.
 //      Neighbouring bins run on one XCD, whose L2 merges the partial lines
 //      at chunk ends.
 // Integer addition is associative, so a row sum does not depend on the order

@@ -129,13 +129,14 @@ struct TcCoreArgs {
 };
 
 // A wave per row, from the highest number down (the rows of one wave then mix
-// heavy and light ones).  Bound by instruction issue: about 12 vector and 12
-// scalar instructions per piece of 64 entries (90% full on R-MAT graphs), plus
-// the LDS bit test and the L2 read of 128 bytes.  2^20 vertices, 4.4 G entries:
-// 2.2 ms (10.8 with a bucketed search of N+(a) per entry).  A core of 65536
+// heavy and light ones), 64 rows looked at together.  Bound by instruction
+// issue: about 12 vector and 12 scalar instructions per piece of 64 entries
+// (90% full on R-MAT graphs); the vector units issue for 74% of the kernel's
+// cycles, the LDS of the bit tests for 35%.  2^20 vertices, 4.4 G entries: 2.0
+// ms (10.8 with a bucketed search of N+(a) per entry).  A core of 65536
 // numbers: 3.7 ms (half the waves fit a CU) and 16384: 3.2 against 3.1 of
 // 32768; then 32-bit positions and loads past a piece's end instead of masked
-// ones: 2.3; workgroups of 8 waves instead of 4: 2.2.
+// ones: 2.3; workgroups of 8 waves instead of 4: 2.2; more of them: 2.0.
 // I: type of an arc position.
 template <typename I>
 __global__ __launch_bounds__(kWaves * 64, 8) void k_tc_core(TcCoreArgs a) {
@@ -316,7 +317,8 @@ bool ensure_tc_core(ll_gpu_graph* g, int level) {
     // 17.9; 2^22 half (0.42) 16 / 58, as many (0.54) 22 / 60, twice (0.67) 45 /
     // 67, four times (0.79) 142 / 87.  So the limit is higher where the core's
     // vertices have 16 times the mean degree (2^22: 23 to 67), and not as high
-    // as it could be.  The share comes from a histogram of the degrees, before
+    // as it could be: R-MAT 2^26 in 11 levels (0.59) 1.53 / 1.84 s, 2^27 in 20
+    // (0.66) 5.2 / 4.5.  The share comes from a histogram of the degrees, before
     // any sort (a rejected graph of 4 M vertices paid 2.1 ms for one).
     const double in_core = double(top_degree_sum(ctx, dout, din, V, kCore));
     const double x = E ? 1.0 - in_core / (2.0 * double(E)) : 0.0;

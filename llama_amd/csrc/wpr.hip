@@ -8,11 +8,12 @@
 //   forward:  r0 = p,  r' = (1-d) p + d W^T r            (pull over in-edges)
 //   adjoint:  l0 = g,  l' = g + d W l                     (pull over out-edges)
 //             dL/dw[e=(u,v)] = d r[u] l[v],  dL/dp = (1-d) l
-// Either direction is one sweep kernel over a CSR whose rows and columns are
-// numbered by descending degree (hot columns then sit in LDS), with a
-// permutation that brings w into entry order once per call; sums are FP64.
-// Bytes per sweep: 8 per edge (column, weight) + 20 per vertex, and a gather
-// of x per edge that misses the LDS table.
+// Either direction is one sweep kernel over a CSR, with a permutation where
+// entries are not in out-edge order that brings w into theirs once per call;
+// sums are FP64.  Large skewed graphs number rows and columns by descending
+// degree, so that hot columns sit in an LDS table (kTableV, kHotShare).  Bytes
+// per sweep: 8 per edge (column, weight) + 20 per vertex (row offset, x, base,
+// y), and a gather of x per edge that misses the table.
 #include "ll_gpu_internal.h"
 #include "rowblocks.h"
 
@@ -66,25 +67,27 @@ __device__ inline void wave_sync() {
 }
 
 // One sweep: a fixed grid of waves taking items in turn, each wave on its own
-// (no workgroup barrier past the first).
+// (no workgroup barrier past the table's).
 //
-// Bound by load latency: a CU keeps few enough gathers of x from L2 in flight
-// that they, not the 8 bytes streamed per edge, set the pace.  So rows and
-// columns are numbered by descending degree: the first kHot entries of x,
-// which take most of the gathers of a skewed graph, are copied to LDS once per
-// workgroup, and the others lie close together.  Everything else an item
-// needs (entries, row offsets, base) is loaded while the wave's item before it
-// is summed.
+// Bound by load latency (with the table, waves wait for 61% of their cycles
+// and the vector units issue for 27%): a CU keeps few enough gathers of x from
+// L2 in flight that they, not the 8 bytes streamed per edge, set the pace.
+// kTable: rows and columns are numbered by descending degree, the first kHot
+// entries of x, which take most of the gathers of a skewed graph, are copied
+// to LDS once per workgroup, and the others lie close together.  Everything
+// else an item needs (entries, row offsets, base) is loaded while the wave's
+// item before it is summed.  Without: workgroups of four waves, sixteen of
+// them where LDS allowed one.
 //
 // A run of short rows: the products are staged in LDS and summed in FP64, rows
 // of up to kThreadRow entries by a lane each, longer ones by kRowLanes lanes
 // each.  A long row is cut into pieces, a wave each; k_wspmv_split adds them
 // in a fixed order, so the result does not depend on the schedule.
 //
-// 2^20 vertices, 16.8 M edges: 69 us a sweep (2.0 TB/s of streamed bytes);
-// 120 us with one workgroup per item and columns by vertex ID, 83 us with the
-// columns but not the rows renumbered (y and base then scattered), 196 us
-// with workgroup-wide items and the same LDS table.  Lanes per row 8 / rows of
+// R-MAT 2^20 vertices, 16.8 M edges, with the table: 69 us a sweep (2.0 TB/s of
+// streamed bytes); 106 without, 120 with one workgroup per item, 83 with the
+// columns but not the rows renumbered (y and base then scattered), 196 with
+// workgroup-wide items and the same LDS table.  Lanes per row 8 / rows of
 // 32 by a lane: 7.94 ms for 100 sweeps, 16 / 16: 8.22, 8 / 8: 8.14; a table of
 // 8192 entries: 8.87.
 template <bool kTable>
