@@ -3,6 +3,7 @@ changes: the read-back buffer (64 KiB), one piece (under 1 MiB), chunks of 2
 MiB moved on in slices of 256 KiB, and more than the staging holds (64 MiB);
 pinned destinations; what the copies cost the host."""
 import ctypes
+import os
 import threading
 import time
 
@@ -134,3 +135,25 @@ def test_small_results_cost_one_round_trip(ctx):
     info = best(dg.snapshot_info)
     assert np.array_equal(out, np.bincount(src, minlength=V).astype(np.uint32))
     assert deg <= 1.5 * plain and info <= 2 * plain, (deg, info, plain)
+
+
+def test_small_uploads_need_no_threads():
+    """A context starts its copy threads for the first array of 1 MiB or more,
+    up or down."""
+    def threads():
+        return len(os.listdir("/proc/self/task"))
+
+    gpu_case("small uploads")
+    c = GpuContext(0)
+    try:
+        dg, _, _ = graph(c, 1000, 100_000, 1)  # 800 KB of IDs
+        dg.adjacency(DIR_OUT)
+        before = threads()
+        dg, _, vals = graph(c, 1000, 131_071, 2)  # 1 MiB less 8 bytes
+        assert np.array_equal(dg.adjacency(DIR_OUT)[1], vals.astype(np.uint32))
+        assert threads() == before
+        dg, _, vals = graph(c, 1000, 131_072, 3)
+        assert np.array_equal(dg.adjacency(DIR_OUT)[1], vals.astype(np.uint32))
+        assert before < threads() <= before + 7
+    finally:
+        c.close()
