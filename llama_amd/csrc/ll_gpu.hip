@@ -185,22 +185,24 @@ void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
     }
     constexpr size_t chunk = size_t(2) << 20, slice = kCopySlice;
     const size_t n = (m + chunk - 1) / chunk;
-    while (c->chunk_ev.size() < n) {
+    while (c->chunk_ev.size() <= n) {
       hipEvent_t e;
       LLG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       c->chunk_ev.push_back(e);
     }
+    // the threads wake when the copy starts, not before: the work queued ahead
+    // of it may take as long as it likes, and they spin for a chunk (woken by
+    // the first chunk instead they cost a copy 35 us)
+    LLG_HIP(hipEventRecord(c->chunk_ev[n], c->stream));
     for (size_t i = 0; i < n; i++) {
       const size_t o = i * chunk;
       LLG_HIP(hipMemcpyAsync(stage + o, p + off + o, std::min(chunk, m - o),
                              hipMemcpyDeviceToHost, c->stream));
       LLG_HIP(hipEventRecord(c->chunk_ev[i], c->stream));
     }
-    // the threads wake with the first chunk, not before: the work queued ahead
-    // of the copy may take as long as it likes, and they spin for a chunk
-    hipError_t err = hipEventSynchronize(c->chunk_ev[0]);
-    LLG_HIP(err);
-    std::atomic<size_t> ready{1};  // chunks in the staging; n + 1 = given up
+    LLG_HIP(hipEventSynchronize(c->chunk_ev[n]));
+    hipError_t err = hipSuccess;
+    std::atomic<size_t> ready{0};  // chunks in the staging; n + 1 = given up
     c->copies.run((m + slice - 1) / slice,
                   [&](size_t i) {
                     const size_t o = i * slice;
@@ -210,7 +212,7 @@ void copy_to_host(ll_gpu_ctx* c, void* dst, const void* src, size_t bytes) {
                     if (r <= n) std::memcpy(d + off + o, stage + o, std::min(slice, m - o));
                   },
                   [&] {
-                    for (size_t i = 1; i < n && err == hipSuccess; i++) {
+                    for (size_t i = 0; i < n && err == hipSuccess; i++) {
                       err = hipEventSynchronize(c->chunk_ev[i]);
                       ready.store(err == hipSuccess ? i + 1 : n + 1, std::memory_order_release);
                     }

@@ -178,7 +178,7 @@ struct ll_gpu_ctx {
   void* pinned = nullptr;      // staging for uploads
   size_t pinned_bytes = 0;
   hipEvent_t pinned_ev[2] = {nullptr, nullptr};
-  std::vector<hipEvent_t> chunk_ev;  // results: one per staging chunk
+  std::vector<hipEvent_t> chunk_ev;  // results: one per staging chunk, and their start
   llgpu::CopyPool copies;      // threads between the staging and the caller's arrays
   void* readback = nullptr;    // small pinned buffer for per-level counter reads
   std::map<std::string, int> tuned;    // autotuner decisions
