@@ -1,6 +1,7 @@
 """Weighted PageRank sweeps at the edges of the sweep items: rows of 0, 1, 8,
-32, 33, 255..257, 511..513, 767..769 and thousands of entries, graphs whose x
-fits the LDS table and one that does not, against FP64."""
+32, 33, 255..257, 511..513, 767..769 and thousands of entries, over the
+vertices' own numbers and, on both sides of the limits from which on it is
+taken, over rows and columns by degree with the LDS table, against FP64."""
 import time
 
 import numpy as np
@@ -21,11 +22,9 @@ D, K = 0.85, 12
 TOL = 2.4e-6
 
 
-@pytest.mark.parametrize("V", [1, 70, 4001, 24576, 24577, 90001])
-def test_rows_of_every_length(ctx, V):
-    gpu_case(f"wpr rows V={V}")
+def check(ctx, V, extra_src, extra_dst):
     rng = np.random.default_rng(V)
-    src, dst = [], []
+    src, dst = [extra_src], [extra_dst]
     for i, d in enumerate(DEGS * 3):
         if V < 2 or d >= 4 * V:
             continue
@@ -33,8 +32,6 @@ def test_rows_of_every_length(ctx, V):
         other = rng.integers(0, V, d)
         (src if i % 2 else dst).append(np.full(d, v))
         (dst if i % 2 else src).append(other)
-    src.append(rng.integers(0, V, 3 * V))
-    dst.append(rng.integers(0, V, 3 * V))
     src, dst = np.concatenate(src), np.concatenate(dst)
     ofs, adj = csr_of(V, src, dst)
     tail = np.repeat(np.arange(V), np.diff(ofs))
@@ -60,10 +57,30 @@ def test_rows_of_every_length(ctx, V):
     assert torch.equal(again, r)  # the sums do not depend on the schedule
 
 
-@pytest.mark.parametrize("V", [24576, 24577, 60001])
+@pytest.mark.parametrize("V", [1, 70, 4001, 24576, 24577, 90001])
+def test_rows_of_every_length(ctx, V):
+    gpu_case(f"wpr rows V={V}")
+    rng = np.random.default_rng(V)
+    check(ctx, V, rng.integers(0, V, 3 * V), rng.integers(0, V, 3 * V))
+
+
+# vertices, edges per vertex, power: the hottest 24576 columns hold 0.49 of the
+# entries with power 3.4, 0.094 with 1; the table is taken in the second, third
+# and last case
+@pytest.mark.parametrize("V,per,power", [(262_143, 5, 3.4), (262_144, 5, 3.4), (262_145, 4, 3.4),
+                                         (262_144, 3, 3.4), (262_144, 5, 1), (400_001, 6, 5)])
+def test_table_form(ctx, V, per, power):
+    gpu_case(f"wpr table form V={V} per={per} power={power}")
+    rng = np.random.default_rng(per)
+    ids = rng.permutation(V)
+    s, d = (ids[(V * rng.random(per * V) ** power).astype(np.int64)] for _ in range(2))
+    check(ctx, V, s, d)
+
+
+@pytest.mark.parametrize("V", [24576, 24577, 262_143, 262_144])
 def test_out_edges_alone(ctx, V):
     """A single-level CSR without its in-edges gives the same forward and
-    adjoint, bit for bit."""
+    adjoint, bit for bit; the last by degree, which it counts over the heads."""
     gpu_case(f"wpr out-edges alone V={V}")
     rng = np.random.default_rng(V)
     src = rng.integers(0, V, 6 * V)
@@ -81,11 +98,13 @@ def test_out_edges_alone(ctx, V):
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
-def test_isolated_vertices_cost_little(ctx):
-    """A few connected vertices among 4 M isolated ones: the first call on the
-    snapshot writes 34 MB of row offsets per direction (10 us at the copy rate)
-    and sorts nearly nothing; 20 ms are many times what it needs."""
-    V, n, m = 1 << 22, 2000, 20_000
+@pytest.mark.parametrize("V,n,m", [(1 << 22, 2000, 20_000), (1 << 20, 30_000, 2_200_000)])
+def test_isolated_vertices_cost_little(ctx, V, n, m):
+    """A few connected vertices among a million or four of isolated ones, by
+    their own numbers and by degree, where the isolated ones come in one run:
+    the first call on the snapshot writes 8 to 34 MB of row offsets per
+    direction (10 us at the copy rate) and sorts 4.4 M entries at most (0.2 ms);
+    20 ms are many times what it needs."""
     rng = np.random.default_rng(3)
     ids = rng.permutation(V)[:n]
     src, dst = ids[rng.integers(0, n, m)], ids[rng.integers(0, n, m)]
