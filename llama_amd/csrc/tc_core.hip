@@ -391,14 +391,18 @@ void tc_core_count(ll_gpu_graph* g, uint64_t* triangles, uint64_t* work, uint64_
   k_zero_ull<<<1, 64, 0, s>>>(out.as<unsigned long long>(), 3);
   {
     TimedLaunch tl(ctx, "k_tc_core");
-    // four workgroups fit a CU; more of them even out the rows of a large graph,
+    // four workgroups fit a CU; more of them even out the rows of many arcs,
     // and each clears its bitmaps once more.  us a count by workgroups a CU 8 /
-    // 16 / 32, R-MAT of 16 edges a vertex: 100000 vertices 167 / 220 / 351,
-    // 300000 442 / 411 / 471, 700000 1210 / 1133 / 1113, 2^20 2214 / 2020 /
-    // 1981, 2^22 13191 / 12253 / 11800; 64: 1964 and 11699 at the last two
-    const uint64_t per_cu = g->V > (uint64_t(1) << 19) ? 32 : g->V > (uint64_t(1) << 17) ? 16 : 8;
-    const unsigned grid = unsigned(std::min<uint64_t>((g->V + kWaves - 1) / kWaves,
-                                                      uint64_t(ctx->num_cus) * per_cu));
+    // 16 / 32, R-MAT, vertices x edges per vertex: 300000 x 4 115 / 169 / -,
+    // 100000 x 16 167 / 220 / 351, 2^20 x 4 400 / 380 / 414, 300000 x 16 442 /
+    // 411 / 471, 700000 x 16 1210 / 1133 / 1113, 2^20 x 16 2214 / 2020 / 1981,
+    // 2^22 x 16 13191 / 12253 / 11800 (64: 1964 and 11699 at the last two).
+    // Fewer yet for few arcs: a star of 500000 32 us with 1954 workgroups, 57
+    // with 4096, 20000 x 16 65 with 1220, 87 with 2048.
+    const uint64_t cus = uint64_t(ctx->num_cus);
+    const uint64_t per_cu = t.arcs > (uint64_t(1) << 23) ? 32 : t.arcs > (uint64_t(3) << 20) ? 16 : 8;
+    const unsigned grid = unsigned(std::min<uint64_t>(
+        {(g->V + kWaves - 1) / kWaves, cus * per_cu, std::max<uint64_t>(t.arcs / 256, cus * 4)}));
     const TcCoreArgs a{t.ofs.as<uint64_t>(), t.nbr.as<uint32_t>(), t.nbc.as<uint16_t>(),
                        t.nout.as<uint32_t>(), g->V, out.as<unsigned long long>()};
     if (t.arcs < (uint64_t(1) << 32)) k_tc_core<uint32_t><<<grid, kWaves * 64, 0, s>>>(a);
